@@ -1337,7 +1337,7 @@ __global__ __launch_bounds__(256) void k_chunks_of_cells(const uint32_t* __restr
 
 // Largest float t with sqrtf(t) <= r (strict: sqrtf(t) < r), sqrtf correctly
 // rounded; r > 0.
-static float sqrt_bound(float r, bool strict) {
+float sqrt_bound(float r, bool strict) {
     auto ok = [&](float t) { return strict ? std::sqrt(t) < r : std::sqrt(t) <= r; };
     const float inf = std::numeric_limits<float>::infinity();
     float t = r * r;

@@ -31,6 +31,7 @@
 // value: every vertex sums its candidates in the cell's fixed order.
 #include <algorithm>
 #include <cmath>
+#include <limits>
 
 #include "common.hpp"
 
@@ -174,78 +175,6 @@ __device__ __forceinline__ int trunc_clamped(float q, int res) {
     return (int)q;
 }
 
-// Rows of one exception particle's box (the reference's per-particle loop):
-// calls emit(z, y, word, bits) for every row word with vertices in the band.
-// The x-run of a row has at most 6 vertices (x in [clamp(i-3), clamp(i+3)))
-// and so touches at most two words; its 6 tests are unrolled and branch-free,
-// so they run as independent chains.
-template <typename Emit>
-__device__ __forceinline__ void exception_rows(const BandArgs& a, const float4& p, int x0, int x1,
-                                               int y0, int y1, int z0, int z1, float limit,
-                                               Emit emit) {
-    const uint32_t w0 = (uint32_t)x0 >> 5;
-    for (int z = z0; z <= z1; ++z) {
-        const float vz = vertex_coord((uint32_t)z, a.sc.minz, a.sc.cell);
-        const float dz = vz - p.z;
-        for (int y = y0; y <= y1; ++y) {
-            const float vy = vertex_coord((uint32_t)y, a.sc.miny, a.sc.cell);
-            const float dy = vy - p.y;
-            uint32_t m0 = 0, m1 = 0;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                const int x = x0 + k;
-                const float vx = vertex_coord((uint32_t)x, a.sc.minx, a.sc.cell);
-                const float dx = vx - p.x;
-                // the reference's |v - p| (same operation order as fma(dz, dz, fma(dy, dy, dx dx)))
-                const float dist =
-                    __builtin_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)));
-                const uint32_t bit = (x < x1 && dist < limit) ? 1u << ((uint32_t)x & 31u) : 0u;
-                if (((uint32_t)x >> 5) == w0) m0 |= bit;
-                else m1 |= bit;
-            }
-            if (m0) emit(z, y, w0, m0);
-            if (m1) emit(z, y, w0 + 1u, m1);
-        }
-    }
-}
-
-// The same tests with wave-uniform loops (the box has at most 7 x 7 x 6
-// vertices), for the windowed path: every lane runs all 294 slots, invalid
-// slots test nothing, and each row ORs its nonzero bits into the LDS window.
-__device__ __forceinline__ void exception_rows_window(const BandArgs& a, const float4& p,
-                                                      bool live, int x0, int x1, int y0, int y1,
-                                                      int z0, int z1, float limit, uint32_t* w,
-                                                      int W0, int Y0, int Z0, int nw, int ny) {
-    const uint32_t w0 = (uint32_t)x0 >> 5;
-    for (int kz = 0; kz < 7; ++kz) {
-        const int z = z0 + kz;
-        const bool zok = live && z <= z1;
-        const float dz = vertex_coord((uint32_t)z, a.sc.minz, a.sc.cell) - p.z;
-#pragma unroll
-        for (int ky = 0; ky < 7; ++ky) {
-            const int y = y0 + ky;
-            const bool ok = zok && y <= y1;
-            const float dy = vertex_coord((uint32_t)y, a.sc.miny, a.sc.cell) - p.y;
-            uint32_t m0 = 0, m1 = 0;
-#pragma unroll
-            for (int kx = 0; kx < 6; ++kx) {
-                const int x = x0 + kx;
-                const float dx = vertex_coord((uint32_t)x, a.sc.minx, a.sc.cell) - p.x;
-                const float dist =
-                    __builtin_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)));
-                const uint32_t bit = (x < x1 && dist < limit) ? 1u << ((uint32_t)x & 31u) : 0u;
-                if (((uint32_t)x >> 5) == w0) m0 |= bit;
-                else m1 |= bit;
-            }
-            if (ok && (m0 | m1)) {
-                const int base = ((z - Z0) * ny + (y - Y0)) * nw + ((int)w0 - W0);
-                if (m0) atomicOr(&w[base], m0);
-                if (m1) atomicOr(&w[base + 1], m1);  // m1 != 0: word w0 + 1 is in the window
-            }
-        }
-    }
-}
-
 __device__ __forceinline__ int wave_min_i(int v) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
@@ -264,83 +193,206 @@ __device__ __forceinline__ void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The reference's per-particle band loop for the exception list, one wave per
-// 64 exceptions.  Device-scope atomics are slow here, so a wave whose boxes
-// fit a window of kWinWords x kWinRows x kWinRows mask words (the common case:
-// the list is filled in sorted order, so a wave's particles are neighbours)
-// ORs its bits into that window in LDS and then adds each nonzero window word
-// to the mask with one atomic; other waves OR straight into the mask.
-constexpr int kWinWords = 3, kWinRows = 16;
-constexpr int kWin = kWinWords * kWinRows * kWinRows;
+// The reference's per-particle band loop (the exact path), for the exception
+// list or, when every surface particle takes it, for the surface flags in
+// particle order.  A wave takes `group` consecutive list entries (particles),
+// one per lane for the box and its cell, and compacts the live ones into LDS;
+// then it treats 8 particles at a time, 8 lanes each: lane k of a particle's 8
+// walks layer z0 + k of its box (at most 7 layers of 7 rows of 6 vertices).
+// `group` shrinks with the particle count (32 down to 8), so that a small
+// frame still has a wave for every 8 particles.  One particle per lane, its 294
+// tests in a row, took 28.9 us for a 960-particle block and 128.9 us for
+// 1,000,000 dam-break particles on the half-hash-cell grid; this form takes 6.3
+// and 41.2 us (groups of 16 and 64: 50 and 52 us).
+//
+// The reference tests the FP32 distance sqrt(d2) < 1.5 h.  The square root is
+// monotonic and correctly rounded, so this is d2 < a.d2_limit exactly, the
+// smallest float whose root fails (found on the host).  d2 = fma(dz, dz,
+// fma(dy, dy, dx dx)) as the reference forms it, its dx dx once per particle.
+// A particle with a NaN coordinate has no vertex in the band.
+//
+// It is bound by the tests' VALU work and then by the ORs: device-scope atomics
+// are slow here, and a word takes bits from every particle within 3 cells of its
+// 32 vertices.  So the bits are gathered in an LDS window first: the waves of a
+// workgroup (up to 128 consecutive sorted particles, whose boxes share their
+// words) use one window when the box of their boxes has at most kExcWindow
+// words; else each wave its own part of it, and a wave whose box does not fit
+// there ORs straight into the mask.  Each nonzero window word then costs one
+// atomic.  (Windows of one wave took 61 us, of 16 waves 71 us: too few, too
+// uneven workgroups.)
+constexpr int kExcWaves = 4;
+constexpr int kExcWindow = 2048;                      // words of the workgroup's window
+constexpr int kExcWaveWindow = kExcWindow / kExcWaves;
+constexpr uint32_t kExcLanes = 8;                     // lanes per particle
+constexpr uint32_t kExcPart = 64 / kExcLanes;         // particles per step of a wave
 
-__global__ __launch_bounds__(256) void k_band_exceptions(BandArgs a) {
-    __shared__ uint32_t win[4][kWin];
+// Words [w0, w0 + nw) of rows [y0, y0 + ny) of layers [z0, z0 + nz) of the mask
+// that the clamped boxes about the cells [lo, hi] touch.
+struct MaskBox {
+    int w0, y0, z0, nw, ny, nz;
+    __device__ __forceinline__ MaskBox(const GridDev& sc, const int* lo, const int* hi) {
+        w0 = clampi(lo[0] - 3, 0, sc.rx - 1) >> 5;
+        y0 = clampi(lo[1] - 3, 0, sc.ry - 1);
+        z0 = clampi(lo[2] - 3, 0, sc.rz - 1);
+        nw = (clampi(hi[0] + 3, 0, sc.rx - 1) >> 5) - w0 + 1;
+        ny = clampi(hi[1] + 3, 0, sc.ry - 1) - y0 + 1;
+        nz = clampi(hi[2] + 3, 0, sc.rz - 1) - z0 + 1;
+    }
+    __device__ __forceinline__ bool fits(int words) const {
+        return (int64_t)nw * ny * nz <= (int64_t)words;
+    }
+    // ORs the window's words into the mask: thread t of n
+    __device__ __forceinline__ void flush(const uint32_t* win, uint32_t* bits, const GridDev& sc,
+                                          uint32_t wx, int t, int n) const {
+        for (int r = t; r < ny * nz; r += n) {
+            const int zi = r / ny, yi = r - zi * ny;
+            uint32_t* row = bits + ((uint64_t)(z0 + zi) * sc.ry + (uint32_t)(y0 + yi)) * wx + w0;
+            for (int k = 0; k < nw; ++k) {
+                const uint32_t m = win[r * nw + k];
+                if (m) atomicOr(row + k, m);
+            }
+        }
+    }
+};
+
+__global__ __launch_bounds__(64 * kExcWaves) void k_band_exceptions(BandArgs a, uint32_t group) {
+    __shared__ float4 pos[kExcWaves][64];  // a wave's live particles, compacted
+    __shared__ int3 cell[kExcWaves][64];   // their scalar cells
+    __shared__ uint32_t window[kExcWindow];
+    __shared__ int box[6];                 // cell box of the workgroup's particles
     const bool by_flags = a.all_exceptions != 0 && a.flags != nullptr;
     const uint32_t count = by_flags ? a.num_particles : a.counters->num_exceptions;
     const uint32_t wx = row_words(a.sc.rx);
-    // The reference compares the FP32 distance with 1.5 h in double.  For a
-    // float d, (double)d < L holds exactly when d < the smallest float >= L.
-    const double L = (double)a.h * 1.5;
-    float limit = (float)L;
-    if ((double)limit < L) limit = __int_as_float(__float_as_int(limit) + 1);
     const uint32_t lane = __lane_id();
-    uint32_t* w = win[threadIdx.x >> 6];
-    const uint32_t stride = gridDim.x * blockDim.x;
-    // wave-uniform loop: every lane of the wave runs the same iterations
-    for (uint32_t e0 = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); e0 < count; e0 += stride) {
-        const uint32_t e = e0 + lane;
-        bool live = e < count;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint64_t per_block = (uint64_t)kExcWaves * group;
+    const int big = 0x3fffffff;
+    // workgroup-uniform loop
+    for (uint64_t b0 = blockIdx.x * per_block; b0 < count; b0 += gridDim.x * per_block) {
+        if (threadIdx.x < 6) box[threadIdx.x] = threadIdx.x < 3 ? big : -big;
+        const uint64_t e = b0 + (uint64_t)wave * group + lane;
+        bool live = lane < group && e < count;
         uint32_t pi = 0;
         if (live) {
             if (by_flags) {
                 live = a.flags[e] != 0u;
-                pi = e;
+                pi = (uint32_t)e;
             } else {
                 pi = a.exceptions[e];
             }
         }
         float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
-        int x0 = 0x7fffffff, x1 = -1, y0 = 0x7fffffff, y1 = -1, z0 = 0x7fffffff, z1 = -1;
         if (live) {
             p = a.sorted[pi];
-            const int i = trunc_clamped(cell_coord(p.x, a.sc.minx, a.sc.cell), a.sc.rx);
-            const int j = trunc_clamped(cell_coord(p.y, a.sc.miny, a.sc.cell), a.sc.ry);
-            const int k = trunc_clamped(cell_coord(p.z, a.sc.minz, a.sc.cell), a.sc.rz);
-            x0 = clampi(i - 3, 0, a.sc.rx - 1); x1 = clampi(i + 3, 0, a.sc.rx - 1);
-            y0 = clampi(j - 3, 0, a.sc.ry - 1); y1 = clampi(j + 3, 0, a.sc.ry - 1);
-            z0 = clampi(k - 3, 0, a.sc.rz - 1); z1 = clampi(k + 3, 0, a.sc.rz - 1);
+            live = p.x == p.x && p.y == p.y && p.z == p.z;
         }
-        // a wave without a surface particle has nothing to do (wave-uniform)
-        if (__ballot(live) == 0) continue;
-        // the wave's window: words [W0, W1] of rows [Y0, Y1] of layers [Z0, Z1]
-        // (over the live lanes; at least one is live)
-        const int W0 = wave_min_i(x0) >> 5, W1 = wave_max_i(x1) >> 5;
-        const int Y0 = wave_min_i(y0), Y1 = wave_max_i(y1);
-        const int Z0 = wave_min_i(z0), Z1 = wave_max_i(z1);
-        const int nw = W1 - W0 + 1, ny = Y1 - Y0 + 1, nz = Z1 - Z0 + 1;
-        if (nw <= kWinWords && ny <= kWinRows && nz <= kWinRows) {
-            const int n = nw * ny * nz;
-            for (int t = (int)lane; t < n; t += 64) w[t] = 0u;
+        const uint64_t m = __ballot(live);
+        const uint32_t n = (uint32_t)__popcll(m);
+        int lo[3] = {big, big, big}, hi[3] = {-big, -big, -big};
+        if (n) {
+            if (live) {
+                lo[0] = hi[0] = trunc_clamped(cell_coord(p.x, a.sc.minx, a.sc.cell), a.sc.rx);
+                lo[1] = hi[1] = trunc_clamped(cell_coord(p.y, a.sc.miny, a.sc.cell), a.sc.ry);
+                lo[2] = hi[2] = trunc_clamped(cell_coord(p.z, a.sc.minz, a.sc.cell), a.sc.rz);
+                pos[wave][mask_rank(m)] = p;
+                cell[wave][mask_rank(m)] = make_int3(lo[0], lo[1], lo[2]);
+            }
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                lo[d] = wave_min_i(lo[d]);
+                hi[d] = wave_max_i(hi[d]);
+            }
+        }
+        __syncthreads();
+        if (n && lane == 0) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                atomicMin(&box[d], lo[d]);
+                atomicMax(&box[3 + d], hi[d]);
+            }
+        }
+        __syncthreads();
+        int blo[3], bhi[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            blo[d] = box[d];
+            bhi[d] = box[3 + d];
+        }
+        __syncthreads();  // box is rewritten by the next round
+        // no surface particle in the workgroup's entries (uniform)
+        if (blo[0] > bhi[0]) continue;
+        MaskBox mb(a.sc, blo, bhi);
+        const bool shared = mb.fits(kExcWindow);
+        uint32_t* win = window;
+        bool windowed = shared;
+        if (!shared && n) {
+            mb = MaskBox(a.sc, lo, hi);
+            windowed = mb.fits(kExcWaveWindow);
+            win = window + wave * kExcWaveWindow;
+        }
+        const int nwin = mb.nw * mb.ny * mb.nz;
+        if (shared) {
+            for (int t = (int)threadIdx.x; t < nwin; t += 64 * kExcWaves) win[t] = 0u;
+            __syncthreads();
+        } else {
+            if (windowed)
+                for (int t = (int)lane; t < nwin; t += 64) win[t] = 0u;
             wave_sync_lds();
-            // lanes without a particle test nothing (in-range dummy bounds)
-            exception_rows_window(a, p, live, live ? x0 : 0, live ? x1 : 0, live ? y0 : 0,
-                                  live ? y1 : 0, live ? z0 : 0, live ? z1 : 0, limit, w, W0, Y0,
-                                  Z0, nw, ny);
-            wave_sync_lds();
-            for (int t = (int)lane; t < n; t += 64) {
-                const uint32_t m = w[t];
-                if (m) {
-                    const int wi = t % nw, yi = (t / nw) % ny, zi = t / (nw * ny);
-                    const uint64_t row = (uint64_t)(Z0 + zi) * a.sc.ry + (uint32_t)(Y0 + yi);
-                    atomicOr(&a.bits[row * wx + (uint32_t)(W0 + wi)], m);
+        }
+        for (uint32_t it = 0; it < n; it += kExcPart) {
+            const uint32_t slot = it + lane / kExcLanes;
+            if (slot >= n) continue;
+            const float4 p = pos[wave][slot];
+            const int3 pc = cell[wave][slot];
+            const int x0 = clampi(pc.x - 3, 0, a.sc.rx - 1), x1 = clampi(pc.x + 3, 0, a.sc.rx - 1);
+            const int y0 = clampi(pc.y - 3, 0, a.sc.ry - 1), y1 = clampi(pc.y + 3, 0, a.sc.ry - 1);
+            const int z0 = clampi(pc.z - 3, 0, a.sc.rz - 1), z1 = clampi(pc.z + 3, 0, a.sc.rz - 1);
+            const int z = z0 + (int)(lane % kExcLanes);
+            if (z > z1) continue;
+            const float dz = vertex_coord((uint32_t)z, a.sc.minz, a.sc.cell) - p.z;
+            // a row has vertices x in [x0, x1), at most 6, in one or two words
+            const uint32_t w0 = (uint32_t)x0 >> 5, sh = (uint32_t)x0 & 31u;
+            const uint32_t valid = (1u << (x1 - x0)) - 1u;
+            float xx[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                const float dx = vertex_coord((uint32_t)(x0 + k), a.sc.minx, a.sc.cell) - p.x;
+                xx[k] = dx * dx;
+            }
+            const int at = ((z - mb.z0) * mb.ny + (y0 - mb.y0)) * mb.nw + ((int)w0 - mb.w0);
+            uint32_t* row = a.bits + ((uint64_t)z * a.sc.ry + (uint32_t)y0) * wx + w0;
+#pragma unroll
+            for (int ky = 0; ky < 7; ++ky) {
+                const float dy = vertex_coord((uint32_t)(y0 + ky), a.sc.miny, a.sc.cell) - p.y;
+                // bit k: d2 < a.d2_limit, as the sign of the difference (exact:
+                // a float difference is negative exactly when it should be)
+                uint32_t in = 0;
+#pragma unroll
+                for (int k = 5; k >= 0; --k) {
+                    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, xx[k]));
+                    in = __builtin_amdgcn_alignbit(in, (uint32_t)__float_as_int(d2 - a.d2_limit),
+                                                   31);
+                }
+                const uint64_t bits = (uint64_t)(in & valid) << sh;
+                const uint32_t m0 = (uint32_t)bits, m1 = (uint32_t)(bits >> 32);
+                if (y0 + ky > y1) continue;
+                if (windowed) {
+                    if (m0) atomicOr(&win[at + ky * mb.nw], m0);
+                    if (m1) atomicOr(&win[at + ky * mb.nw + 1], m1);
+                } else {
+                    if (m0) atomicOr(row + (uint64_t)ky * wx, m0);
+                    if (m1) atomicOr(row + (uint64_t)ky * wx + 1, m1);
                 }
             }
+        }
+        if (shared) {
+            __syncthreads();
+            mb.flush(win, a.bits, a.sc, wx, (int)threadIdx.x, 64 * kExcWaves);
+            __syncthreads();
+        } else {
             wave_sync_lds();
-        } else if (live) {
-            exception_rows(a, p, x0, x1, y0, y1, z0, z1, limit,
-                           [&](int z, int y, uint32_t word, uint32_t m) {
-                               atomicOr(&a.bits[((uint64_t)z * a.sc.ry + y) * wx + word], m);
-                           });
+            if (windowed && n) mb.flush(win, a.bits, a.sc, wx, (int)lane, 64);
+            wave_sync_lds();
         }
     }
 }
@@ -729,7 +781,9 @@ fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s) {
     // (z); `sbits` is consumed
     uint32_t* sb = const_cast<uint32_t*>(a.sbits);
     const dim3 tiles((wx + kTW - 1) / kTW, (a.sc.ry + kTY - 1) / kTY, (a.sc.rz + kTZ - 1) / kTZ);
-    if (tiles.y <= 65535u && tiles.z <= 65535u) {
+    if (a.all_exceptions) {
+        // no seeds: the exact path alone sets bits of the mask the caller cleared
+    } else if (tiles.y <= 65535u && tiles.z <= 65535u) {
         hipLaunchKernelGGL(k_dilate_box, tiles, dim3(kDilateThreads), 0, s, (const uint8_t*)sb, a.bits, wx,
                            a.sc);
         FSR_LAUNCH_CHECK("k_dilate_box");
@@ -744,8 +798,21 @@ fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s) {
                            (uint64_t)wx * a.sc.ry, a.sc.rz, (uint64_t)a.sc.rz);
         FSR_LAUNCH_CHECK("k_dilate_rows(z)");
     }
-    const int eb = persistent_blocks(ctx, 256, 4, TUNE_BAND);
-    hipLaunchKernelGGL(k_band_exceptions, dim3(eb), dim3(256), 0, s, a);
+    // six workgroups of 4 waves per CU
+    const uint32_t eb = 6u * (uint32_t)ctx->num_cus;
+    // 1.5 h in double, as the smallest float that is not below it: for a float
+    // d, (double)d < L holds exactly when d < that float
+    const double L = (double)a.h * 1.5;
+    float limit = (float)L;
+    if ((double)limit < L) limit = std::nextafter(limit, std::numeric_limits<float>::infinity());
+    BandArgs b = a;
+    b.d2_limit = limit > 0.0f ? std::nextafter(sqrt_bound(limit, true),
+                                               std::numeric_limits<float>::infinity())
+                              : -1.0f;
+    const uint32_t waves = (uint32_t)kExcWaves * eb;
+    const uint32_t per = (a.num_particles + waves - 1u) / waves;
+    const uint32_t group = std::min(32u, std::max(8u, (per + 7u) / 8u * 8u));
+    hipLaunchKernelGGL(k_band_exceptions, dim3(eb), dim3(64 * kExcWaves), 0, s, b, group);
     FSR_LAUNCH_CHECK("k_band_exceptions");
     return FSR_OK;
 }

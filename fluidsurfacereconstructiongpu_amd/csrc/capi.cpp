@@ -255,12 +255,17 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
     FSR_TRY(arena_typed(ctx, A_BAND_TMP, W, &tmp));
     FSR_TRY(arena_typed(ctx, A_BAND_BITS, W, &bits));
     FSR_TRY(arena_typed(ctx, A_EXCEPTIONS, n, &exc));
-    // counters, stats and the band seed mask start at zero; cleared in the
-    // launch that initialises the hash grid
+    const int all_exceptions = band_dilation_exact(scg, sim->smoothing_radius) ? 0 : 1;
+    // counters, stats and the band seed mask (or the band mask itself, when no
+    // particle seeds a dilation) start at zero; cleared in the launch that
+    // initialises the hash grid
     FillList fills;
     fills.add(counters, 0u, sizeof(Counters) / 4);
     fills.add(stats, 0u, sizeof(fsr_frame_stats) / 4);
-    fills.add(sbits, 0u, 8ull * W);
+    if (all_exceptions)
+        fills.add(bits, 0u, W);
+    else
+        fills.add(sbits, 0u, 8ull * W);
     // the dense field outside the band keeps the fill: 0, or the byte 100 for
     // Yu13 (the reference's memset of the Yu13 grid)
     fills.add(phi, yu13 ? 0x64646464u : 0u, V);
@@ -286,7 +291,7 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
     sa.exceptions = exc;
     sa.counters = counters;
     sa.st = stats;
-    sa.all_exceptions = band_dilation_exact(scg, sim->smoothing_radius) ? 0 : 1;
+    sa.all_exceptions = all_exceptions;
     sa.radius_count = (!yu13 && ctx->surface_mode == FSR_SURFACE_RADIUS_COUNT) ? 1 : 0;
     uint32_t* involve = nullptr;
     if (yu13) FSR_TRY(arena_typed(ctx, A_INVOLVE, C, &involve));

@@ -440,8 +440,12 @@ struct BandArgs {
     // instead of the exception list, whose order is that of the appends.
     const uint32_t* flags;
     uint32_t num_particles;
-    int all_exceptions;
+    int all_exceptions;        // the mask `bits` is cleared by the caller then
+    float d2_limit = 0.0f;     // set by band_build
 };
+// Largest float t with sqrtf(t) <= r (strict: sqrtf(t) < r), sqrtf correctly
+// rounded; r > 0.
+float sqrt_bound(float r, bool strict);
 fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s);
 // Returns 1 when every vertex of the reference's band box lies within 1.5 h of
 // the particle, so the band equals a box dilation of the surface cells.

@@ -478,7 +478,11 @@ fsr_status fsr_estimation_of_surface_vertices(fsr_context* ctx, const fsr_sim_pa
     FSR_TRY(arena_typed(ctx, A_BAND_BITS, W, &bits));
     FSR_TRY(arena_typed(ctx, A_EXCEPTIONS, nn, &exc));
     FSR_TRY(arena_typed(ctx, A_SORTED, nn, &p4));
-    FSR_TRY(fill_u32(sbits, 0u, 8ull * W, s));
+    const int all_exceptions = band_dilation_exact(*sc, sim->smoothing_radius) ? 0 : 1;
+    if (all_exceptions)
+        FSR_TRY(fill_u32(bits, 0u, W, s));
+    else
+        FSR_TRY(fill_u32(sbits, 0u, 8ull * W, s));
     if (num_particles) {
         hipLaunchKernelGGL(k_pack_f4, dim3(blocks_for(num_particles)), dim3(256), 0, s, particles,
                            (const float*)nullptr, num_particles, p4);
@@ -494,7 +498,7 @@ fsr_status fsr_estimation_of_surface_vertices(fsr_context* ctx, const fsr_sim_pa
         a.exceptions = exc;
         a.counters = ct;
         a.st = st;
-        a.all_exceptions = band_dilation_exact(*sc, sim->smoothing_radius) ? 0 : 1;
+        a.all_exceptions = all_exceptions;
         FSR_TRY(surface_seed_from_flags(ctx, a, s));
     }
     BandArgs ba;
@@ -510,7 +514,7 @@ fsr_status fsr_estimation_of_surface_vertices(fsr_context* ctx, const fsr_sim_pa
     ba.st = st;
     ba.flags = surface_flags;
     ba.num_particles = num_particles;
-    ba.all_exceptions = band_dilation_exact(*sc, sim->smoothing_radius) ? 0 : 1;
+    ba.all_exceptions = all_exceptions;
     FSR_TRY(band_build(ctx, ba, s));
     hipLaunchKernelGGL(k_bits_to_dense, dim3(blocks_for(V)), dim3(256), 0, s, bits, g.rx, wx, V,
                        is_surface_grid);
