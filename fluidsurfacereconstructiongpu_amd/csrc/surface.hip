@@ -42,32 +42,57 @@ __device__ __forceinline__ int trunc_cell(float q, int res) {
     return (int)q;
 }
 
+// Surface cells, and the frame's surface particle count (the particles of those
+// cells; st may be null): counted here, once per cell, because the per-particle
+// pass would end in an atomic per workgroup on one address, and about a
+// thousand of those took most of its time.
 __global__ __launch_bounds__(256) void k_cell_surface(const float* __restrict__ occupancy,
-                                                      GridDev sp, uint8_t* __restrict__ surf_cell) {
+                                                      const fsr_index_range* __restrict__ ranges,
+                                                      GridDev sp, uint8_t* __restrict__ surf_cell,
+                                                      fsr_frame_stats* __restrict__ st,
+                                                      int all_exceptions) {
+    __shared__ uint32_t part[4];
     const uint32_t C = sp.rx * sp.ry * sp.rz;
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    const uint32_t x = c % sp.rx, y = (c / sp.rx) % sp.ry, z = c / (sp.rx * sp.ry);
-    uint8_t surf = 0;
-    if (x < sp.rx - 1 && y < sp.ry - 1 && z < sp.rz - 1 && occupancy[c] >= 1.0f) {
-        // the clamped 3^3 block as 27 clamped offsets (a clamped offset repeats
-        // a cell of the block, which leaves the test unchanged), all read with
-        // no early exit, so that their loads issue together
+    uint32_t n_surf = 0;
+    for (uint64_t c0 = (uint64_t)blockIdx.x * 256u; c0 < C; c0 += (uint64_t)gridDim.x * 256u) {
+        const uint64_t cc = c0 + threadIdx.x;
+        if (cc >= C) break;
+        const uint32_t c = (uint32_t)cc;
+        const uint32_t x = c % sp.rx, y = (c / sp.rx) % sp.ry, z = c / (sp.rx * sp.ry);
+        uint8_t surf = 0;
+        if (x < sp.rx - 1 && y < sp.ry - 1 && z < sp.rz - 1 && occupancy[c] >= 1.0f) {
+            // the clamped 3^3 block as 27 clamped offsets (a clamped offset repeats
+            // a cell of the block, which leaves the test unchanged), all read with
+            // no early exit, so that their loads issue together
+            const fsr_index_range own = ranges[c];
 #pragma unroll
-        for (int dz = -1; dz <= 1; ++dz) {
-            const uint32_t zz = (uint32_t)clampi((int)z + dz, 0, sp.rz - 1);
+            for (int dz = -1; dz <= 1; ++dz) {
+                const uint32_t zz = (uint32_t)clampi((int)z + dz, 0, sp.rz - 1);
 #pragma unroll
-            for (int dy = -1; dy <= 1; ++dy) {
-                const uint32_t yy = (uint32_t)clampi((int)y + dy, 0, sp.ry - 1);
+                for (int dy = -1; dy <= 1; ++dy) {
+                    const uint32_t yy = (uint32_t)clampi((int)y + dy, 0, sp.ry - 1);
 #pragma unroll
-                for (int dx = -1; dx <= 1; ++dx) {
-                    const uint32_t xx = (uint32_t)clampi((int)x + dx, 0, sp.rx - 1);
-                    surf |= occupancy[(zz * sp.ry + yy) * sp.rx + xx] < 1.0f ? 1 : 0;
+                    for (int dx = -1; dx <= 1; ++dx) {
+                        const uint32_t xx = (uint32_t)clampi((int)x + dx, 0, sp.rx - 1);
+                        surf |= occupancy[(zz * sp.ry + yy) * sp.rx + xx] < 1.0f ? 1 : 0;
+                    }
                 }
             }
+            if (surf) n_surf += own.end - own.start;
+        }
+        surf_cell[c] = surf;
+    }
+    if (!st) return;
+    const uint32_t sum = wave_sum(n_surf);
+    if (__lane_id() == 0) part[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t total = part[0] + part[1] + part[2] + part[3];
+        if (total) {
+            atomicAdd(&st->num_surface_particles, total);
+            if (all_exceptions) atomicAdd(&st->band_exceptions, total);
         }
     }
-    surf_cell[c] = surf;
 }
 
 // Involve counts (K4, the Yu13 half): an occupied cell within the clamped 5^3
@@ -137,15 +162,15 @@ __device__ __forceinline__ bool seed_particle(const SurfaceArgs& a, uint32_t i, 
 // dependent load rather than once per element.
 constexpr uint32_t kPerThread = 4;
 
-// Surface flags from the surface hash cells (ZB05 occupancy method), band
-// seeding, and the frame's surface / exception counts.  Grid-stride with a
-// block-uniform trip count over a bounded grid: the two counters take one
-// atomic per block, and thousands of atomics on one address serialise.
+// Surface flags from the surface hash cells (ZB05 occupancy method) and band
+// seeding.  HBM-bound in the large: 4N read, 4N written, 16 bytes and a byte
+// store per surface particle.
 __global__ __launch_bounds__(256) void k_flags_from_cells(SurfaceArgs a,
                                                           const uint8_t* __restrict__ surf_cell) {
     const uint32_t C = a.sp.rx * a.sp.ry * a.sp.rz;
     const uint32_t span = blockDim.x * kPerThread;
-    uint32_t n_surf = 0, n_exc = 0;
+    const bool seeds = a.sbits && !a.all_exceptions;
+    uint32_t n_exc = 0;
     for (uint32_t base = blockIdx.x * span; base < a.n; base += gridDim.x * span) {
         uint32_t key[kPerThread];
 #pragma unroll
@@ -160,22 +185,22 @@ __global__ __launch_bounds__(256) void k_flags_from_cells(SurfaceArgs a,
             surf[k] = key[k] < C && surf_cell[key[k]] != 0;
             if (i < a.n) a.flags[i] = surf[k] ? 1u : 0u;
         }
+        if (!seeds) continue;
         // positions only of the surface particles (the band seeds)
         float4 p[kPerThread];
 #pragma unroll
         for (uint32_t k = 0; k < kPerThread; ++k) {
             const uint32_t i = base + k * blockDim.x + threadIdx.x;
-            p[k] = (a.sbits && surf[k] && !a.all_exceptions) ? a.sorted[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            p[k] = surf[k] ? a.sorted[i] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
         for (uint32_t k = 0; k < kPerThread; ++k) {
             const uint32_t i = base + k * blockDim.x + threadIdx.x;
-            const bool exc = a.sbits ? seed_particle(a, i, p[k].x, p[k].y, p[k].z, surf[k]) : false;
-            n_surf += surf[k] ? 1u : 0u;
-            n_exc += exc ? 1u : 0u;
+            n_exc += seed_particle(a, i, p[k].x, p[k].y, p[k].z, surf[k]) ? 1u : 0u;
         }
     }
-    if (a.st) block_count_add2(&a.st->num_surface_particles, n_surf, &a.st->band_exceptions, n_exc);
+    // particles outside the scalar grid: few, if any
+    if (seeds && a.st) wave_count_add(&a.st->band_exceptions, n_exc);
 }
 
 // Particles outside the hash grid (sorted last, in no cell): one thread each,
@@ -498,8 +523,8 @@ fsr_status surface_seed_from_flags(fsr_context* ctx, const SurfaceArgs& a, hipSt
 fsr_status surface_occupancy(fsr_context* ctx, const SurfaceArgs& a, uint8_t* surf_cell,
                              uint32_t* involve, hipStream_t s) {
     const uint32_t C = a.sp.rx * a.sp.ry * a.sp.rz;
-    hipLaunchKernelGGL(k_cell_surface, dim3((C + 255) / 256), dim3(256), 0, s, a.occupancy,
-                       a.sp, surf_cell);
+    hipLaunchKernelGGL(k_cell_surface, dim3(std::min((C + 255) / 256, 1024u)), dim3(256), 0, s,
+                       a.occupancy, a.ranges, a.sp, surf_cell, a.st, a.all_exceptions);
     FSR_LAUNCH_CHECK("k_cell_surface");
     if (involve) {
         uint8_t* tmp;
