@@ -433,14 +433,14 @@ __device__ __forceinline__ uint32_t nb_reduce4_u(uint32_t x) {
 
 // The tiles of n staged candidates (a multiple of 16) against the NT lane
 // tiles.  rows: the queue at the first staged entry.
-template <bool kCov, int NT>
+template <bool kCov, int NT, int kStride>
 __device__ __forceinline__ void nb_tiles(const float* __restrict__ rows, uint32_t n,
                                          const float (&b1)[NT], v4f (&acc)[kCov ? 3 : 1][NT],
                                          uint32_t (&cnt)[NT], float le_s2) {
     const uint32_t lane = __lane_id();
-    const float* a1p = rows + (lane >> 4) * kNbStride + (lane & 15u);
-    const float* a2p = rows + (lane & 3u) * kNbStride + 4u * (lane >> 4);
-    const float* cqp = rows + NbRows<kCov>::kQ * kNbStride + 4u * (lane >> 4);
+    const float* a1p = rows + (lane >> 4) * kStride + (lane & 15u);
+    const float* a2p = rows + (lane & 3u) * kStride + 4u * (lane >> 4);
+    const float* cqp = rows + NbRows<kCov>::kQ * kStride + 4u * (lane >> 4);
     for (uint32_t tb = 0; tb < n; tb += 16u) {
         const float a1 = a1p[tb];
         const float4 cq = *reinterpret_cast<const float4*>(cqp + tb);
@@ -476,7 +476,7 @@ __device__ __forceinline__ void nb_tiles(const float* __restrict__ rows, uint32_
         if (kCov) {
 #pragma unroll
             for (int g = 1; g < 3; ++g) {
-                const float4 ag = *reinterpret_cast<const float4*>(a2p + (4 * g) * kNbStride + tb);
+                const float4 ag = *reinterpret_cast<const float4*>(a2p + (4 * g) * kStride + tb);
 #pragma unroll
                 for (int T = 0; T < NT; ++T) acc[g][T] = __builtin_amdgcn_mfma_f32_4x4x1f32(ag.x, w[T][0], acc[g][T], 0, 0, 0);
 #pragma unroll
@@ -487,6 +487,52 @@ __device__ __forceinline__ void nb_tiles(const float* __restrict__ rows, uint32_
                 for (int T = 0; T < NT; ++T) acc[g][T] = __builtin_amdgcn_mfma_f32_4x4x1f32(ag.w, w[T][3], acc[g][T], 0, 0, 0);
             }
         }
+    }
+}
+
+// One full batch of 64 staged candidates against one lane tile: the operations
+// of nb_tiles<kCov, 1> in its order, with the four steps' distance products and
+// weights formed side by side (one tile alone leaves each product's latency in
+// the open).
+template <bool kCov, int kStride>
+__device__ __forceinline__ void nb_tile64(const float* __restrict__ rows, float b1,
+                                          v4f (&acc)[kCov ? 3 : 1][1], uint32_t& cnt,
+                                          float le_s2) {
+    const uint32_t lane = __lane_id();
+    const float* a1p = rows + (lane >> 4) * kStride + (lane & 15u);
+    const float* a2p = rows + (lane & 3u) * kStride + 4u * (lane >> 4);
+    const float* cqp = rows + NbRows<kCov>::kQ * kStride + 4u * (lane >> 4);
+    v4f w[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const float4 cq = *reinterpret_cast<const float4*>(cqp + 16 * t);
+        w[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1p[16 * t], b1, v4f{cq.x, cq.y, cq.z, cq.w},
+                                                    0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float s2 = w[t][r];
+            if (kCov) cnt += s2 <= le_s2 ? 1u : 0u;
+            w[t][r] = __builtin_amdgcn_fmed3f(
+                __builtin_fmaf(-s2, __builtin_amdgcn_sqrtf(fabsf(s2)), 1.0f), 0.0f, 1.0f);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        float4 a2[kCov ? 3 : 1];
+#pragma unroll
+        for (int g = 0; g < (kCov ? 3 : 1); ++g)
+            a2[g] = *reinterpret_cast<const float4*>(a2p + (4 * g) * kStride + 16 * t);
+#pragma unroll
+        for (int g = 0; g < (kCov ? 3 : 1); ++g) acc[g][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[g].x, w[t][0], acc[g][0], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < (kCov ? 3 : 1); ++g) acc[g][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[g].y, w[t][1], acc[g][0], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < (kCov ? 3 : 1); ++g) acc[g][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[g].z, w[t][2], acc[g][0], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < (kCov ? 3 : 1); ++g) acc[g][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a2[g].w, w[t][3], acc[g][0], 0, 0, 0);
     }
 }
 
@@ -559,7 +605,7 @@ __device__ __forceinline__ void nb_chunk(float* __restrict__ q, const float* __r
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            nb_tiles<kCov, NT>(q + head, 64u, b1, acc, cnt, le_s2);
+            nb_tiles<kCov, NT, kNbStride>(q + head, 64u, b1, acc, cnt, le_s2);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -584,7 +630,7 @@ __device__ __forceinline__ void nb_chunk(float* __restrict__ q, const float* __r
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        nb_tiles<kCov, NT>(q + head, n, b1, acc, cnt, le_s2);
+        nb_tiles<kCov, NT, kNbStride>(q + head, n, b1, acc, cnt, le_s2);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -702,21 +748,221 @@ struct NbLds {
     float vtx[4][64];
 };
 
+// One workgroup per chunk, for frames with few chunks.  A wave per chunk takes a
+// chunk's whole latency (some 180 staging rounds of dependent loads and up to
+// 4 tiles per 16 candidates, one after another) even when most of the chip is
+// idle: 31,000 particles are 600 chunks for 4096 wave slots.  Here the 4 waves
+// of a workgroup share a chunk: each stages a quarter of a 256-candidate round
+// into one LDS ring, in candidate order, and each evaluates one of the chunk's
+// 16-particle tiles.  The chunk's box, the kept candidates, their order and
+// every tile's operations are those of the wave-per-chunk form, so the results
+// are the same bits.  Per round two barriers: counts (which also says that the
+// previous round's batches are evaluated), and entries.
+//
+// Which form (nch chunks, G workgroups): the shared form up to nch = 3 G, i.e.
+// while a wave per chunk would leave a quarter of the 4 G wave slots empty.
+// Dam-break frames, smoothing / covariance, wave per chunk -> workgroup per
+// chunk: 31k particles (0.5 G) 184 / 234 -> 86 / 147 us; 125k (2.1 / 2.6 G) 387 /
+// 563 -> 245 / 432 us; 244k (4.2 / 5.2 G) 424 / 614 -> 479 / 737 us.  Frames
+// of a batch share the chip, so a lane's limit is divided by the frames in
+// flight (coop_limit): 8 Yu13 frames of 60k particles took 3% longer with the
+// whole limit, 4 of 30k are 24% faster either way.
+constexpr int kCoopQueue = 512;   // ring entries: 63 waiting + 256 new, 256 being read
+constexpr int kCoopStride = kCoopQueue + 16;
+template <bool kCov>
+struct NbCoopLds {
+    float queue[NbRows<kCov>::kRows * kCoopStride];
+    float vtx[kAnisoThreads / 64][4][64];
+    uint32_t count[kAnisoThreads / 64];
+};
+
+__device__ __forceinline__ uint32_t coop_chunk(uint32_t i, uint32_t nch) {
+    // workgroup i % 8 runs on XCD i % 8: each XCD takes a contiguous eighth
+    const uint32_t per = (nch + 7u) >> 3;
+    const uint32_t k = i >> 3;
+    return k < per ? (i & 7u) * per + k : nch;
+}
+
+// Tile `wave` of a chunk of `tiles` 16-particle tiles: as nb_chunk; lane l gets
+// the sums of the tile's particle l % 16.
+template <bool kCov>
+__device__ __forceinline__ void nb_coop(NbCoopLds<kCov>& L, uint32_t wave, uint32_t tiles,
+                                        const float4* __restrict__ sorted, BlockRows& br,
+                                        float ox, float oy, float oz, const float* bb0,
+                                        const float* bb1, float inv_r2, float cull2, float le_s2,
+                                        uint32_t& n_kept, v4f& s1, v4f& s2a, v4f& s2b,
+                                        uint32_t& count) {
+    const uint32_t lane = __lane_id();
+    constexpr int G = kCov ? 3 : 1;
+    const uint32_t total = br.total;
+    float* q = L.queue;
+    const bool mine = wave < tiles;
+    float b1[1];
+    v4f acc[G][1];
+    uint32_t cnt[1] = {0};
+    b1[0] = L.vtx[wave][lane >> 4][16u * wave + (lane & 15u)];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g][0] = v4f{0.f, 0.f, 0.f, 0.f};
+    uint32_t head = 0, fill = 0;
+    float4 next = make_float4(0.f, 0.f, 0.f, 0.f);
+    {
+        const uint32_t off = br.offset(64u * wave, 64u * wave + lane);
+        if (64u * wave + lane < total) next = sorted[off + 64u * wave + lane];
+    }
+    for (uint32_t base = 0; base < total; base += 256u) {
+        const uint32_t g = base + 64u * wave + lane;
+        const float4 cand = next;
+        if (base + 256u < total) {
+            const uint32_t off = br.offset(base + 256u + 64u * wave, g + 256u);
+            if (g + 256u < total) next = sorted[off + g + 256u];
+        }
+        bool keep = false;
+        float px = 0.f, py = 0.f, pz = 0.f;
+        if (g < total) {
+            px = cand.x - ox;
+            py = cand.y - oy;
+            pz = cand.z - oz;
+            keep = box_dist2(px, py, pz, bb0, bb1) < cull2;
+        }
+        const uint64_t m = __ballot(keep);
+        if (lane == 0) L.count[wave] = (uint32_t)__popcll(m);
+        __syncthreads();
+        uint32_t before = 0, added = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kAnisoThreads / 64; ++w) {
+            const uint32_t c = L.count[w];
+            before += w < wave ? c : 0u;
+            added += c;
+        }
+        if (keep) {
+            const uint32_t slot = (head + fill + before + mask_rank(m)) & (kCoopQueue - 1);
+            q[slot] = px;
+            q[kCoopStride + slot] = py;
+            q[2 * kCoopStride + slot] = pz;
+            q[NbRows<kCov>::kQ * kCoopStride + slot] =
+                __builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px)) * inv_r2;
+            if (kCov) {
+                q[(kNbXX + 0) * kCoopStride + slot] = px * px;
+                q[(kNbXX + 1) * kCoopStride + slot] = px * py;
+                q[(kNbXX + 2) * kCoopStride + slot] = px * pz;
+                q[(kNbXX + 3) * kCoopStride + slot] = py * py;
+                q[(kNbYZ + 0) * kCoopStride + slot] = py * pz;
+                q[(kNbYZ + 1) * kCoopStride + slot] = pz * pz;
+            }
+        }
+        fill += added;
+        n_kept += wave == 0 ? added : 0u;
+        __syncthreads();
+        for (; fill >= 64u; fill -= 64u) {
+            if (mine) nb_tile64<kCov, kCoopStride>(q + head, b1[0], acc, cnt[0], le_s2);
+            head = (head + 64u) & (kCoopQueue - 1);
+        }
+    }
+    if (fill) {
+        // pad to a multiple of 16 with entries of weight 0 and no count
+        // (s2 = 1e30); head is a multiple of 64, so the pad does not wrap
+        const uint32_t n = (fill + 15u) & ~15u;
+        if (wave == 0 && lane >= fill && lane < n) {
+            q[head + lane] = 0.f;
+            q[kCoopStride + head + lane] = 0.f;
+            q[2 * kCoopStride + head + lane] = 0.f;
+            q[NbRows<kCov>::kQ * kCoopStride + head + lane] = 1.0e30f;
+            if (kCov) {
+#pragma unroll
+                for (int k = 0; k < 6; ++k) q[(kNbXX + k) * kCoopStride + head + lane] = 0.f;
+            }
+        }
+        __syncthreads();
+        if (mine) nb_tiles<kCov, 1, kCoopStride>(q + head, n, b1, acc, cnt, le_s2);
+    }
+    // the next chunk rewrites the ring from its start, and the vertex operands
+    __syncthreads();
+    s1 = acc[0][0];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s1[c] = nb_reduce4(s1[c]);
+    s2a = v4f{0.f, 0.f, 0.f, 0.f};
+    s2b = s2a;
+    count = 0;
+    if (kCov) {
+        s2a = acc[G - 2][0];
+        s2b = acc[G - 1][0];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s2a[c] = nb_reduce4(s2a[c]);
+        s2b[0] = nb_reduce4(s2b[0]);
+        s2b[1] = nb_reduce4(s2b[1]);
+        count = nb_reduce4_u(cnt[0]);
+    }
+}
+
+// The smoothed and mean position of a particle from its sums.
+__device__ __forceinline__ void smooth_store(const v4f& s1, const float* o, float lambda,
+                                             const float4& self, uint32_t i,
+                                             float4* __restrict__ mean_out,
+                                             float4* __restrict__ smooth_out) {
+    if (!(s1[3] > 0.0f)) return;
+    const float inv = 1.0f / s1[3];
+    const float mx = o[0] + s1[0] * inv, my = o[1] + s1[1] * inv, mz = o[2] + s1[2] * inv;
+    mean_out[i] = make_float4(mx, my, mz, 0.0f);
+    const float a = 1.0f - lambda;
+    smooth_out[i] = make_float4(a * self.x + lambda * mx, a * self.y + lambda * my,
+                                a * self.z + lambda * mz, 0.0f);
+}
+
+template <bool kCoop>
 __global__ __launch_bounds__(kAnisoThreads, 5) void k_smooth_mc(
     const float4* __restrict__ sorted, const fsr_index_range* __restrict__ ranges, GridDev sp,
     float radius, float lambda, ChunkList cl, const float4* __restrict__ cell_box,
-    float4* __restrict__ mean_out, float4* __restrict__ smooth_out, uint32_t* __restrict__ work) {
-    __shared__ __align__(16) NbLds<false> lds[kAnisoThreads / 64];
+    float4* __restrict__ mean_out, float4* __restrict__ smooth_out, uint32_t* __restrict__ work,
+    uint32_t coop_max) {
+    __shared__ __align__(16) union {
+        NbLds<false> wave[kAnisoThreads / 64];
+        NbCoopLds<false> group;
+    } lds;
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
-    float* q = lds[wave].queue;
-    float* vt = &lds[wave].vtx[0][0];
-    q[kNbOne * kNbStride + lane] = 1.0f;
-    q[kNbOne * kNbStride + 64 + lane] = 1.0f;
     const uint32_t nch = *cl.num_chunks;
     const float inv_r2 = 1.0f / (radius * radius);
-    uint32_t step = 0;
+    const float c2 = radius * radius * kRadiusCull;
     uint32_t n_staged = 0, n_kept = 0;
+    if (kCoop && nch <= coop_max) {
+        NbCoopLds<false>& L = lds.group;
+        for (uint32_t t = threadIdx.x; t < (uint32_t)kCoopQueue; t += kAnisoThreads)
+            L.queue[kNbOne * kCoopStride + t] = 1.0f;
+        // workgroup-uniform
+        for (uint32_t turn = blockIdx.x; turn < ((nch + 7u) & ~7u); turn += gridDim.x) {
+            const uint32_t ch = coop_chunk(turn, nch);
+            if (ch >= nch) continue;
+            const uint32_t c = cl.chunk_cell[ch];
+            const uint32_t k = ch - cl.chunk_off[c];
+            const fsr_index_range own = ranges[c];
+            const uint32_t i = own.start + 64u * k + lane;
+            const bool live = i < own.end;
+            const int cx = (int)(c % sp.rx), cy = (int)((c / sp.rx) % sp.ry),
+                      cz = (int)(c / (sp.rx * sp.ry));
+            float4 self = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (live) self = sorted[i];
+            float o[3], bb0[3], bb1[3], rel[3];
+            nb_setup(live, self.x, self.y, self.z, inv_r2, &L.vtx[wave][0][0], o, bb0, bb1, rel);
+            const CellCull cc = chunk_cull(cell_box, sp.rx * sp.ry * sp.rz, o, bb0, bb1);
+            BlockRows br = block_rows<2>(ranges, sp, cx, cy, cz, &cc);
+            wave_lds_sync();
+            n_staged += wave == 0 ? br.total : 0u;
+            v4f s1, s2a, s2b;
+            uint32_t count;
+            const uint32_t cnt = min(64u, own.end - (own.start + 64u * k));
+            nb_coop<false>(L, wave, (cnt + 15u) >> 4, sorted, br, o[0], o[1], o[2], bb0, bb1,
+                           inv_r2, c2, 0.f, n_kept, s1, s2a, s2b, count);
+            if (live && (lane >> 4) == wave)
+                smooth_store(s1, o, lambda, self, i, mean_out, smooth_out);
+        }
+        if (work) write_work(work, n_staged, n_kept);
+        return;
+    }
+    float* q = lds.wave[wave].queue;
+    float* vt = &lds.wave[wave].vtx[0][0];
+    q[kNbOne * kNbStride + lane] = 1.0f;
+    q[kNbOne * kNbStride + 64 + lane] = 1.0f;
+    uint32_t step = 0;
     for (;;) {
         const uint32_t ch = next_item_xcd(cl.next, nch, step);
         if (ch >= nch) break;
@@ -735,52 +981,100 @@ __global__ __launch_bounds__(kAnisoThreads, 5) void k_smooth_mc(
         BlockRows br = block_rows<2>(ranges, sp, cx, cy, cz, &cc);
         const uint32_t total = br.total;
         n_staged += total;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
         v4f s1, s2a, s2b;
         uint32_t count;
         const uint32_t cnt = min(64u, own.end - (own.start + 64u * k));
-        const float c2 = radius * radius * kRadiusCull;
         switch ((cnt + 15u) >> 4) {
             case 1: nb_chunk<false, 1>(q, vt, sorted, br, total, o[0], o[1], o[2], bb0, bb1, inv_r2, c2, 0.f, n_kept, s1, s2a, s2b, count); break;
             case 2: nb_chunk<false, 2>(q, vt, sorted, br, total, o[0], o[1], o[2], bb0, bb1, inv_r2, c2, 0.f, n_kept, s1, s2a, s2b, count); break;
             case 3: nb_chunk<false, 3>(q, vt, sorted, br, total, o[0], o[1], o[2], bb0, bb1, inv_r2, c2, 0.f, n_kept, s1, s2a, s2b, count); break;
             default: nb_chunk<false, 4>(q, vt, sorted, br, total, o[0], o[1], o[2], bb0, bb1, inv_r2, c2, 0.f, n_kept, s1, s2a, s2b, count); break;
         }
-        if (live && s1[3] > 0.0f) {
-            const float inv = 1.0f / s1[3];
-            const float mx = o[0] + s1[0] * inv, my = o[1] + s1[1] * inv, mz = o[2] + s1[2] * inv;
-            mean_out[i] = make_float4(mx, my, mz, 0.0f);
-            const float a = 1.0f - lambda;
-            smooth_out[i] = make_float4(a * self.x + lambda * mx, a * self.y + lambda * my,
-                                        a * self.z + lambda * mz, 0.0f);
-        }
-        (void)rel;
+        if (live) smooth_store(s1, o, lambda, self, i, mean_out, smooth_out);
     }
     if (work) write_work(work, n_staged, n_kept);
 }
 
-__global__ __launch_bounds__(kAnisoThreads, 4) void k_covariance_mc(CovArgs a, ChunkList cl) {
-    __shared__ __align__(16) NbLds<true> lds[kAnisoThreads / 64];
+// sum w v v^T with v = q'' - m'' from the moments about the chunk's origin, and
+// G of the particle.
+__device__ __forceinline__ void cov_store(const CovArgs& a, const v4f& s1, const v4f& s2a,
+                                          const v4f& s2b, const float* rel, uint32_t count,
+                                          uint32_t gi, uint32_t i) {
+    const float mx = rel[0], my = rel[1], mz = rel[2];
+    const float sw = s1[3];
+    const float sx = s1[0], sy = s1[1], sz = s1[2];
+    const float c00 = s2a[0] - 2.0f * sx * mx + sw * mx * mx;
+    const float c01 = s2a[1] - sx * my - sy * mx + sw * mx * my;
+    const float c02 = s2a[2] - sx * mz - sz * mx + sw * mx * mz;
+    const float c11 = s2a[3] - 2.0f * sy * my + sw * my * my;
+    const float c12 = s2b[0] - sy * mz - sz * my + sw * my * mz;
+    const float c22 = s2b[1] - 2.0f * sz * mz + sw * mz * mz;
+    cov_finish(a, gi, i, count, sw, c00, c01, c02, c11, c12, c22);
+}
+
+template <bool kCoop>
+__global__ __launch_bounds__(kAnisoThreads, 4) void k_covariance_mc(CovArgs a, ChunkList cl,
+                                                                     uint32_t coop_max) {
+    __shared__ __align__(16) union {
+        NbLds<true> wave[kAnisoThreads / 64];
+        NbCoopLds<true> group;
+    } lds;
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
-    float* q = lds[wave].queue;
-    float* vt = &lds[wave].vtx[0][0];
-    q[kNbOne * kNbStride + lane] = 1.0f;
-    q[kNbOne * kNbStride + 64 + lane] = 1.0f;
-    q[kNbZero * kNbStride + lane] = 0.0f;
-    q[kNbZero * kNbStride + 64 + lane] = 0.0f;
-    q[(kNbZero + 1) * kNbStride + lane] = 0.0f;
-    q[(kNbZero + 1) * kNbStride + 64 + lane] = 0.0f;
     const uint32_t nch = *cl.num_chunks;
     const float r = a.radius;
     const float inv_r2 = 1.0f / (r * r);
     const float c2 = r * r * kRadiusCull;
     // the neighbour test |q - m| <= r on s2 = |q - m|^2 / r^2
     const float le_s2 = a.d2_le_r * inv_r2;
-    uint32_t step = 0;
     uint32_t n_staged = 0, n_kept = 0;
+    if (kCoop && nch <= coop_max) {
+        NbCoopLds<true>& L = lds.group;
+        for (uint32_t t = threadIdx.x; t < (uint32_t)kCoopQueue; t += kAnisoThreads) {
+            L.queue[kNbOne * kCoopStride + t] = 1.0f;
+            L.queue[kNbZero * kCoopStride + t] = 0.0f;
+            L.queue[(kNbZero + 1) * kCoopStride + t] = 0.0f;
+        }
+        // workgroup-uniform
+        for (uint32_t turn = blockIdx.x; turn < ((nch + 7u) & ~7u); turn += gridDim.x) {
+            const uint32_t ch = coop_chunk(turn, nch);
+            if (ch >= nch) continue;
+            const uint32_t c = cl.chunk_cell[ch];
+            const uint32_t k = ch - cl.chunk_off[c];
+            const fsr_index_range own = a.ranges[c];
+            const uint32_t i = own.start + 64u * k + lane;
+            const bool live = i < own.end;
+            const int cx = (int)(c % a.sp.rx), cy = (int)((c / a.sp.rx) % a.sp.ry),
+                      cz = (int)(c / (a.sp.rx * a.sp.ry));
+            float4 m = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (live) m = a.mean[i];
+            float o[3], bb0[3], bb1[3], rel[3];
+            nb_setup(live, m.x, m.y, m.z, inv_r2, &L.vtx[wave][0][0], o, bb0, bb1, rel);
+            const CellCull cc = chunk_cull(a.cell_box, a.sp.rx * a.sp.ry * a.sp.rz, o, bb0, bb1);
+            BlockRows br = block_rows<2>(a.ranges, a.sp, cx, cy, cz, &cc);
+            wave_lds_sync();
+            n_staged += wave == 0 ? br.total : 0u;
+            v4f s1, s2a, s2b;
+            uint32_t count;
+            const uint32_t cnt = min(64u, own.end - (own.start + 64u * k));
+            nb_coop<true>(L, wave, (cnt + 15u) >> 4, a.sorted, br, o[0], o[1], o[2], bb0, bb1,
+                          inv_r2, c2, le_s2, n_kept, s1, s2a, s2b, count);
+            if (live && (lane >> 4) == wave)
+                cov_store(a, s1, s2a, s2b, rel, count, a.involve_off[c] + (i - own.start), i);
+        }
+        if (a.work) write_work(a.work, n_staged, n_kept);
+        return;
+    }
+    float* q = lds.wave[wave].queue;
+    float* vt = &lds.wave[wave].vtx[0][0];
+    q[kNbOne * kNbStride + lane] = 1.0f;
+    q[kNbOne * kNbStride + 64 + lane] = 1.0f;
+    q[kNbZero * kNbStride + lane] = 0.0f;
+    q[kNbZero * kNbStride + 64 + lane] = 0.0f;
+    q[(kNbZero + 1) * kNbStride + lane] = 0.0f;
+    q[(kNbZero + 1) * kNbStride + 64 + lane] = 0.0f;
+    uint32_t step = 0;
     for (;;) {
         const uint32_t ch = next_item_xcd(cl.next, nch, step);
         if (ch >= nch) break;
@@ -800,9 +1094,7 @@ __global__ __launch_bounds__(kAnisoThreads, 4) void k_covariance_mc(CovArgs a, C
         BlockRows br = block_rows<2>(a.ranges, a.sp, cx, cy, cz, &cc);
         const uint32_t total = br.total;
         n_staged += total;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
         v4f s1, s2a, s2b;
         uint32_t count;
         const uint32_t cnt = min(64u, own.end - (own.start + 64u * k));
@@ -812,20 +1104,7 @@ __global__ __launch_bounds__(kAnisoThreads, 4) void k_covariance_mc(CovArgs a, C
             case 3: nb_chunk<true, 3>(q, vt, a.sorted, br, total, o[0], o[1], o[2], bb0, bb1, inv_r2, c2, le_s2, n_kept, s1, s2a, s2b, count); break;
             default: nb_chunk<true, 4>(q, vt, a.sorted, br, total, o[0], o[1], o[2], bb0, bb1, inv_r2, c2, le_s2, n_kept, s1, s2a, s2b, count); break;
         }
-        if (live) {
-            // sum w v v^T with v = q'' - m'' from the moments about the origin
-            const float mx = rel[0], my = rel[1], mz = rel[2];
-            const float sw = s1[3];
-            const float sx = s1[0], sy = s1[1], sz = s1[2];
-            const float c00 = s2a[0] - 2.0f * sx * mx + sw * mx * mx;
-            const float c01 = s2a[1] - sx * my - sy * mx + sw * mx * my;
-            const float c02 = s2a[2] - sx * mz - sz * mx + sw * mx * mz;
-            const float c11 = s2a[3] - 2.0f * sy * my + sw * my * my;
-            const float c12 = s2b[0] - sy * mz - sz * my + sw * my * mz;
-            const float c22 = s2b[1] - 2.0f * sz * mz + sw * mz * mz;
-            cov_finish(a, a.involve_off[c] + (i - own.start), i, count, sw, c00, c01, c02, c11,
-                       c12, c22);
-        }
+        if (live) cov_store(a, s1, s2a, s2b, rel, count, a.involve_off[c] + (i - own.start), i);
     }
     if (a.work) write_work(a.work, n_staged, n_kept);
 }
@@ -1425,9 +1704,11 @@ fsr_status aniso_smooth(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     FSR_TRY(reset_xcd(a.counters, s));
     uint32_t* work;
     FSR_TRY(work_section(ctx, WORK_SMOOTH, &work));
-    hipLaunchKernelGGL(k_smooth_mc, dim3(blocks), dim3(kAnisoThreads), 0, s, a.sorted,
-                       a.ranges, a.sp, a.aniso_radius, a.lambda, cl, box, a.mean, a.smooth,
-                       work);
+    // at least n / 64 chunks: a large frame takes the build without the shared form
+    const uint32_t coop_max = coop_limit(ctx, blocks);
+    auto smooth = a.n / 64u <= coop_max ? k_smooth_mc<true> : k_smooth_mc<false>;
+    hipLaunchKernelGGL(smooth, dim3(blocks), dim3(kAnisoThreads), 0, s, a.sorted, a.ranges, a.sp,
+                       a.aniso_radius, a.lambda, cl, box, a.mean, a.smooth, work, coop_max);
     FSR_LAUNCH_CHECK("k_smooth_mc");
     return FSR_OK;
 }
@@ -1481,7 +1762,9 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     FSR_TRY(work_section(ctx, WORK_COV, &ca.work));
     FSR_TRY(cell_boxes(ctx, a, s, &ca.cell_box));
     FSR_TRY(reset_xcd(a.counters, s));
-    hipLaunchKernelGGL(k_covariance_mc, dim3(blocks_cov), dim3(kAnisoThreads), 0, s, ca, cl2);
+    // the chunks hold the involved particles only, so the test is on the device
+    hipLaunchKernelGGL(k_covariance_mc<true>, dim3(blocks_cov), dim3(kAnisoThreads), 0, s, ca, cl2,
+                       coop_limit(ctx, blocks_cov));
     FSR_LAUNCH_CHECK("k_covariance_mc");
     return FSR_OK;
 }

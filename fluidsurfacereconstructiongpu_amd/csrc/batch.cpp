@@ -79,6 +79,9 @@ std::vector<std::pair<uint32_t, uint32_t>> schedule(const fsr_frame_desc* frames
 fsr_status enqueue(fsr_batch* b, fsr_method method, const fsr_aniso_param* aniso,
                    const fsr_frame_desc* frames, uint32_t n, uint64_t* ts) {
     const uint32_t L = (uint32_t)b->lanes.size();
+    // frames that really run side by side: one per lane, at most one per
+    // hardware queue (4)
+    for (fsr_context* c : b->lanes) c->in_flight = (int)std::max(1u, std::min(std::min(L, n), 4u));
     FSR_HIP(hipEventRecord(b->fork, b->origin));
     for (uint32_t l = 0; l < L; ++l) FSR_HIP(hipStreamWaitEvent(b->streams[l], b->fork, 0));
     for (const auto& fl : schedule(frames, n, L)) {

@@ -70,6 +70,10 @@ int persistent_blocks(fsr_context* ctx, int threads, int per_cu, TuneClass cls) 
     return std::max(1, ctx->num_cus * (t > 0 ? std::min(t, per_cu) : per_cu));
 }
 
+uint32_t coop_limit(const fsr_context* ctx, int blocks) {
+    return 3u * (uint32_t)blocks / (uint32_t)std::max(1, ctx->in_flight);
+}
+
 static fsr_status check_grid(const fsr_grid_info* g, const char* name) {
     if (!g) {
         set_error(std::string(name) + " is null");

@@ -301,6 +301,7 @@ struct fsr_context {
     bool capturing = false;                  // inside a graph capture: no arena growth
     bool save_adjoint = false;               // frames keep what the adjoint needs
     int surface_mode = 0;                    // fsr_surface_mode of ZB05 / Akinci12 frames
+    int in_flight = 1;                       // frames that share the GPU (lanes of a batch)
     fsr::AdjointState adj;
     fsr::Arena arena;
     // stage profiling: ring of (FSR_NUM_STAGES + 1) events per frame
@@ -565,6 +566,9 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
 // Grid of a persistent kernel: CUs x workgroups per CU (the tuned value of
 // `cls` when set, else `per_cu`).
 int persistent_blocks(fsr_context* ctx, int threads, int per_cu, TuneClass cls);
+// Most chunks for which a neighbour kernel of `blocks` workgroups of 4 waves
+// shares each chunk among a workgroup's waves.
+uint32_t coop_limit(const fsr_context* ctx, int blocks);
 
 // util.hip: writes the 100 MHz device clock (s_memrealtime) to *out
 fsr_status device_timestamp(uint64_t* out, hipStream_t s);
