@@ -263,18 +263,6 @@ struct FieldBackArgs {
     float* g_pos;                 // float3[N], caller order
 };
 
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
 // The gather evaluates its pairs in 16 x 16 particle/vertex tiles on the
 // matrix cores (as the forward field): per 16 staged vertices and 16
 // particles of the chunk
@@ -415,9 +403,10 @@ __global__ __launch_bounds__(kAdjThreads, 4) void k_field_zb05_backward_mc(Field
         vb[64 + lane] = 2.0f * py * inv_r2;
         vb[128 + lane] = 2.0f * pz * inv_r2;
         vb[192 + lane] = 1.0f - __builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px)) * inv_r2;
-        const float bx0 = wave_min(live ? px : 3.0e38f), bx1 = wave_max(live ? px : -3.0e38f);
-        const float by0 = wave_min(live ? py : 3.0e38f), by1 = wave_max(live ? py : -3.0e38f);
-        const float bz0 = wave_min(live ? pz : 3.0e38f), bz1 = wave_max(live ? pz : -3.0e38f);
+        float bx0, bx1, by0, by1, bz0, bz1;
+        wave_range(live, px, &bx0, &bx1);
+        wave_range(live, py, &by0, &by1);
+        wave_range(live, pz, &bz0, &bz1);
         wave_lds_sync();
 
         auto chunk = [&](auto ntc) {

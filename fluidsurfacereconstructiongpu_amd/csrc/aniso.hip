@@ -204,18 +204,6 @@ __device__ __forceinline__ void write_work(uint32_t* __restrict__ sec, uint32_t 
 }
 
 // ---------------------------------------------------------------- K10 -------
-__device__ __forceinline__ float wave_minf(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
-__device__ __forceinline__ float wave_maxf(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
 // Squared distance from (x, y, z) to the box [b0, b1].
 __device__ __forceinline__ float box_dist2(float x, float y, float z, const float* b0,
                                            const float* b1) {
@@ -229,9 +217,9 @@ __device__ __forceinline__ float box_dist2(float x, float y, float z, const floa
 // Bounding box of the live lanes' points.
 __device__ __forceinline__ void wave_box(bool live, float x, float y, float z, float* b0,
                                          float* b1) {
-    b0[0] = wave_minf(live ? x : 3.0e38f); b1[0] = wave_maxf(live ? x : -3.0e38f);
-    b0[1] = wave_minf(live ? y : 3.0e38f); b1[1] = wave_maxf(live ? y : -3.0e38f);
-    b0[2] = wave_minf(live ? z : 3.0e38f); b1[2] = wave_maxf(live ? z : -3.0e38f);
+    wave_range(live, x, &b0[0], &b1[0]);
+    wave_range(live, y, &b0[1], &b1[1]);
+    wave_range(live, z, &b0[2], &b1[2]);
 }
 
 // Candidates farther than r * (1 + 5e-4) from the bounding box of a chunk's
@@ -711,8 +699,8 @@ __global__ __launch_bounds__(64) void k_cell_box(const fsr_index_range* __restri
             u.x = fmaxf(u.x, p.x); u.y = fmaxf(u.y, p.y); u.z = fmaxf(u.z, p.z);
         }
     }
-    l.x = wave_minf(l.x); l.y = wave_minf(l.y); l.z = wave_minf(l.z);
-    u.x = wave_maxf(u.x); u.y = wave_maxf(u.y); u.z = wave_maxf(u.z);
+    l.x = wave_min_f(l.x); l.y = wave_min_f(l.y); l.z = wave_min_f(l.z);
+    u.x = wave_max_f(u.x); u.y = wave_max_f(u.y); u.z = wave_max_f(u.z);
     if (lane == 0) {
         if (r.start != 0xFFFFFFFFu && r.end > r.start) {
             l.w = w;
@@ -1182,18 +1170,6 @@ __device__ __forceinline__ double noninv_poly(const double* __restrict__ m, doub
     return A * (A * (A * m[0] + 3.0 * sB) + 3.0 * sB2) + sB3;
 }
 
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
 // LDS queue of one field wave: a ring of kAfQueue staged candidates, stored
 // as rows of kAfStride floats (structure of arrays).  Rows 0-3 and 4-7 are the
 // A operands of the two matrix products, (M00, M11, M22, M01) and (M02, M12,
@@ -1300,9 +1276,10 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
         vt[6 * kAfStride + lane] = 2.0f * vx;
         vt[7 * kAfStride + lane] = 2.0f * vy;
         vt[8 * kAfStride + lane] = 2.0f * vz;
-        const float bx0 = wave_min(live ? vx : 3.0e38f), bx1 = wave_max(live ? vx : -3.0e38f);
-        const float by0 = wave_min(live ? vy : 3.0e38f), by1 = wave_max(live ? vy : -3.0e38f);
-        const float bz0 = wave_min(live ? vz : 3.0e38f), bz1 = wave_max(live ? vz : -3.0e38f);
+        float bx0, bx1, by0, by1, bz0, bz1;
+        wave_range(live, vx, &bx0, &bx1);
+        wave_range(live, vy, &by0, &by1);
+        wave_range(live, vz, &bz0, &bz1);
         // the block's candidate rows; with the non-involved moments only the
         // cells whose involved particles can reach the chunk's vertices
         BlockRows br;
@@ -1534,9 +1511,9 @@ __global__ __launch_bounds__(64) void k_cell_moments_boxes(
         }
     }
     if (lane < (uint32_t)kNonInvMoments) mom[(uint64_t)c * kNonInvMoments + lane] = acc;
-    l.x = wave_minf(l.x); l.y = wave_minf(l.y); l.z = wave_minf(l.z);
-    u.x = wave_maxf(u.x); u.y = wave_maxf(u.y); u.z = wave_maxf(u.z);
-    l.w = wave_maxf(l.w);
+    l.x = wave_min_f(l.x); l.y = wave_min_f(l.y); l.z = wave_min_f(l.z);
+    u.x = wave_max_f(u.x); u.y = wave_max_f(u.y); u.z = wave_max_f(u.z);
+    l.w = wave_max_f(l.w);
     if (lane == 0) {
         if (l.w > 0.0f) {
             l.w = l.w * 1.002f + 1.0e-12f;

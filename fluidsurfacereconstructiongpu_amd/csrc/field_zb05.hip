@@ -64,27 +64,6 @@ __device__ __forceinline__ float swz_xor(float v) {
     return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x1F | (M << 10)));
 }
 
-// Minimum / maximum over the wave, returned in a scalar register.
-__device__ __forceinline__ float wave_min_u(float v) {
-    v = fminf(v, swz_xor<1>(v));
-    v = fminf(v, swz_xor<2>(v));
-    v = fminf(v, swz_xor<4>(v));
-    v = fminf(v, swz_xor<8>(v));
-    v = fminf(v, swz_xor<16>(v));
-    return fminf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)),
-                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32)));
-}
-
-__device__ __forceinline__ float wave_max_u(float v) {
-    v = fmaxf(v, swz_xor<1>(v));
-    v = fmaxf(v, swz_xor<2>(v));
-    v = fmaxf(v, swz_xor<4>(v));
-    v = fmaxf(v, swz_xor<8>(v));
-    v = fmaxf(v, swz_xor<16>(v));
-    return fmaxf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)),
-                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32)));
-}
-
 // Inclusive sum within each row of 16 lanes (DPP row shifts; lanes whose
 // source lies before the row start add 0).
 __device__ __forceinline__ uint32_t row16_inclusive_sum(uint32_t v) {
@@ -365,9 +344,10 @@ __global__ __launch_bounds__(kFieldThreads, 6) void k_field_zb05(FieldArgs a, Ba
         vt[384 + lane] = 1.0f - __builtin_fmaf(vz, vz, __builtin_fmaf(vy, vy, vx * vx)) * inv_r2;
         // bounding box of the chunk's vertices
         const bool live = has_vertex;
-        const float bx0 = wave_min_u(live ? vx : 3.0e38f), bx1 = wave_max_u(live ? vx : -3.0e38f);
-        const float by0 = wave_min_u(live ? vy : 3.0e38f), by1 = wave_max_u(live ? vy : -3.0e38f);
-        const float bz0 = wave_min_u(live ? vz : 3.0e38f), bz1 = wave_max_u(live ? vz : -3.0e38f);
+        float bx0, bx1, by0, by1, bz0, bz1;
+        wave_range(live, vx, &bx0, &bx1);
+        wave_range(live, vy, &by0, &by1);
+        wave_range(live, vz, &bz0, &bz1);
         wave_lds_sync();
         const int nt = (int)((cnt + 15u) >> 4);
         // The rest of the chunk, compiled once per tile count NT, so that the

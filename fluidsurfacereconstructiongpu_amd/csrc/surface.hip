@@ -270,18 +270,6 @@ __global__ __launch_bounds__(256) void k_colorfield_tail(SurfaceArgs a, float ma
     block_count_add2(&a.st->num_surface_particles, n_surf, &a.st->band_exceptions, n_exc);
 }
 
-__device__ __forceinline__ float wave_minf(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
-__device__ __forceinline__ float wave_maxf(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-    return v;
-}
-
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -381,9 +369,10 @@ __global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, C
         };
         float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
         if (live) p = a.sorted[i];
-        const float bx0 = wave_minf(live ? p.x : 3.0e38f), bx1 = wave_maxf(live ? p.x : -3.0e38f);
-        const float by0 = wave_minf(live ? p.y : 3.0e38f), by1 = wave_maxf(live ? p.y : -3.0e38f);
-        const float bz0 = wave_minf(live ? p.z : 3.0e38f), bz1 = wave_maxf(live ? p.z : -3.0e38f);
+        float bx0, bx1, by0, by1, bz0, bz1;
+        wave_range(live, p.x, &bx0, &bx1);
+        wave_range(live, p.y, &by0, &by1);
+        wave_range(live, p.z, &bz0, &bz1);
         uint32_t count = 0, count_r = 0, kept = 0, fill = 0;
         float gx = 0.f, gy = 0.f, gz = 0.f;
         auto run = [&](uint32_t n) {
