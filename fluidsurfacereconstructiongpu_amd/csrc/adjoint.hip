@@ -32,7 +32,6 @@
 // Results are written in the caller's particle order through the sort
 // permutation; particles outside the hash grid get 0.
 #include "common.hpp"
-#include <type_traits>
 
 #include "mc_tables.h"
 
@@ -276,8 +275,9 @@ struct FieldBackArgs {
 // Vertices whose coefficient is zero, or that lie at least 1.00005 R from the
 // bounding box of the chunk's particles, add exactly 0 to every particle and
 // are dropped at staging (order-preserving compaction, as in the forward).
-constexpr int kAdjQueue = 128;
-constexpr int kAdjStride = 144;
+// The queue is a ring of kAdjQueue entries: 63 waiting + 256 new, 256 being read.
+constexpr int kAdjQueue = 512;
+constexpr int kAdjStride = kAdjQueue + 16;
 // rows: x', y', z', 1, ux, uy, uz, c - u.x', -|x'|^2/R^2
 constexpr int kAdjOne = 3, kAdjU = 4, kAdjQ = 8, kAdjRows = 9;
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -287,83 +287,80 @@ __device__ __forceinline__ float adj_swz_xor(float v) {
     return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x1F | (M << 10)));
 }
 
-template <int NT>
-__device__ __forceinline__ void adj_tiles(const float* __restrict__ rows, uint32_t n,
-                                          const float (&bt)[NT], const float (&bk)[NT],
-                                          v4f (&gu)[NT], v4f (&gx)[NT]) {
+// n staged vertices (a multiple of 16, from `rows`) against one 16-particle tile.
+__device__ __forceinline__ void adj_tile(const float* __restrict__ rows, uint32_t n, float bt,
+                                         float bk, v4f& gu, v4f& gx) {
     const uint32_t lane = __lane_id();
     const float* a1p = rows + (lane >> 4) * kAdjStride + (lane & 15u);
     const float* k1p = rows + (kAdjU + (lane >> 4)) * kAdjStride + (lane & 15u);
     const float* a2p = rows + (lane & 3u) * kAdjStride + 4u * (lane >> 4);
     const float* u2p = rows + (kAdjU + (lane & 3u)) * kAdjStride + 4u * (lane >> 4);
     const float* cqp = rows + kAdjQ * kAdjStride + 4u * (lane >> 4);
+    const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
     for (uint32_t tb = 0; tb < n; tb += 16u) {
-        const float a1 = a1p[tb];
-        const float k1 = k1p[tb];
         const float4 cq = *reinterpret_cast<const float4*>(cqp + tb);
-        const v4f c1 = v4f{cq.x, cq.y, cq.z, cq.w};
-        const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
-        v4f t[NT], kd[NT];
+        v4f t = __builtin_amdgcn_mfma_f32_16x16x4f32(a1p[tb], bt, v4f{cq.x, cq.y, cq.z, cq.w}, 0, 0, 0);
+        v4f kd = __builtin_amdgcn_mfma_f32_16x16x4f32(k1p[tb], bk, zero, 0, 0, 0);
 #pragma unroll
-        for (int T = 0; T < NT; ++T) t[T] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, bt[T], c1, 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) kd[T] = __builtin_amdgcn_mfma_f32_16x16x4f32(k1, bk[T], zero, 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float tp = __builtin_amdgcn_fmed3f(t[T][r], 0.0f, 1.0f);
-                const float t2 = tp * tp;
-                t[T][r] = t2 * tp;
-                kd[T][r] = kd[T][r] * t2;
-            }
+        for (int r = 0; r < 4; ++r) {
+            const float tp = __builtin_amdgcn_fmed3f(t[r], 0.0f, 1.0f);
+            const float t2 = tp * tp;
+            t[r] = t2 * tp;
+            kd[r] = kd[r] * t2;
         }
         const float4 au = *reinterpret_cast<const float4*>(u2p + tb);
         const float4 ax = *reinterpret_cast<const float4*>(a2p + tb);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gu[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(au.x, t[T][0], gu[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gu[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(au.y, t[T][1], gu[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gu[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(au.z, t[T][2], gu[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gu[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(au.w, t[T][3], gu[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gx[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.x, kd[T][0], gx[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gx[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.y, kd[T][1], gx[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gx[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.z, kd[T][2], gx[T], 0, 0, 0);
-#pragma unroll
-        for (int T = 0; T < NT; ++T) gx[T] = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.w, kd[T][3], gx[T], 0, 0, 0);
+        gu = __builtin_amdgcn_mfma_f32_4x4x1f32(au.x, t[0], gu, 0, 0, 0);
+        gu = __builtin_amdgcn_mfma_f32_4x4x1f32(au.y, t[1], gu, 0, 0, 0);
+        gu = __builtin_amdgcn_mfma_f32_4x4x1f32(au.z, t[2], gu, 0, 0, 0);
+        gu = __builtin_amdgcn_mfma_f32_4x4x1f32(au.w, t[3], gu, 0, 0, 0);
+        gx = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.x, kd[0], gx, 0, 0, 0);
+        gx = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.y, kd[1], gx, 0, 0, 0);
+        gx = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.z, kd[2], gx, 0, 0, 0);
+        gx = __builtin_amdgcn_mfma_f32_4x4x1f32(ax.w, kd[3], gx, 0, 0, 0);
     }
 }
 
-__global__ __launch_bounds__(kAdjThreads, 4) void k_field_zb05_backward_mc(FieldBackArgs a) {
-    struct WaveLds {
-        float queue[kAdjRows * kAdjStride];
-        float bt[4][64];   // per lane: (2p'/R^2, c0)
-    };
-    __shared__ __align__(16) WaveLds lds[kAdjThreads / 64];
+// A workgroup per chunk: its 4 waves stage a quarter each of a 256-vertex round
+// into one LDS ring, in candidate order, and each evaluates one of the chunk's
+// 16-particle tiles.  A chunk's work varies from nothing (no band vertex near)
+// to some 290 rounds of 64 vertices (a particle at the surface); with a wave per
+// chunk a SIMD that drew heavy ones ran long after the others had finished, and
+// a frame's few thousand chunks leave no others to level it.  Shared, a heavy
+// chunk loads all 4 SIMDs of a CU.  Per round two barriers: counts (which also
+// says that the previous batches are evaluated), and entries.  Bound by VALU and
+// matrix issue, then by the imbalance that is left.  Ball of n particles, wave
+// per chunk -> workgroup per chunk: 16k 354 -> 168 us, 64k 524 -> 297, 125k 760 ->
+// 405, 256k (192^3) 817 -> 564, 700k 1149 -> 1072.
+__global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(FieldBackArgs a) {
+    constexpr uint32_t kWaves = kAdjThreads / 64;
+    __shared__ __align__(16) float q[kAdjRows * kAdjStride];
+    __shared__ float bt_lds[kWaves][4][64];  // per lane: (2p'/R^2, c0)
+    __shared__ uint32_t count[kWaves];
+    __shared__ uint32_t next_chunk;
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nch = *a.num_chunks;
     const float inv_r2 = 1.0f / a.radius_sq;
     const float cull_r2 = a.radius_sq * 1.0001f;
-    float* q = lds[wave].queue;
-    float* vb = &lds[wave].bt[0][0];
-    q[kAdjOne * kAdjStride + lane] = 1.0f;
-    q[kAdjOne * kAdjStride + 64 + lane] = 1.0f;
+    float* vb = &bt_lds[wave][0][0];
+    for (uint32_t t = threadIdx.x; t < (uint32_t)kAdjQueue; t += kAdjThreads)
+        q[kAdjOne * kAdjStride + t] = 1.0f;
     uint32_t step = 0;
-    for (;;) {
-        const uint32_t ch = next_item_xcd(a.next, nch, step);
-        if (ch >= nch) break;
+    if (wave == 0) {
+        const uint32_t first = next_item_xcd(a.next, nch, step);
+        if (lane == 0) next_chunk = first;
+    }
+    __syncthreads();
+    // workgroup-uniform
+    for (uint32_t ch = next_chunk; ch < nch; ch = next_chunk) {
         const uint32_t c = a.chunk_cell[ch];
         const uint32_t k = ch - a.chunk_off[c];
         const fsr_index_range own = a.ranges[c];
         const uint32_t i = own.start + 64u * k + lane;
         const bool live = i < own.end;
         const uint32_t cnt = min(64u, own.end - (own.start + 64u * k));
+        const bool mine = wave < ((cnt + 15u) >> 4);
         const uint32_t qcx = c % a.sp.rx, qcy = (c / a.sp.rx) % a.sp.ry, qcz = c / (a.sp.rx * a.sp.ry);
 
         // 9 runs of band slots: virtual cells (q + radius) + {-1, 0, 1}^3
@@ -408,122 +405,110 @@ __global__ __launch_bounds__(kAdjThreads, 4) void k_field_zb05_backward_mc(Field
         wave_range(live, py, &by0, &by1);
         wave_range(live, pz, &bz0, &bz1);
         wave_lds_sync();
-
-        auto chunk = [&](auto ntc) {
-            constexpr int NT = decltype(ntc)::value;
-            float bt[NT], bk[NT];
-            v4f gu[NT], gx[NT];
-            const float* bsrc = vb + 64 * (lane >> 4) + (lane & 15u);
-            // (p', 1) of particle 16T + l%16, component l/16, from the LDS copy
-            // of 2p'/R^2 (times R^2 / 2) and a 1 for the fourth
+        v4f gu = v4f{0.f, 0.f, 0.f, 0.f}, gx = gu;
+        // (p', 1) of particle 16 wave + l%16, component l/16, from the LDS copy
+        // of 2p'/R^2 (times R^2 / 2) and a 1 for the fourth
+        const float bt = vb[64 * (lane >> 4) + 16u * wave + (lane & 15u)];
+        const float bk = (lane >> 4) == 3u ? 1.0f : bt * (0.5f * a.radius_sq);
+        uint32_t head = 0, fill = 0;
+        float4 ncf = make_float4(0.f, 0.f, 0.f, 0.f), nvp = ncf;
+        {
+            const uint32_t g0 = 64u * wave;
+            const uint32_t off = run_offset(g0, g0 + lane);
+            if (g0 + lane < total) {
+                ncf = a.coef[off + g0 + lane];
+                nvp = a.vpos[off + g0 + lane];
+            }
+        }
+        for (uint32_t base = 0; base < total; base += 256u) {
+            const uint32_t gi = base + 64u * wave + lane;
+            const float4 cf = ncf, vp = nvp;
+            if (base + 256u < total) {
+                const uint32_t off = run_offset(base + 256u + 64u * wave, gi + 256u);
+                if (gi + 256u < total) {
+                    ncf = a.coef[off + gi + 256u];
+                    nvp = a.vpos[off + gi + 256u];
+                }
+            }
+            bool keep = false;
+            float xx = 0.f, xy = 0.f, xz = 0.f;
+            if (gi < total && (cf.x != 0.0f || cf.y != 0.0f || cf.z != 0.0f || cf.w != 0.0f)) {
+                xx = vp.x - ox;
+                xy = vp.y - oy;
+                xz = vp.z - oz;
+                const float dx = xx - __builtin_amdgcn_fmed3f(xx, bx0, bx1);
+                const float dy = xy - __builtin_amdgcn_fmed3f(xy, by0, by1);
+                const float dz = xz - __builtin_amdgcn_fmed3f(xz, bz0, bz1);
+                keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull_r2;
+            }
+            const uint64_t m = __ballot(keep);
+            if (lane == 0) count[wave] = (uint32_t)__popcll(m);
+            __syncthreads();
+            uint32_t before = 0, added = 0;
 #pragma unroll
-            for (int T = 0; T < NT; ++T) {
-                bt[T] = bsrc[16 * T];
-                bk[T] = (lane >> 4) == 3u ? 1.0f : bt[T] * (0.5f * a.radius_sq);
-                gu[T] = v4f{0.f, 0.f, 0.f, 0.f};
-                gx[T] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (uint32_t w = 0; w < kWaves; ++w) {
+                const uint32_t n = count[w];
+                before += w < wave ? n : 0u;
+                added += n;
             }
-            uint32_t head = 0, fill = 0;
-            float4 ncf = make_float4(0.f, 0.f, 0.f, 0.f), nvp = ncf;
-            {
-                const uint32_t off = run_offset(0u, lane);
-                if (lane < total) {
-                    const uint32_t slot = off + lane;
-                    ncf = a.coef[slot];
-                    nvp = a.vpos[slot];
-                }
+            if (keep) {
+                const uint32_t slot = (head + fill + before + mask_rank(m)) & (kAdjQueue - 1);
+                q[slot] = xx;
+                q[kAdjStride + slot] = xy;
+                q[2 * kAdjStride + slot] = xz;
+                q[kAdjU * kAdjStride + slot] = cf.x;
+                q[(kAdjU + 1) * kAdjStride + slot] = cf.y;
+                q[(kAdjU + 2) * kAdjStride + slot] = cf.z;
+                q[(kAdjU + 3) * kAdjStride + slot] =
+                    cf.w - __builtin_fmaf(cf.z, xz, __builtin_fmaf(cf.y, xy, cf.x * xx));
+                q[kAdjQ * kAdjStride + slot] =
+                    -(__builtin_fmaf(xz, xz, __builtin_fmaf(xy, xy, xx * xx)) * inv_r2);
             }
-            for (uint32_t base = 0; base < total; base += 64u) {
-                const uint32_t gi = base + lane;
-                const float4 cf = ncf, vp = nvp;
-                if (base + 64u < total) {
-                    const uint32_t off = run_offset(base + 64u, gi + 64u);
-                    if (gi + 64u < total) {
-                        const uint32_t slot = off + gi + 64u;
-                        ncf = a.coef[slot];
-                        nvp = a.vpos[slot];
-                    }
-                }
-                bool keep = false;
-                float xx = 0.f, xy = 0.f, xz = 0.f;
-                if (gi < total && (cf.x != 0.0f || cf.y != 0.0f || cf.z != 0.0f || cf.w != 0.0f)) {
-                    xx = vp.x - ox;
-                    xy = vp.y - oy;
-                    xz = vp.z - oz;
-                    const float dx = xx - __builtin_amdgcn_fmed3f(xx, bx0, bx1);
-                    const float dy = xy - __builtin_amdgcn_fmed3f(xy, by0, by1);
-                    const float dz = xz - __builtin_amdgcn_fmed3f(xz, bz0, bz1);
-                    keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull_r2;
-                }
-                const uint64_t m = __ballot(keep);
-                if (keep) {
-                    const uint32_t slot = (head + fill + mask_rank(m)) & (kAdjQueue - 1);
-                    q[slot] = xx;
-                    q[kAdjStride + slot] = xy;
-                    q[2 * kAdjStride + slot] = xz;
-                    q[kAdjU * kAdjStride + slot] = cf.x;
-                    q[(kAdjU + 1) * kAdjStride + slot] = cf.y;
-                    q[(kAdjU + 2) * kAdjStride + slot] = cf.z;
-                    q[(kAdjU + 3) * kAdjStride + slot] =
-                        cf.w - __builtin_fmaf(cf.z, xz, __builtin_fmaf(cf.y, xy, cf.x * xx));
-                    q[kAdjQ * kAdjStride + slot] =
-                        -(__builtin_fmaf(xz, xz, __builtin_fmaf(xy, xy, xx * xx)) * inv_r2);
-                }
-                fill += (uint32_t)__popcll(m);
-                if (fill >= 64u) {
-                    wave_lds_sync();
-                    adj_tiles<NT>(q + head, 64u, bt, bk, gu, gx);
-                    wave_lds_sync();
-                    head ^= 64u;
-                    fill -= 64u;
-                }
+            fill += added;
+            __syncthreads();
+            for (; fill >= 64u; fill -= 64u) {
+                if (mine) adj_tile(q + head, 64u, bt, bk, gu, gx);
+                head = (head + 64u) & (kAdjQueue - 1);
             }
-            if (fill) {
-                // pad to 16 with entries that add 0: t < 0, u = 0
-                const uint32_t n = (fill + 15u) & ~15u;
-                if (lane >= fill && lane < n) {
+        }
+        // the next chunk, fetched under the last batch
+        if (wave == 0) {
+            const uint32_t nx = next_item_xcd(a.next, nch, step);
+            if (lane == 0) next_chunk = nx;
+        }
+        if (fill) {
+            // pad to 16 with entries that add 0: t < 0, u = 0 (head is a
+            // multiple of 64, so the pad does not wrap)
+            const uint32_t n = (fill + 15u) & ~15u;
+            if (wave == 0 && lane >= fill && lane < n) {
 #pragma unroll
-                    for (int rr = 0; rr < kAdjQ; ++rr)
-                        if (rr != kAdjOne) q[rr * kAdjStride + head + lane] = 0.f;
-                    q[kAdjQ * kAdjStride + head + lane] = -1.0e30f;
-                }
-                wave_lds_sync();
-                adj_tiles<NT>(q + head, n, bt, bk, gu, gx);
-                wave_lds_sync();
+                for (int rr = 0; rr < kAdjQ; ++rr)
+                    if (rr != kAdjOne) q[rr * kAdjStride + head + lane] = 0.f;
+                q[kAdjQ * kAdjStride + head + lane] = -1.0e30f;
             }
-            // the four partial sums of each particle; lane l keeps particle l
-            const uint32_t my = lane >> 4;
-            v4f su = gu[0], sx = gx[0];
+            __syncthreads();
+            if (mine) adj_tile(q + head, n, bt, bk, gu, gx);
+        }
+        // the next chunk rewrites the ring from its start
+        __syncthreads();
+        // the four partial sums of each particle; the lanes of the wave's tile
+        // write theirs
+        v4f su = gu, sx = gx;
 #pragma unroll
-            for (int T = 0; T < NT; ++T) {
-                v4f u4 = gu[T], x4 = gx[T];
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc) {
-                    float y = u4[cc];
-                    y += adj_swz_xor<16>(y);
-                    u4[cc] = y + __shfl_xor(y, 32, 64);
-                    float z = x4[cc];
-                    z += adj_swz_xor<16>(z);
-                    x4[cc] = z + __shfl_xor(z, 32, 64);
-                }
-                if (my == (uint32_t)T) {
-                    su = u4;
-                    sx = x4;
-                }
-            }
-            if (live) {
-                const float s6 = 6.0f * inv_r2;
-                const uint64_t o = 3ull * a.perm[i];
-                a.g_pos[o + 0] = -__builtin_fmaf(s6, __builtin_fmaf(-sx[3], px, sx[0]), su[0]);
-                a.g_pos[o + 1] = -__builtin_fmaf(s6, __builtin_fmaf(-sx[3], py, sx[1]), su[1]);
-                a.g_pos[o + 2] = -__builtin_fmaf(s6, __builtin_fmaf(-sx[3], pz, sx[2]), su[2]);
-            }
-        };
-        switch ((cnt + 15u) >> 4) {
-            case 1: chunk(std::integral_constant<int, 1>{}); break;
-            case 2: chunk(std::integral_constant<int, 2>{}); break;
-            case 3: chunk(std::integral_constant<int, 3>{}); break;
-            default: chunk(std::integral_constant<int, 4>{}); break;
+        for (int cc = 0; cc < 4; ++cc) {
+            float y = su[cc];
+            y += adj_swz_xor<16>(y);
+            su[cc] = y + __shfl_xor(y, 32, 64);
+            float z = sx[cc];
+            z += adj_swz_xor<16>(z);
+            sx[cc] = z + __shfl_xor(z, 32, 64);
+        }
+        if (live && (lane >> 4) == wave) {
+            const float s6 = 6.0f * inv_r2;
+            const uint64_t o = 3ull * a.perm[i];
+            a.g_pos[o + 0] = -__builtin_fmaf(s6, __builtin_fmaf(-sx[3], px, sx[0]), su[0]);
+            a.g_pos[o + 1] = -__builtin_fmaf(s6, __builtin_fmaf(-sx[3], py, sx[1]), su[1]);
+            a.g_pos[o + 2] = -__builtin_fmaf(s6, __builtin_fmaf(-sx[3], pz, sx[2]), su[2]);
         }
     }
 }
@@ -608,7 +593,7 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
     a.radius = st.bc.radius;
     a.radius_sq = st.radius_sq;
     a.g_pos = g_pos;
-    const int blocks = persistent_blocks(ctx, kAdjThreads, 4, TUNE_FIELD);
+    const int blocks = persistent_blocks(ctx, kAdjThreads, 6, TUNE_FIELD);
     hipLaunchKernelGGL(k_field_zb05_backward_mc, dim3(blocks), dim3(kAdjThreads), 0, s, a);
     FSR_LAUNCH_CHECK("k_field_zb05_backward_mc");
     return FSR_OK;
