@@ -249,7 +249,7 @@ struct FieldBackArgs {
     const uint32_t* chunk_cell;
     const uint32_t* chunk_off;
     const uint32_t* num_chunks;
-    uint32_t* next;               // per-XCD fetch counters (next_item_xcd)
+    uint32_t* next;               // per-XCD fetch counters (ItemFetch)
     const uint32_t* cell_off;     // virtual cell -> first cell-major slot
     const uint32_t* cell_cnt;
     const uint32_t* cell_band;    // cell-major slot -> vertex id
@@ -338,6 +338,8 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
     __shared__ float bt_lds[kWaves][4][64];  // per lane: (2p'/R^2, c0)
     __shared__ uint32_t count[kWaves];
     __shared__ uint32_t next_chunk;
+    __shared__ FetchState fetch;
+    fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nch = *a.num_chunks;
@@ -346,9 +348,9 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
     float* vb = &bt_lds[wave][0][0];
     for (uint32_t t = threadIdx.x; t < (uint32_t)kAdjQueue; t += kAdjThreads)
         q[kAdjOne * kAdjStride + t] = 1.0f;
-    uint32_t step = 0;
+    ItemFetch<1, true> items(a.next, nch, &fetch);
     if (wave == 0) {
-        const uint32_t first = next_item_xcd(a.next, nch, step);
+        const uint32_t first = items.next(0);
         if (lane == 0) next_chunk = first;
     }
     __syncthreads();
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
         }
         // the next chunk, fetched under the last batch
         if (wave == 0) {
-            const uint32_t nx = next_item_xcd(a.next, nch, step);
+            const uint32_t nx = items.next(0);
             if (lane == 0) next_chunk = nx;
         }
         if (fill) {

@@ -183,7 +183,7 @@ struct ChunkList {
     const uint32_t* chunk_cell;  // chunk -> cell
     const uint32_t* chunk_off;   // cell -> first chunk
     const uint32_t* num_chunks;  // device count
-    uint32_t* next;              // per-XCD fetch counters (next_item_xcd)
+    uint32_t* next;              // per-XCD fetch counters (ItemFetch)
 };
 
 // Work records of the neighbour kernels: one section per kernel (smoothing,
@@ -906,6 +906,8 @@ __global__ __launch_bounds__(kAnisoThreads, 5) void k_smooth_mc(
         NbLds<false> wave[kAnisoThreads / 64];
         NbCoopLds<false> group;
     } lds;
+    __shared__ FetchState fetch;
+    fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nch = *cl.num_chunks;
@@ -950,9 +952,9 @@ __global__ __launch_bounds__(kAnisoThreads, 5) void k_smooth_mc(
     float* vt = &lds.wave[wave].vtx[0][0];
     q[kNbOne * kNbStride + lane] = 1.0f;
     q[kNbOne * kNbStride + 64 + lane] = 1.0f;
-    uint32_t step = 0;
+    ItemFetch<kAnisoThreads / 64, kCoop> items(cl.next, nch, &fetch);
     for (;;) {
-        const uint32_t ch = next_item_xcd(cl.next, nch, step);
+        const uint32_t ch = items.next(wave);
         if (ch >= nch) break;
         const uint32_t c = cl.chunk_cell[ch];
         const uint32_t k = ch - cl.chunk_off[c];
@@ -1008,6 +1010,8 @@ __global__ __launch_bounds__(kAnisoThreads, 4) void k_covariance_mc(CovArgs a, C
         NbLds<true> wave[kAnisoThreads / 64];
         NbCoopLds<true> group;
     } lds;
+    __shared__ FetchState fetch;
+    fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nch = *cl.num_chunks;
@@ -1062,9 +1066,9 @@ __global__ __launch_bounds__(kAnisoThreads, 4) void k_covariance_mc(CovArgs a, C
     q[kNbZero * kNbStride + 64 + lane] = 0.0f;
     q[(kNbZero + 1) * kNbStride + lane] = 0.0f;
     q[(kNbZero + 1) * kNbStride + 64 + lane] = 0.0f;
-    uint32_t step = 0;
+    ItemFetch<kAnisoThreads / 64, kCoop> items(cl.next, nch, &fetch);
     for (;;) {
-        const uint32_t ch = next_item_xcd(cl.next, nch, step);
+        const uint32_t ch = items.next(wave);
         if (ch >= nch) break;
         const uint32_t c = cl.chunk_cell[ch];
         const uint32_t k = ch - cl.chunk_off[c];
@@ -1230,18 +1234,20 @@ __device__ __forceinline__ void aniso_tiles(const float* __restrict__ rows, uint
 
 // kWaves: the resident waves per SIMD the register allocation is bounded for
 // (5: 96 VGPRs; 4: 128 VGPRs).
-template <int kWaves>
+template <int kWaves, bool kSmall>
 __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFieldArgs a) {
     __shared__ __align__(16) float queue[kAnisoThreads / 64][kAfRows * kAfStride];
+    __shared__ FetchState fetch;
+    fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nch = *a.num_chunks;
     const int R = a.bc.radius;
     float* q = queue[wave];
-    uint32_t step = 0;
     uint32_t n_staged = 0, n_kept = 0;
+    ItemFetch<kAnisoThreads / 64, kSmall> items(a.next, nch, &fetch);
     for (;;) {
-        const uint32_t ch = next_item_xcd(a.next, nch, step);
+        const uint32_t ch = items.next(wave);
         if (ch >= nch) break;
         const uint32_t v = a.bc.chunk_cell[ch];
         const int cx = (int)(v % a.bc.vcx) - R;
@@ -1739,9 +1745,10 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     FSR_TRY(work_section(ctx, WORK_COV, &ca.work));
     FSR_TRY(cell_boxes(ctx, a, s, &ca.cell_box));
     FSR_TRY(reset_xcd(a.counters, s));
-    // the chunks hold the involved particles only, so the test is on the device
-    hipLaunchKernelGGL(k_covariance_mc<true>, dim3(blocks_cov), dim3(kAnisoThreads), 0, s, ca, cl2,
-                       coop_limit(ctx, blocks_cov));
+    // the chunks hold the involved particles only, at most all
+    const uint32_t coop_max = coop_limit(ctx, blocks_cov);
+    auto cov = a.n / 64u <= 2u * coop_max ? k_covariance_mc<true> : k_covariance_mc<false>;
+    hipLaunchKernelGGL(cov, dim3(blocks_cov), dim3(kAnisoThreads), 0, s, ca, cl2, coop_max);
     FSR_LAUNCH_CHECK("k_covariance_mc");
     return FSR_OK;
 }
@@ -1831,10 +1838,10 @@ fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOu
         FSR_LAUNCH_CHECK("k_cull_radius_to_w");
     }
     FSR_TRY(reset_xcd(a.counters, s));
-    if (field_waves == 4)
-        hipLaunchKernelGGL(k_field_aniso<4>, dim3(blocks), dim3(kAnisoThreads), 0, s, fa);
-    else
-        hipLaunchKernelGGL(k_field_aniso<5>, dim3(blocks), dim3(kAnisoThreads), 0, s, fa);
+    auto kernel = field_waves == 4 ? k_field_aniso<4, false> : k_field_aniso<5, false>;
+    if (few_chunks(ctx, a.n))
+        kernel = field_waves == 4 ? k_field_aniso<4, true> : k_field_aniso<5, true>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kAnisoThreads), 0, s, fa);
     FSR_LAUNCH_CHECK("k_field_aniso");
     return FSR_OK;
 }

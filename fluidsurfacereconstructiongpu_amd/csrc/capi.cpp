@@ -74,6 +74,10 @@ uint32_t coop_limit(const fsr_context* ctx, int blocks) {
     return 3u * (uint32_t)blocks / (uint32_t)std::max(1, ctx->in_flight);
 }
 
+bool few_chunks(const fsr_context* ctx, uint32_t n) {
+    return (uint64_t)n * (uint64_t)std::max(1, ctx->in_flight) <= 131072u;
+}
+
 static fsr_status check_grid(const fsr_grid_info* g, const char* name) {
     if (!g) {
         set_error(std::string(name) + " is null");
@@ -379,6 +383,7 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
         fa.counters = counters;
         fa.saved = nullptr;
         fa.work = nullptr;
+        fa.num_particles = n;
         if (ctx->save_adjoint) FSR_TRY(arena_typed(ctx, A_ADJ_VERT, V, &fa.saved));
         FSR_TRY(field_zb05(ctx, fa, s));
     }

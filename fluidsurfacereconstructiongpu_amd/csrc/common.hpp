@@ -180,43 +180,144 @@ __device__ __forceinline__ uint32_t clip_word(uint32_t word, uint32_t w, uint32_
     return word;
 }
 
-// XCD-aware dynamic work fetch for persistent kernels.  The work list [0, total)
-// is cut into 64 contiguous sub-segments, 8 per XCD in list order (XCD x owns
-// the x-th eighth of the list); workgroups are dispatched round-robin over the
-// 8 XCDs, so blockIdx % 8 names the XCD.  A wave takes items from its XCD's
-// sub-segments first (neighbouring items share particle data, which then stays
-// in that XCD's L2), starting at the sub-segment its workgroup index picks, then
-// from the other XCDs' eighths.  `step` (0 at start) is the wave's position in
-// that order.  Same-address atomics serialise (about 30 ns each here), so the
-// list has 64 counters, next64[32 k] on separate 128-byte lines, all starting at
-// 0, and a sub-segment seen exhausted by a plain (possibly stale, never early)
-// read is passed without an atomic.  Returns total when every item is taken.
-// Wave-uniform.
+// XCD-aware work fetch for persistent kernels.  The work list [0, total) is cut
+// into 64 contiguous sub-segments, 8 per XCD in list order (XCD x owns the x-th
+// eighth of the list); workgroups are dispatched round-robin over the 8 XCDs, so
+// blockIdx % 8 names the XCD, and (blockIdx / 8) % 8 the workgroup's home among
+// the XCD's 8.  Neighbouring items share particle data, which then stays in that
+// XCD's L2.  Each sub-segment goes by a counter: first the home's, then the others
+// of the XCD, then the other XCDs'.  Same-address atomics serialise (about 30 ns
+// each), so there are 64 counters, next64[32 k] on separate 128-byte lines, all
+// starting at 0.  A workgroup keeps in LDS which positions of its order are
+// exhausted (FetchState, cleared by fetch_init) and looks at a counter before it
+// adds to it.
+//
+// kSmall = false, for lists known to be long: the positions one after another.
+// kSmall = true, for lists that may be short against the fetchers (the waves, or
+// the workgroups when their waves share an item: kUnits per workgroup):
+//   * a list no longer than the fetchers is dealt out: each takes the item at its
+//     place in its home, if there is one, and is done, without a memory access
+//     (thousands of waves looking for work that is not there hold up those that
+//     work: the colour field of a 150k-particle frame took 240 us fetching from
+//     counters, 180 us dealt);
+//   * past its XCD's own sub-segments one wave reads the other XCDs' counters
+//     together: one after another they leave a wave some 15 us behind its last
+//     item (960-particle ZB05 field 25 -> 17 us).
+// The second form takes more registers; in a long list its cost per item showed
+// (7% more VALU instructions in the anisotropic field of a 1M-particle frame,
+// from spills and recomputed addresses, 830 -> 905 us) and its gain did not.
 constexpr uint32_t kFetchSegments = 64;
 
-__device__ __forceinline__ uint32_t next_item_xcd(uint32_t* next64, uint32_t total,
-                                                  uint32_t& step) {
-    const uint32_t xcd = blockIdx.x & 7u;
-    const uint32_t sub0 = (blockIdx.x >> 3) & 7u;
-    const uint32_t seg = (total + kFetchSegments - 1u) / kFetchSegments;
-    while (step < kFetchSegments) {
-        const uint32_t k = ((xcd + (step >> 3)) & 7u) * 8u + ((sub0 + step) & 7u);
-        const uint32_t lo = k * seg;
-        const uint32_t hi = min(lo + seg, total);
-        if (lo < hi) {
-            uint32_t* ctr = &next64[32u * k];
-            const uint32_t seen = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (seen < hi - lo) {
-                uint32_t idx = 0;
-                if (__lane_id() == 0) idx = atomicAdd(ctr, 1u);
-                idx = __builtin_amdgcn_readfirstlane(idx);
-                if (lo + idx < hi) return lo + idx;
+struct FetchState {
+    uint32_t gone[2];  // long lists: [0] = positions exhausted; else bit s: position s is
+};
+
+// Clears the workgroup's state; every thread of the workgroup calls it.
+__device__ __forceinline__ void fetch_init(FetchState* st) {
+    if (threadIdx.x < 2) st->gone[threadIdx.x] = 0;
+    __syncthreads();
+}
+
+template <uint32_t kUnits, bool kSmall>
+struct ItemFetch {
+    uint32_t* next64;
+    FetchState* st;
+    uint32_t total, seg;
+    bool first;
+
+    __device__ __forceinline__ ItemFetch(uint32_t* next64_, uint32_t total_, FetchState* st_)
+        : next64(next64_), st(st_), total(__builtin_amdgcn_readfirstlane(total_)),
+          seg((total + kFetchSegments - 1u) / kFetchSegments), first(true) {}
+
+    // sub-segment at position s of the order of workgroup b
+    static __device__ __forceinline__ uint32_t at(uint32_t s, uint32_t b) {
+        return (((b & 7u) + (s >> 3)) & 7u) * 8u + (((b >> 3) + s) & 7u);
+    }
+    __device__ __forceinline__ uint32_t items(uint32_t k) const {
+        const uint32_t lo = min(k * seg, total);
+        return min(lo + seg, total) - lo;
+    }
+    // whether sub-segment k has items left, as last written
+    __device__ __forceinline__ bool has_items(uint32_t k) const {
+        return __hip_atomic_load(&next64[32u * k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+               items(k);
+    }
+    __device__ __forceinline__ uint64_t gone() const {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(
+            __hip_atomic_load(&st->gone[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        const uint32_t hi = __builtin_amdgcn_readfirstlane(
+            __hip_atomic_load(&st->gone[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        return ((uint64_t)hi << 32) | lo;
+    }
+
+    __device__ __forceinline__ uint32_t next_long() {
+        uint32_t step = __builtin_amdgcn_readfirstlane(
+            __hip_atomic_load(&st->gone[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        while (step < kFetchSegments) {
+            const uint32_t k = at(step, blockIdx.x);
+            const uint32_t lo = k * seg, hi = min(lo + seg, total);
+            if (lo < hi) {
+                uint32_t* ctr = &next64[32u * k];
+                const uint32_t seen =
+                    __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (seen < hi - lo) {
+                    uint32_t idx = 0;
+                    if (__lane_id() == 0) idx = atomicAdd(ctr, 1u);
+                    idx = __builtin_amdgcn_readfirstlane(idx);
+                    if (lo + idx < hi) return lo + idx;
+                }
+            }
+            ++step;
+            if (__lane_id() == 0) atomicMax(&st->gone[0], step);
+        }
+        return total;
+    }
+
+    // The next item, or total when there is none; unit: this fetcher's index in its
+    // workgroup.  Wave-uniform, all lanes active.  The asm statements hide where
+    // the lane and workgroup numbers come from: without them the positions'
+    // sub-segments, sizes and addresses are computed before the caller's loop and
+    // held in registers through it, which made the field kernels spill.
+    __device__ __forceinline__ uint32_t next(uint32_t unit) {
+        if (!kSmall) return next_long();
+        // every home has gridDim.x / 64 workgroups at least
+        if (seg <= kUnits * (gridDim.x >> 6)) {
+            const uint32_t k = at(0, blockIdx.x), rank = (blockIdx.x >> 6) * kUnits + unit;
+            const bool take = first && rank < items(k);
+            first = false;
+            return take ? k * seg + rank : total;
+        }
+        uint32_t misses = 0;
+        for (;;) {
+            const uint64_t g = gone();
+            if (g == ~0ull) return total;
+            const uint32_t s = (uint32_t)__builtin_ctzll(~g);
+            uint32_t b = blockIdx.x, lane = __lane_id();
+            asm volatile("" : "+s"(b));
+            asm volatile("" : "+v"(lane));
+            uint64_t done = 0;
+            if (s >= 8u && misses >= 2u) {
+                // the other XCDs' counters at once: lane l looks at position l
+                done = __ballot(lane >= 8u && !((g >> lane) & 1u) && !has_items(at(lane, b)));
+                misses = 0;
+            } else {
+                const uint32_t k = at(s, b);
+                if (has_items(k)) {
+                    uint32_t idx = 0;
+                    if (lane == 0) idx = atomicAdd(&next64[32u * k], 1u);
+                    idx = __builtin_amdgcn_readfirstlane(idx);
+                    if (idx < items(k)) return k * seg + idx;
+                }
+                done = 1ull << s;
+                ++misses;
+            }
+            if (lane == 0) {
+                if ((uint32_t)done) atomicOr(&st->gone[0], (uint32_t)done);
+                if (done >> 32) atomicOr(&st->gone[1], (uint32_t)(done >> 32));
             }
         }
-        ++step;
     }
-    return total;
-}
+};
 
 // Adds a per-lane count into a global counter with one atomic per wave.
 __device__ __forceinline__ void wave_count_add(uint32_t* counter, uint32_t v) {
@@ -522,6 +623,7 @@ struct FieldArgs {
     float4* saved;         // optional, cell-major [B]: (x - xbar, sum w) for the adjoint
     uint32_t* work;        // set by field_zb05: per chunk, candidates staged, candidates
                            // kept by the box test, 16 x 16 tile steps evaluated
+    uint32_t num_particles;
 };
 fsr_status field_zb05(fsr_context* ctx, const FieldArgs& a, hipStream_t s);
 fsr_status fill_f32(float* p, float value, uint64_t n, hipStream_t s);
@@ -615,6 +717,11 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
 // Grid of a persistent kernel: CUs x workgroups per CU (the tuned value of
 // `cls` when set, else `per_cu`).
 int persistent_blocks(fsr_context* ctx, int threads, int per_cu, TuneClass cls);
+// Whether a frame of n particles takes the field kernels' build for few chunks: up
+// to 131,072 particles (64k: 14,000 ZB05 chunks on 6144 waves, field 92 -> 83 us;
+// 118k 90 -> 83 us; both builds within 1% at 244k), divided by the frames in flight
+// (8 ZB05 frames of 60k in a batch: 831 us with it, 814 without).
+bool few_chunks(const fsr_context* ctx, uint32_t n);
 // Most chunks for which a neighbour kernel of `blocks` workgroups of 4 waves
 // shares each chunk among a workgroup's waves.
 uint32_t coop_limit(const fsr_context* ctx, int blocks);

@@ -173,14 +173,17 @@ __device__ uint32_t chunk_vertex(const BandCompactOut& bc, uint32_t rx, uint32_t
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// LDS queue of one wave, structure of arrays: rows x', y', z', a row of ones
-// and a row of -q, kQueue entries each.  The first four rows start 144 floats
-// apart, so the 16-entry slices that one matrix operand reads from them fall
-// into distinct LDS banks.
+// LDS queue, structure of arrays: rows x', y', z', a row of ones and a row of -q
+// (rows 0 to 4).  The rows start 16 floats more than a multiple of 64 apart, so
+// the 16-entry slices that one matrix operand reads from the first four fall
+// into distinct LDS banks.  One wave: a ring of kQueue entries; a workgroup
+// that shares a chunk: kCoopQueue (63 waiting + 256 new, 256 being read).
 constexpr int kQueue = 128;
-constexpr int kRowStride = 144;
-constexpr int kRowX = 0, kRowY = 144, kRowZ = 288, kRowOne = 432, kRowQ = 576;
-constexpr int kQueueFloats = 704;
+constexpr int kRowStride = kQueue + 16;
+constexpr int kRowX = 0, kRowY = 1, kRowZ = 2, kRowOne = 3, kRowQ = 4, kRows = 5;
+constexpr int kCoopQueue = 512;
+constexpr int kCoopStride = kCoopQueue + 16;
+constexpr int kFieldWaves = kFieldThreads / 64;
 
 // Sums of w and w p' for the NT 16-vertex tiles of one chunk over n staged
 // candidates (n a multiple of 16), on the matrix cores.  Per 16 candidates and
@@ -196,13 +199,13 @@ constexpr int kQueueFloats = 704;
 //      sum w p' (x, y, z) and sum w for vertex l%16 over the candidates
 //      congruent to l/16 in each group of 16.
 // The caller adds the four partial sums of a vertex (lanes l%16 + 16m).
-template <int NT>
+template <int NT, int kStride>
 __device__ __forceinline__ void accumulate(const float* __restrict__ rows, uint32_t n,
                                            const float (&b1)[NT], v4f (&acc)[NT]) {
     const uint32_t lane = __lane_id();
-    const float* a1p = rows + (lane >> 4) * kRowStride + (lane & 15u);
-    const float* a2p = rows + (lane & 3u) * kRowStride + 4u * (lane >> 4);
-    const float* cqp = rows + kRowQ + 4u * (lane >> 4);
+    const float* a1p = rows + (lane >> 4) * kStride + (lane & 15u);
+    const float* a2p = rows + (lane & 3u) * kStride + 4u * (lane >> 4);
+    const float* cqp = rows + 4 * kStride + 4u * (lane >> 4);
     for (uint32_t tb = 0; tb < n; tb += 16u) {
         const float a1 = a1p[tb];
         const float4 a2 = *reinterpret_cast<const float4*>(a2p + tb);
@@ -240,116 +243,309 @@ __device__ __forceinline__ void accumulate(const float* __restrict__ rows, uint3
     }
 }
 
+// What the lanes of a wave know about their chunk.
+struct Chunk {
+    uint32_t cnt, first, vid;    // vertices; first cell-major slot; this lane's vertex id
+    bool has_vertex;
+    float ox, oy, oz;            // cell corner: the local origin
+    float lo[3], hi[3];          // box of the chunk's vertices
+    uint32_t nrows, total;       // candidate rows (x-runs) and candidates
+    uint32_t rp, ro;             // lane j < nrows: first candidate index of row j, and
+                                 // the offset from candidate index to sorted index in it
+    uint32_t jc;
+
+    // Row lookup: jc is a row whose first candidate index is at most the first
+    // index nb of the round being located (rows only grow with the index).  The
+    // rows that start before the round's end are visited with wave-uniform reads
+    // of rp and ro; a lane takes the last one that starts at or before its index
+    // gg.  Empty rows share their first index with the next row, which is
+    // visited after them.
+    __device__ __forceinline__ uint32_t row_offset(uint32_t nb, uint32_t gg) {
+        uint32_t off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
+        for (uint32_t jj = jc + 1u; jj < nrows; ++jj) {
+            const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)rp, (int)jj);
+            if (pj >= nb + 64u) break;
+            if (gg >= pj) off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jj);
+            jc = jj;
+        }
+        return off;
+    }
+};
+
+// Loads chunk ch: its vertices (listed through `scratch`, 64 words of LDS, when
+// the cell-major list is not materialised), their operands into vt (rows of 64:
+// x', y', z', a_x, a_y, a_z, c_x), their box, and the candidate rows.
+__device__ __forceinline__ Chunk load_chunk(const FieldArgs& a, const BandCompactOut& bc,
+                                            const VertexDiv& vd, uint32_t ch, float inv_r2,
+                                            float* __restrict__ vt, uint32_t* scratch) {
+    const uint32_t lane = __lane_id();
+    const int r = bc.radius;
+    Chunk c;
+    const uint32_t v = bc.chunk_cell[ch];
+    const int cx = (int)(v % bc.vcx) - r;
+    const int cy = (int)((v / bc.vcx) % bc.vcy) - r;
+    const int cz = (int)(v / (bc.vcx * bc.vcy)) - r;
+    const uint32_t k = ch - bc.chunk_off[v];
+    const uint32_t ccount = bc.cell_cnt[v];
+    c.first = bc.cell_off[v] + 64u * k;
+    c.cnt = min(64u, ccount - 64u * k);
+    // the chunk's vertex ids (before the candidate rows, whose registers live
+    // through the staging loop)
+    c.vid = 0;
+    if (bc.cell_band) {
+        if (lane < c.cnt) c.vid = bc.cell_band[c.first + lane];
+    } else {
+        c.vid = chunk_vertex(bc, a.sc.rx, a.sc.ry, v, k, c.cnt, scratch);
+    }
+
+    // candidate rows of the clamped 3^3 block
+    const int x0 = clampi(cx - 1, 0, a.sp.rx - 1), x1 = clampi(cx + 1, 0, a.sp.rx - 1);
+    const int y0 = clampi(cy - 1, 0, a.sp.ry - 1), y1 = clampi(cy + 1, 0, a.sp.ry - 1);
+    const int z0 = clampi(cz - 1, 0, a.sp.rz - 1), z1 = clampi(cz + 1, 0, a.sp.rz - 1);
+    const int ny = y1 - y0 + 1;
+    c.nrows = (uint32_t)(ny * (z1 - z0 + 1));
+    uint32_t len = 0, rs = 0;
+    if (lane < c.nrows) {
+        const int yy = y0 + (int)lane % ny, zz = z0 + (int)lane / ny;
+        const uint32_t rowc = ((uint32_t)zz * a.sp.ry + yy) * a.sp.rx;
+        // the row's 3 cells as clamped offsets (a repeated edge cell leaves
+        // the run unchanged), loaded together
+        fsr_index_range rg[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) rg[d] = a.ranges[rowc + clampi(cx - 1 + d, x0, x1)];
+        uint32_t s = 0xFFFFFFFFu, e = 0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (rg[d].start != 0xFFFFFFFFu) {
+                if (s == 0xFFFFFFFFu) s = rg[d].start;
+                e = rg[d].end;
+            }
+        }
+        if (s != 0xFFFFFFFFu) { rs = s; len = e - s; }
+    }
+    // nrows <= 9: the prefix over the first 16 lanes is the whole prefix
+    const uint32_t incl = row16_inclusive_sum(len);
+    c.total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 15);
+    c.rp = incl - len;
+    c.ro = rs - c.rp;
+    c.jc = 0;
+
+    c.ox = __builtin_fmaf((float)cx, a.sp.cell, a.sp.minx);
+    c.oy = __builtin_fmaf((float)cy, a.sp.cell, a.sp.miny);
+    c.oz = __builtin_fmaf((float)cz, a.sp.cell, a.sp.minz);
+    float vx = 0.f, vy = 0.f, vz = 0.f;
+    // lanes with a vertex (an id past the grid would mean an empty slot)
+    c.has_vertex = lane < c.cnt && c.vid < a.sc.rx * a.sc.ry * a.sc.rz;
+    if (c.has_vertex) {
+        const uint32_t iz = fast_div(c.vid, vd.rxy);
+        const uint32_t rem = c.vid - iz * (a.sc.rx * a.sc.ry);
+        const uint32_t iy = fast_div(rem, vd.rx);
+        const uint32_t ix = rem - iy * a.sc.rx;
+        vx = vertex_coord(ix, a.sc.minx, a.sc.cell) - c.ox;
+        vy = vertex_coord(iy, a.sc.miny, a.sc.cell) - c.oy;
+        vz = vertex_coord(iz, a.sc.minz, a.sc.cell) - c.oz;
+    }
+    vt[lane] = vx;
+    vt[64 + lane] = vy;
+    vt[128 + lane] = vz;
+    vt[192 + lane] = 2.0f * vx * inv_r2;
+    vt[256 + lane] = 2.0f * vy * inv_r2;
+    vt[320 + lane] = 2.0f * vz * inv_r2;
+    vt[384 + lane] = 1.0f - __builtin_fmaf(vz, vz, __builtin_fmaf(vy, vy, vx * vx)) * inv_r2;
+    wave_range(c.has_vertex, vx, &c.lo[0], &c.hi[0]);
+    wave_range(c.has_vertex, vy, &c.lo[1], &c.hi[1]);
+    wave_range(c.has_vertex, vz, &c.lo[2], &c.hi[2]);
+    return c;
+}
+
+// The field at this lane's vertex from its sums (sum w p', sum w).
+__device__ __forceinline__ void store_vertex(const FieldArgs& a, const Chunk& c, const v4f& s4,
+                                             const float* __restrict__ vt) {
+    const uint32_t lane = __lane_id();
+    float4 keep_out = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float sw = s4[3];
+    if (sw > 0.0f) {
+        const float inv = 1.0f / sw;
+        const float dx = vt[lane] - s4[0] * inv;
+        const float dy = vt[64 + lane] - s4[1] * inv;
+        const float dz = vt[128 + lane] - s4[2] * inv;
+        a.phi[c.vid] = __builtin_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx))) -
+                       a.particle_radius;
+        keep_out = make_float4(dx, dy, dz, sw);
+    }
+    // for the adjoint: x - xbar and sum w, at the vertex's cell-major slot
+    if (a.saved) a.saved[c.first + lane] = keep_out;
+}
+
+// One LDS block per wave, so every per-lane LDS address is one base register
+// plus an immediate offset; or one per workgroup, in the shared form.
+struct WaveLds {
+    float queue[kRows * kRowStride];
+    // per lane: x', y', z' of its vertex (for the end) and (a_x, a_y, a_z, c_x)
+    float vtx[7][64];
+};
+struct GroupLds {
+    float queue[kRows * kCoopStride];
+    float vtx[kFieldWaves][7][64];
+    uint32_t count[kFieldWaves];
+    uint32_t next_chunk;
+};
+
+// The shared form: the 4 waves of a workgroup treat a chunk together, for frames
+// with few chunks (see coop_limit).  Each wave stages a quarter of a
+// 256-candidate round into one ring, in candidate order, and evaluates one of
+// the chunk's 16-vertex tiles: the candidates, their order and every tile's
+// operations are those of the wave form, so the field is the same bits.  Per
+// round two barriers: counts (which also says that the previous batches are
+// evaluated), and entries.
+__device__ __forceinline__ void field_shared(const FieldArgs& a, const BandCompactOut& bc,
+                                             const VertexDiv& vd, GroupLds& L, uint32_t num_chunks,
+                                             float inv_r2, float cull_r2, FetchState* fetch) {
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = threadIdx.x >> 6;
+    float* q = L.queue;
+    float* vt = &L.vtx[wave][0][0];
+    for (uint32_t t = threadIdx.x; t < (uint32_t)kCoopQueue; t += kFieldThreads)
+        q[kRowOne * kCoopStride + t] = 1.0f;
+    ItemFetch<1, true> items(a.counters->xcd_field, num_chunks, fetch);
+    if (wave == 0) {
+        const uint32_t nx = items.next(0);
+        if (lane == 0) L.next_chunk = nx;
+    }
+    __syncthreads();
+    // workgroup-uniform
+    for (uint32_t ch = L.next_chunk; ch < num_chunks; ch = L.next_chunk) {
+        Chunk c = load_chunk(a, bc, vd, ch, inv_r2, vt, reinterpret_cast<uint32_t*>(vt));
+        wave_lds_sync();
+        const uint32_t nt = (c.cnt + 15u) >> 4;
+        const bool mine = wave < nt;
+        float b1[1] = {vt[192 + 64 * (lane >> 4) + 16u * wave + (lane & 15u)]};
+        v4f acc[1] = {v4f{0.f, 0.f, 0.f, 0.f}};
+        uint32_t head = 0, fill = 0, n_kept = 0, n_steps = 0;
+        float3 next = make_float3(0.f, 0.f, 0.f);
+        {
+            const uint32_t g = 64u * wave + lane;
+            const uint32_t off = c.row_offset(64u * wave, g);
+            if (g < c.total) next = load_xyz(a.sorted + (off + g));
+        }
+        for (uint32_t base = 0; base < c.total; base += 256u) {
+            const uint32_t g = base + 64u * wave + lane;
+            const float3 p = next;
+            if (base + 256u < c.total) {
+                const uint32_t off = c.row_offset(base + 256u + 64u * wave, g + 256u);
+                if (g + 256u < c.total) next = load_xyz(a.sorted + (off + g + 256u));
+            }
+            const float px = p.x - c.ox, py = p.y - c.oy, pz = p.z - c.oz;
+            const float dx = px - __builtin_amdgcn_fmed3f(px, c.lo[0], c.hi[0]);
+            const float dy = py - __builtin_amdgcn_fmed3f(py, c.lo[1], c.hi[1]);
+            const float dz = pz - __builtin_amdgcn_fmed3f(pz, c.lo[2], c.hi[2]);
+            const bool keep =
+                g < c.total &&
+                __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull_r2;
+            const uint64_t m = __ballot(keep);
+            if (lane == 0) L.count[wave] = (uint32_t)__popcll(m);
+            __syncthreads();
+            uint32_t before = 0, added = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < (uint32_t)kFieldWaves; ++w) {
+                const uint32_t n = L.count[w];
+                before += w < wave ? n : 0u;
+                added += n;
+            }
+            if (keep) {
+                const uint32_t slot = (head + fill + before + mask_rank(m)) & (kCoopQueue - 1);
+                q[kRowX * kCoopStride + slot] = px;
+                q[kRowY * kCoopStride + slot] = py;
+                q[kRowZ * kCoopStride + slot] = pz;
+                q[kRowQ * kCoopStride + slot] =
+                    -(__builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px)) * inv_r2);
+            }
+            fill += added;
+            n_kept += added;
+            __syncthreads();
+            for (; fill >= 64u; fill -= 64u) {
+                if (mine) accumulate<1, kCoopStride>(q + head, 64u, b1, acc);
+                head = (head + 64u) & (kCoopQueue - 1);
+                n_steps += 4u * nt;
+            }
+        }
+        // the next chunk, fetched under the last batch
+        if (wave == 0) {
+            const uint32_t nx = items.next(0);
+            if (lane == 0) L.next_chunk = nx;
+        }
+        if (fill) {
+            // pad to a multiple of 16 with entries of weight 0 (t < 0 for
+            // every vertex); head is a multiple of 64, so the pad does not wrap
+            const uint32_t n = (fill + 15u) & ~15u;
+            if (wave == 0 && lane >= fill && lane < n) {
+                q[kRowX * kCoopStride + head + lane] = 0.f;
+                q[kRowY * kCoopStride + head + lane] = 0.f;
+                q[kRowZ * kCoopStride + head + lane] = 0.f;
+                q[kRowQ * kCoopStride + head + lane] = -1.0e30f;
+            }
+            n_steps += (n >> 4) * nt;
+            __syncthreads();
+            if (mine) accumulate<1, kCoopStride>(q + head, n, b1, acc);
+        }
+        // the next chunk rewrites the ring from its start
+        __syncthreads();
+        // the four partial sums of each vertex; the lanes of the wave's tile
+        // write theirs
+        v4f s4 = acc[0];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            float x = s4[d];
+            x += swz_xor<16>(x);
+            s4[d] = x + __shfl_xor(x, 32, 64);
+        }
+        if (c.has_vertex && (lane >> 4) == wave) store_vertex(a, c, s4, vt);
+        if (threadIdx.x == 0) {
+            uint32_t* w = a.work + 3u * ch;
+            w[0] = c.total;
+            w[1] = n_kept;
+            w[2] = n_steps;
+        }
+        // vt holds the vertices until here
+        wave_lds_sync();
+    }
+}
+
+// kShared: the build for smaller frames, whose chunks may be few (their count is
+// known on the device only): it has the shared form, taken at up to coop_max
+// chunks, and the fetch for short lists.
+template <bool kShared>
 __global__ __launch_bounds__(kFieldThreads, 6) void k_field_zb05(FieldArgs a, BandCompactOut bc,
-                                                              VertexDiv vd) {
-    // one LDS block per wave, so every per-lane LDS address is one base
-    // register plus an immediate offset
-    struct WaveLds {
-        float queue[kQueueFloats];
-        // per lane: x', y', z' of its vertex (for the end) and (a_x, a_y, a_z, c_x)
-        float vtx[7][64];
-    };
-    __shared__ __align__(16) WaveLds lds[kFieldThreads / 64];
+                                                              VertexDiv vd, uint32_t coop_max) {
+    __shared__ __align__(16) union {
+        WaveLds wave[kFieldWaves];
+        GroupLds group;
+    } lds;
+    __shared__ FetchState fetch;
+    fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t num_chunks = a.counters->num_chunks;
     const float inv_r2 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(1.0f / a.radius_sq)));
     const float cull_r2 = a.radius_sq * 1.0001f;
-    const int r = bc.radius;
-    float* q = lds[wave].queue;
-    q[kRowOne + lane] = 1.0f;
-    q[kRowOne + 64 + lane] = 1.0f;
     // the work record ends with a marker after the last chunk
     if (blockIdx.x == 0 && threadIdx.x == 0) a.work[3u * num_chunks] = 0xFFFFFFFFu;
+    if (kShared && num_chunks <= coop_max) {
+        field_shared(a, bc, vd, lds.group, num_chunks, inv_r2, cull_r2, &fetch);
+        return;
+    }
+    float* q = lds.wave[wave].queue;
+    float* vt = &lds.wave[wave].vtx[0][0];
+    q[kRowOne * kRowStride + lane] = 1.0f;
+    q[kRowOne * kRowStride + 64 + lane] = 1.0f;
 
-    uint32_t step = 0;
+    ItemFetch<kFieldWaves, kShared> items(a.counters->xcd_field, num_chunks, &fetch);
     for (;;) {
-        const uint32_t ch = next_item_xcd(a.counters->xcd_field, num_chunks, step);
+        const uint32_t ch = items.next(wave);
         if (ch >= num_chunks) break;
-
-        const uint32_t v = bc.chunk_cell[ch];
-        const int cx = (int)(v % bc.vcx) - r;
-        const int cy = (int)((v / bc.vcx) % bc.vcy) - r;
-        const int cz = (int)(v / (bc.vcx * bc.vcy)) - r;
-        const uint32_t k = ch - bc.chunk_off[v];
-        const uint32_t ccount = bc.cell_cnt[v];
-        const uint32_t first = bc.cell_off[v] + 64u * k;
-        const uint32_t cnt = min(64u, ccount - 64u * k);
-        // the chunk's vertex ids (before the candidate rows, whose registers
-        // live through the staging loop)
-        uint32_t vid = 0;
-        if (bc.cell_band) {
-            if (lane < cnt) vid = bc.cell_band[first + lane];
-        } else {
-            vid = chunk_vertex(bc, a.sc.rx, a.sc.ry, v, k, cnt, reinterpret_cast<uint32_t*>(q));
-        }
-
-        // candidate rows of the clamped 3^3 block
-        const int x0 = clampi(cx - 1, 0, a.sp.rx - 1), x1 = clampi(cx + 1, 0, a.sp.rx - 1);
-        const int y0 = clampi(cy - 1, 0, a.sp.ry - 1), y1 = clampi(cy + 1, 0, a.sp.ry - 1);
-        const int z0 = clampi(cz - 1, 0, a.sp.rz - 1), z1 = clampi(cz + 1, 0, a.sp.rz - 1);
-        const int ny = y1 - y0 + 1;
-        const int nrows = ny * (z1 - z0 + 1);
-        uint32_t len = 0, rs = 0;
-        if ((int)lane < nrows) {
-            const int yy = y0 + (int)lane % ny, zz = z0 + (int)lane / ny;
-            const uint32_t rowc = ((uint32_t)zz * a.sp.ry + yy) * a.sp.rx;
-            // the row's 3 cells as clamped offsets (a repeated edge cell leaves
-            // the run unchanged), loaded together
-            fsr_index_range rg[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) rg[d] = a.ranges[rowc + clampi(cx - 1 + d, x0, x1)];
-            uint32_t s = 0xFFFFFFFFu, e = 0;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                if (rg[d].start != 0xFFFFFFFFu) {
-                    if (s == 0xFFFFFFFFu) s = rg[d].start;
-                    e = rg[d].end;
-                }
-            }
-            if (s != 0xFFFFFFFFu) { rs = s; len = e - s; }
-        }
-        // nrows <= 9: the prefix over the first 16 lanes is the whole prefix.
-        // Lane j < nrows keeps the first candidate index of row j (rp) and the
-        // offset from candidate index to sorted index in that row (ro).
-        const uint32_t incl = row16_inclusive_sum(len);
-        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 15);
-        const uint32_t rp = incl - len;
-        const uint32_t ro = rs - rp;
-
-        // cell corner as the local origin
-        const float ox = __builtin_fmaf((float)cx, a.sp.cell, a.sp.minx);
-        const float oy = __builtin_fmaf((float)cy, a.sp.cell, a.sp.miny);
-        const float oz = __builtin_fmaf((float)cz, a.sp.cell, a.sp.minz);
-
-        float vx = 0.f, vy = 0.f, vz = 0.f;
-        // lanes with a vertex (an id past the grid would mean an empty slot)
-        const bool has_vertex = lane < cnt && vid < a.sc.rx * a.sc.ry * a.sc.rz;
-        if (has_vertex) {
-            const uint32_t iz = fast_div(vid, vd.rxy);
-            const uint32_t rem = vid - iz * (a.sc.rx * a.sc.ry);
-            const uint32_t iy = fast_div(rem, vd.rx);
-            const uint32_t ix = rem - iy * a.sc.rx;
-            vx = vertex_coord(ix, a.sc.minx, a.sc.cell) - ox;
-            vy = vertex_coord(iy, a.sc.miny, a.sc.cell) - oy;
-            vz = vertex_coord(iz, a.sc.minz, a.sc.cell) - oz;
-        }
-        float* vt = &lds[wave].vtx[0][0];
-        vt[lane] = vx;
-        vt[64 + lane] = vy;
-        vt[128 + lane] = vz;
-        vt[192 + lane] = 2.0f * vx * inv_r2;
-        vt[256 + lane] = 2.0f * vy * inv_r2;
-        vt[320 + lane] = 2.0f * vz * inv_r2;
-        vt[384 + lane] = 1.0f - __builtin_fmaf(vz, vz, __builtin_fmaf(vy, vy, vx * vx)) * inv_r2;
-        // bounding box of the chunk's vertices
-        const bool live = has_vertex;
-        float bx0, bx1, by0, by1, bz0, bz1;
-        wave_range(live, vx, &bx0, &bx1);
-        wave_range(live, vy, &by0, &by1);
-        wave_range(live, vz, &bz0, &bz1);
+        Chunk c = load_chunk(a, bc, vd, ch, inv_r2, vt, reinterpret_cast<uint32_t*>(q));
         wave_lds_sync();
-        const int nt = (int)((cnt + 15u) >> 4);
+        const int nt = (int)((c.cnt + 15u) >> 4);
         // The rest of the chunk, compiled once per tile count NT, so that the
         // accumulators keep fixed registers across the staging loop.
         auto run = [&](auto ntc) {
@@ -372,58 +568,39 @@ __global__ __launch_bounds__(kFieldThreads, 6) void k_field_zb05(FieldArgs a, Ba
             // this lane's candidate of the next round is loaded one round ahead,
             // so the load overlaps the culling and the accumulation of the
             // current one
-            //
-            // Row lookup: jc is a row whose first candidate index is at most
-            // the first index nb of the round being located (rows only grow
-            // with the index).  The rows that start inside the round are
-            // visited with wave-uniform reads of rp and ro; a lane takes the
-            // last one that starts at or before its index gg.  Empty rows
-            // share their first index with the next row, which is visited
-            // after them.
-            uint32_t jc = 0;
-            auto row_offset = [&](uint32_t nb, uint32_t gg) {
-                uint32_t off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
-                for (uint32_t jj = jc + 1u; jj < (uint32_t)nrows; ++jj) {
-                    const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)rp, (int)jj);
-                    if (pj >= nb + 64u) break;
-                    if (gg >= pj) off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jj);
-                    jc = jj;
-                }
-                return off;
-            };
             float3 next = make_float3(0.f, 0.f, 0.f);
             {
-                const uint32_t off = row_offset(0u, lane);
-                if (lane < total) next = load_xyz(a.sorted + (off + lane));
+                const uint32_t off = c.row_offset(0u, lane);
+                if (lane < c.total) next = load_xyz(a.sorted + (off + lane));
             }
-            for (uint32_t base = 0; base < total; base += 64u) {
+            for (uint32_t base = 0; base < c.total; base += 64u) {
                 const uint32_t g = base + lane;
                 const float3 p = next;
-                if (base + 64u < total) {
+                if (base + 64u < c.total) {
                     const uint32_t gn = g + 64u;
-                    const uint32_t off = row_offset(base + 64u, gn);
-                    if (gn < total) next = load_xyz(a.sorted + (off + gn));
+                    const uint32_t off = c.row_offset(base + 64u, gn);
+                    if (gn < c.total) next = load_xyz(a.sorted + (off + gn));
                 }
                 bool keep = false;
                 float px = 0.f, py = 0.f, pz = 0.f;
-                if (g < total) {
-                    px = p.x - ox;
-                    py = p.y - oy;
-                    pz = p.z - oz;
+                if (g < c.total) {
+                    px = p.x - c.ox;
+                    py = p.y - c.oy;
+                    pz = p.z - c.oz;
                     // distance to the box per axis: p - clamp(p, lo, hi), whose
                     // square equals that of max(lo - p, p - hi, 0) exactly
-                    const float dx = px - __builtin_amdgcn_fmed3f(px, bx0, bx1);
-                    const float dy = py - __builtin_amdgcn_fmed3f(py, by0, by1);
-                    const float dz = pz - __builtin_amdgcn_fmed3f(pz, bz0, bz1);
+                    const float dx = px - __builtin_amdgcn_fmed3f(px, c.lo[0], c.hi[0]);
+                    const float dy = py - __builtin_amdgcn_fmed3f(py, c.lo[1], c.hi[1]);
+                    const float dz = pz - __builtin_amdgcn_fmed3f(pz, c.lo[2], c.hi[2]);
                     keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull_r2;
                 }
                 const uint64_t m = __ballot(keep);
                 if (keep) {
                     const uint32_t slot = (head + fill + mask_rank(m)) & (kQueue - 1);
-                    q[kRowX + slot] = px;
-                    q[kRowY + slot] = py;
-                    q[kRowZ + slot] = pz;
-                    q[kRowQ + slot] =
+                    q[kRowX * kRowStride + slot] = px;
+                    q[kRowY * kRowStride + slot] = py;
+                    q[kRowZ * kRowStride + slot] = pz;
+                    q[kRowQ * kRowStride + slot] =
                         -(__builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px)) * inv_r2);
                 }
                 fill += (uint32_t)__popcll(m);
@@ -431,7 +608,7 @@ __global__ __launch_bounds__(kFieldThreads, 6) void k_field_zb05(FieldArgs a, Ba
                 if (fill >= 64u) {
                     n_steps += 4u * NT;
                     wave_lds_sync();
-                    accumulate<NT>(q + head, 64u, b1, acc);
+                    accumulate<NT, kRowStride>(q + head, 64u, b1, acc);
                     wave_lds_sync();
                     head ^= 64u;
                     fill -= 64u;
@@ -442,14 +619,14 @@ __global__ __launch_bounds__(kFieldThreads, 6) void k_field_zb05(FieldArgs a, Ba
                 // every vertex); head + 64 <= kQueue, so the pad does not wrap
                 const uint32_t n = (fill + 15u) & ~15u;
                 if (lane >= fill && lane < n) {
-                    q[kRowX + head + lane] = 0.f;
-                    q[kRowY + head + lane] = 0.f;
-                    q[kRowZ + head + lane] = 0.f;
-                    q[kRowQ + head + lane] = -1.0e30f;
+                    q[kRowX * kRowStride + head + lane] = 0.f;
+                    q[kRowY * kRowStride + head + lane] = 0.f;
+                    q[kRowZ * kRowStride + head + lane] = 0.f;
+                    q[kRowQ * kRowStride + head + lane] = -1.0e30f;
                 }
                 n_steps += (n >> 4) * NT;
                 wave_lds_sync();
-                accumulate<NT>(q + head, n, b1, acc);
+                accumulate<NT, kRowStride>(q + head, n, b1, acc);
                 wave_lds_sync();
             }
             // add the four partial sums of each vertex; lane l then holds the
@@ -459,33 +636,18 @@ __global__ __launch_bounds__(kFieldThreads, 6) void k_field_zb05(FieldArgs a, Ba
 #pragma unroll
             for (int T = 0; T < NT; ++T) {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    float x = acc[T][c];
+                for (int d = 0; d < 4; ++d) {
+                    float x = acc[T][d];
                     x += swz_xor<16>(x);
                     x += __shfl_xor(x, 32, 64);
-                    acc[T][c] = x;
+                    acc[T][d] = x;
                 }
                 if (my == (uint32_t)T) s4 = acc[T];
             }
-            if (has_vertex) {
-                float4 keep_out = make_float4(0.f, 0.f, 0.f, 0.f);
-                const float sw = s4[3];
-                if (sw > 0.0f) {
-                    const float inv = 1.0f / sw;
-                    const float dx = vt[lane] - s4[0] * inv;
-                    const float dy = vt[64 + lane] - s4[1] * inv;
-                    const float dz = vt[128 + lane] - s4[2] * inv;
-                    a.phi[vid] =
-                        __builtin_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx))) -
-                        a.particle_radius;
-                    keep_out = make_float4(dx, dy, dz, sw);
-                }
-                // for the adjoint: x - xbar and sum w, at the vertex's cell-major slot
-                if (a.saved) a.saved[first + lane] = keep_out;
-            }
+            if (c.has_vertex) store_vertex(a, c, s4, vt);
             if (lane == 0) {
                 uint32_t* w = a.work + 3u * ch;
-                w[0] = total;
+                w[0] = c.total;
                 w[1] = n_kept;
                 w[2] = n_steps;
             }
@@ -512,7 +674,9 @@ fsr_status field_zb05(fsr_context* ctx, const FieldArgs& a, hipStream_t s) {
     VertexDiv vd;
     vd.rx = make_fast_div(a.sc.rx);
     vd.rxy = make_fast_div(a.sc.rx * a.sc.ry);
-    hipLaunchKernelGGL(k_field_zb05, dim3(blocks), dim3(kFieldThreads), 0, s, fa, *a.bc, vd);
+    auto kernel = few_chunks(ctx, a.num_particles) ? k_field_zb05<true> : k_field_zb05<false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kFieldThreads), 0, s, fa, *a.bc, vd,
+                       coop_limit(ctx, blocks));
     FSR_LAUNCH_CHECK("k_field_zb05");
     return FSR_OK;
 }

@@ -590,6 +590,7 @@ fsr_status fsr_update_scalar_grid_values_compacted(
     fa.counters = ct;
     fa.saved = nullptr;
     fa.work = nullptr;
+    fa.num_particles = num_particles;
     return field_zb05(ctx, fa, s);
 }
 

@@ -295,8 +295,11 @@ struct ColorChunks {
 // |r|^2 rsqrt(|r|^2), one reciprocal square root per pair within h and no
 // square root: the distance enters the gradient through (1 - |r|/h)^2, which
 // vanishes where the two forms of the test could differ.
+template <bool kSmall>
 __global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, ColorChunks cl) {
     __shared__ float4 queue[4][128];
+    __shared__ FetchState fetch;
+    fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     float4* q = queue[wave];
@@ -310,9 +313,9 @@ __global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, C
     // work of this wave: candidates staged and kept (wave-uniform), and this
     // lane's pairs within h
     uint32_t n_staged = 0, n_kept = 0, n_inh = 0;
-    uint32_t step = 0;
+    ItemFetch<4, kSmall> items(cl.next, nch, &fetch);
     for (;;) {
-        const uint32_t ch = next_item_xcd(cl.next, nch, step);
+        const uint32_t ch = items.next(wave);
         if (ch >= nch) break;
         const uint32_t c = cl.chunk_cell[ch];
         const uint32_t k = ch - cl.chunk_off[c];
@@ -550,7 +553,11 @@ fsr_status surface_colorfield(fsr_context* ctx, const SurfaceArgs& a, float mass
     FSR_TRY(arena_typed(ctx, A_COLOR_WORK, 3ull * blocks * 4, &work));
     ColorChunks cl{scratch + 2ull * C, scratch + C, total, a.counters->xcd_next, work};
     FSR_TRY(reset_xcd(a.counters, s));
-    hipLaunchKernelGGL(k_colorfield, dim3(blocks), dim3(256), 0, s, a, mass, cl);
+    // n / 64 chunks and up to as many remainders: a list that may be shorter than
+    // the waves is dealt out (see ItemFetch)
+    auto kernel = a.n / 64u <= 4u * (uint32_t)(blocks / ctx->in_flight) ? k_colorfield<true>
+                                                                         : k_colorfield<false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, a, mass, cl);
     FSR_LAUNCH_CHECK("k_colorfield");
     // particles outside the grid (a device-side count)
     hipLaunchKernelGGL(k_colorfield_tail, dim3(64), dim3(256), 0, s, a, mass);

@@ -1,8 +1,9 @@
 """The neighbour kernels treat a chunk (64 particles or vertices of one hash
 cell) with one wave, or share it among the 4 waves of a workgroup when the frame
-has few chunks.  Both forms evaluate the same candidates in the same order, so a
+has few chunks; and they deal a short chunk list out to the waves, or fetch from
+counters.  All forms evaluate the same candidates in the same order, so a
 frame's outputs are the same bits: a launch limit of one workgroup per CU moves
-these frames from the shared form to the wave form."""
+these frames from the shared form and the dealt list to the others."""
 import ctypes
 
 import numpy as np
@@ -22,7 +23,10 @@ FRAMES = {
     "dam": lambda m, scale: ds.dam_break(n_target=61_003, block=(64, 32, 32), spacing=0.0125,
                                          grid_res=104, method=m, scale=scale),
 }
-CASES = [("yu13", "lattice36"), ("yu13", "dam")]
+FRAMES["small"] = lambda m, scale: ds.jittered_lattice(n_side=17, grid_res=56, scale=scale,
+                                                       method=m)
+CASES = [("yu13", "lattice36"), ("yu13", "dam"), ("zb05", "small"), ("zb05", "dam"),
+         ("akinci12", "small"), ("akinci12", "dam")]
 
 
 def frame_outputs(fr, method, per_cu):
@@ -37,6 +41,10 @@ def frame_outputs(fr, method, per_cu):
     if method == "yu13":
         out["mean"] = rec.buffer("mean_pos", np.uint32, 4 * fr.n)
         out["G"] = rec.buffer("g_matrices", np.uint32, 9 * res.stats["num_involved_particles"])
+    else:
+        _, cap = rec.ctx.buffer_ptr("field_work")
+        w = rec.buffer("field_work", np.uint32, cap)
+        out["work"] = w[: np.nonzero(w == 0xFFFFFFFF)[0][0]]
     return out, res.stats
 
 
@@ -49,3 +57,5 @@ def test_shared_and_wave_chunks_agree(torch_cuda, method, name):
     assert st == st1
     for k in shared:
         assert np.array_equal(shared[k], wave[k]), k
+    if name == "small" and method == "zb05":
+        assert 3 * 256 < len(shared["work"]) // 3 <= 3 * 6 * 256
