@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
     __shared__ __align__(16) float q[kAdjRows * kAdjStride];
     __shared__ float bt_lds[kWaves][4][64];  // per lane: (2p'/R^2, c0)
     __shared__ uint32_t count[kWaves];
-    __shared__ uint32_t next_chunk;
+    __shared__ uint32_t next_chunk[2];  // by the chunk's parity: see the loop's end
     __shared__ FetchState fetch;
     fetch_init(&fetch);
     const uint32_t lane = __lane_id();
@@ -351,11 +351,12 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
     ItemFetch<1, true> items(a.next, nch, &fetch);
     if (wave == 0) {
         const uint32_t first = items.next(0);
-        if (lane == 0) next_chunk = first;
+        if (lane == 0) next_chunk[0] = first;
     }
     __syncthreads();
     // workgroup-uniform
-    for (uint32_t ch = next_chunk; ch < nch; ch = next_chunk) {
+    uint32_t parity = 0;
+    for (uint32_t ch = next_chunk[0]; ch < nch; ch = next_chunk[parity]) {
         const uint32_t c = a.chunk_cell[ch];
         const uint32_t k = ch - a.chunk_off[c];
         const fsr_index_range own = a.ranges[c];
@@ -473,10 +474,13 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
                 head = (head + 64u) & (kAdjQueue - 1);
             }
         }
-        // the next chunk, fetched under the last batch
+        // the next chunk, fetched under the last batch; in the other one, as a
+        // chunk without candidates has no barrier before this, and a wave may
+        // still have to read this one's
+        parity ^= 1u;
         if (wave == 0) {
             const uint32_t nx = items.next(0);
-            if (lane == 0) next_chunk = nx;
+            if (lane == 0) next_chunk[parity] = nx;
         }
         if (fill) {
             // pad to 16 with entries that add 0: t < 0, u = 0 (head is a

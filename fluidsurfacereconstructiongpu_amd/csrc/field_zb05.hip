@@ -388,7 +388,7 @@ struct GroupLds {
     float queue[kRows * kCoopStride];
     float vtx[kFieldWaves][7][64];
     uint32_t count[kFieldWaves];
-    uint32_t next_chunk;
+    uint32_t next_chunk[2];  // by the chunk's parity: see the loop's end
 };
 
 // The shared form: the 4 waves of a workgroup treat a chunk together, for frames
@@ -410,11 +410,12 @@ __device__ __forceinline__ void field_shared(const FieldArgs& a, const BandCompa
     ItemFetch<1, true> items(a.counters->xcd_field, num_chunks, fetch);
     if (wave == 0) {
         const uint32_t nx = items.next(0);
-        if (lane == 0) L.next_chunk = nx;
+        if (lane == 0) L.next_chunk[0] = nx;
     }
     __syncthreads();
     // workgroup-uniform
-    for (uint32_t ch = L.next_chunk; ch < num_chunks; ch = L.next_chunk) {
+    uint32_t parity = 0;
+    for (uint32_t ch = L.next_chunk[0]; ch < num_chunks; ch = L.next_chunk[parity]) {
         Chunk c = load_chunk(a, bc, vd, ch, inv_r2, vt, reinterpret_cast<uint32_t*>(vt));
         wave_lds_sync();
         const uint32_t nt = (c.cnt + 15u) >> 4;
@@ -469,10 +470,13 @@ __device__ __forceinline__ void field_shared(const FieldArgs& a, const BandCompa
                 n_steps += 4u * nt;
             }
         }
-        // the next chunk, fetched under the last batch
+        // the next chunk, fetched under the last batch; in the other one, as a
+        // chunk without candidates has no barrier before this, and a wave may
+        // still have to read this one's
+        parity ^= 1u;
         if (wave == 0) {
             const uint32_t nx = items.next(0);
-            if (lane == 0) L.next_chunk = nx;
+            if (lane == 0) L.next_chunk[parity] = nx;
         }
         if (fill) {
             // pad to a multiple of 16 with entries of weight 0 (t < 0 for
