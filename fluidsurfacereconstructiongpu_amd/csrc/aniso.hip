@@ -1196,16 +1196,16 @@ constexpr int kAfOneMinusC = 8, kAfBz = 9, kAfCoef = 10, kAfRows = 11;
 // at the particle).  Lane l holds the pairs of candidates 4(l/16)+r (r = 0..3)
 // with vertex l%16 of each tile and adds c e^3 to part[T]; the caller adds
 // the partial sums of the four lane groups of a vertex.
-template <int NT>
+template <int NT, int kStride>
 __device__ __forceinline__ void aniso_tiles(const float* __restrict__ rows, uint32_t n,
                                             const float (&b1)[NT], const float (&b2)[NT],
                                             const float (&z2)[NT], float (&part)[NT]) {
     const uint32_t lane = __lane_id();
-    const float* a1p = rows + (lane >> 4) * kAfStride + (lane & 15u);
-    const float* a2p = rows + (4u + (lane >> 4)) * kAfStride + (lane & 15u);
-    const float* cp = rows + kAfOneMinusC * kAfStride + 4u * (lane >> 4);
-    const float* zp = rows + kAfBz * kAfStride + 4u * (lane >> 4);
-    const float* kp = rows + kAfCoef * kAfStride + 4u * (lane >> 4);
+    const float* a1p = rows + (lane >> 4) * kStride + (lane & 15u);
+    const float* a2p = rows + (4u + (lane >> 4)) * kStride + (lane & 15u);
+    const float* cp = rows + kAfOneMinusC * kStride + 4u * (lane >> 4);
+    const float* zp = rows + kAfBz * kStride + 4u * (lane >> 4);
+    const float* kp = rows + kAfCoef * kStride + 4u * (lane >> 4);
     for (uint32_t tb = 0; tb < n; tb += 16u) {
         const float a1 = a1p[tb];
         const float a2 = a2p[tb];
@@ -1232,45 +1232,284 @@ __device__ __forceinline__ void aniso_tiles(const float* __restrict__ rows, uint
     }
 }
 
+// Queue entry of a candidate at p (relative to the cell corner) with record
+// (r0, r1).
+template <int kStride>
+__device__ __forceinline__ void af_enter(float* __restrict__ q, float px, float py, float pz,
+                                         const float4& r0, const float4& r1) {
+    const float M00 = r0.x, M11 = r0.y, M22 = r0.z, M01 = r0.w;
+    const float M02 = r1.x, M12 = r1.y;
+    const float bx = M00 * px + M01 * py + M02 * pz;
+    const float by = M01 * px + M11 * py + M12 * pz;
+    const float bz = M02 * px + M12 * py + M22 * pz;
+    const float cc = px * bx + py * by + pz * bz;
+    q[0 * kStride] = M00;
+    q[1 * kStride] = M11;
+    q[2 * kStride] = M22;
+    q[3 * kStride] = M01;
+    q[4 * kStride] = M02;
+    q[5 * kStride] = M12;
+    q[6 * kStride] = bx;
+    q[7 * kStride] = by;
+    q[kAfOneMinusC * kStride] = 1.0f - cc;
+    q[kAfBz * kStride] = bz;
+    q[kAfCoef * kStride] = r1.z;
+}
+
+// A field chunk as its waves know it: virtual cell, this lane's vertex (relative
+// to the cell corner o), the box of the chunk's vertices and the candidate rows.
+struct AfChunk {
+    uint32_t v, cnt, vid;
+    bool live;
+    float o[3], x[3], b0[3], b1[3];
+    BlockRows br;
+};
+
+// Value of the field at a vertex from its candidates' sum.
+__device__ __forceinline__ void af_store(const AnisoFieldArgs& a, const AfChunk& c, float sum) {
+    if (a.block_mom) {
+        const double px = (double)(c.x[0] + c.o[0]) - a.ox, py = (double)(c.x[1] + c.o[1]) - a.oy,
+                     pz = (double)(c.x[2] + c.o[2]) - a.oz;
+        const double pn = noninv_poly(a.block_mom + (uint64_t)kNonInvMoments * c.v, px, py, pz);
+        a.phi[c.vid] = (float)((double)sum + pn - 0.5);
+    } else {
+        a.phi[c.vid] = sum - 0.5f;
+    }
+}
+
+// Cell, vertices and their box (the rows follow with af_rows).
+__device__ __forceinline__ void af_vertices(const AnisoFieldArgs& a, uint32_t ch, AfChunk& c,
+                                            int (&cell)[3]) {
+    const uint32_t lane = __lane_id();
+    const int R = a.bc.radius;
+    c.v = a.bc.chunk_cell[ch];
+    cell[0] = (int)(c.v % a.bc.vcx) - R;
+    cell[1] = (int)((c.v / a.bc.vcx) % a.bc.vcy) - R;
+    cell[2] = (int)(c.v / (a.bc.vcx * a.bc.vcy)) - R;
+    const uint32_t k = ch - a.bc.chunk_off[c.v];
+    const uint32_t first = a.bc.cell_off[c.v] + 64u * k;
+    c.cnt = min(64u, a.bc.cell_cnt[c.v] - 64u * k);
+    c.o[0] = __builtin_fmaf((float)cell[0], a.sp.cell, a.sp.minx);
+    c.o[1] = __builtin_fmaf((float)cell[1], a.sp.cell, a.sp.miny);
+    c.o[2] = __builtin_fmaf((float)cell[2], a.sp.cell, a.sp.minz);
+    c.vid = 0;
+    c.x[0] = c.x[1] = c.x[2] = 0.f;
+    c.live = lane < c.cnt;
+    if (c.live) {
+        c.vid = a.bc.cell_band[first + lane];
+        const uint32_t ix = c.vid % a.sc.rx;
+        const uint32_t iy = (c.vid / a.sc.rx) % a.sc.ry;
+        const uint32_t iz = c.vid / (a.sc.rx * a.sc.ry);
+        c.x[0] = vertex_coord(ix, a.sc.minx, a.sc.cell) - c.o[0];
+        c.x[1] = vertex_coord(iy, a.sc.miny, a.sc.cell) - c.o[1];
+        c.x[2] = vertex_coord(iz, a.sc.minz, a.sc.cell) - c.o[2];
+    }
+}
+
+// The box, and the block's candidate rows; with the non-involved moments only
+// the cells whose involved particles can reach the chunk's vertices.
+__device__ __forceinline__ void af_rows(const AnisoFieldArgs& a, const int (&cell)[3], AfChunk& c) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) wave_range(c.live, c.x[d], &c.b0[d], &c.b1[d]);
+    if (a.block_mom) {
+        CellCull cc;
+        cc.lo = a.cell_lo;
+        cc.hi = a.cell_hi;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            cc.b0[d] = c.b0[d] + c.o[d];
+            cc.b1[d] = c.b1[d] + c.o[d];
+        }
+        c.br = block_rows<2>(a.ranges, a.sp, cell[0], cell[1], cell[2], &cc);
+    } else {
+        c.br = block_rows<2>(a.ranges, a.sp, cell[0], cell[1], cell[2]);
+    }
+}
+
+struct AfWaveLds {
+    float queue[kAnisoThreads / 64][kAfRows * kAfStride];
+};
+struct AfGroupLds {
+    float queue[kAfRows * kCoopStride];
+    uint32_t count[kAnisoThreads / 64];
+    uint32_t next_chunk[2];  // by the chunk's parity: see the loop's end
+};
+
+// The field with a workgroup's waves sharing each chunk (see coop_limit): a
+// wave stages a quarter of a 256-candidate round, and evaluates one of the
+// chunk's 16-vertex tiles.  Candidates, their order, the batches of 64 and
+// every tile's operations are those of the wave form, so the field is the same
+// bits.  The survivors' records are loaded in one round and enter the ring in
+// the next, as there; two barriers a round, one after the counts (the previous
+// batches are evaluated by then) and one after the entries.  A frame with few
+// chunks is bound by the time of a chunk, which this cuts: 9,216-particle block
+// 60 -> 31 us, 31k-particle dam break at 113^3 165 -> 140.  It holds to 6 chunks
+// per workgroup (64k particles at 150^3 175 -> 157 us with that limit, 174 with
+// 3; 125k particles at 190^3, 281 us either way, take 307 with a limit of 12).
+__device__ __forceinline__ void field_aniso_shared(const AnisoFieldArgs& a, AfGroupLds& L,
+                                                   uint32_t nch, FetchState* fetch) {
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = threadIdx.x >> 6;
+    float* q = L.queue;
+    uint32_t n_staged = 0, n_kept = 0;
+    ItemFetch<1, true> items(a.next, nch, fetch);
+    if (wave == 0) {
+        const uint32_t nx = items.next(0);
+        if (lane == 0) L.next_chunk[0] = nx;
+    }
+    __syncthreads();
+    // workgroup-uniform
+    uint32_t parity = 0;
+    for (uint32_t ch = L.next_chunk[0]; ch < nch; ch = L.next_chunk[parity]) {
+        AfChunk c;
+        int cell[3];
+        af_vertices(a, ch, c, cell);
+        af_rows(a, cell, c);
+        const uint32_t total = c.br.total;
+        n_staged += wave == 0 ? total : 0u;
+        const uint32_t nt = (c.cnt + 15u) >> 4;
+        const bool mine = wave < nt;
+        // lane l: component l/16 of the operands of vertex 16 wave + l%16
+        float b1[1], b2[1], z2[1], tot = 0.f;
+        {
+            const int src = (int)(16u * wave + (lane & 15u));
+            const float vx = __shfl(c.x[0], src, 64), vy = __shfl(c.x[1], src, 64),
+                        vz = __shfl(c.x[2], src, 64);
+            const uint32_t k = lane >> 4;
+            b1[0] = k == 0u ? -(vx * vx) : k == 1u ? -(vy * vy) : k == 2u ? -(vz * vz)
+                                                                : -(2.0f * vx * vy);
+            b2[0] = k == 0u ? -(2.0f * vx * vz) : k == 1u ? -(2.0f * vy * vz)
+                                                : k == 2u ? 2.0f * vx : 2.0f * vy;
+            z2[0] = 2.0f * vz;
+        }
+        uint32_t head = 0, fill = 0;
+        float4 np4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        uint32_t nj = c.br.offset(64u * wave, 64u * wave + lane) + 64u * wave + lane;
+        if (64u * wave + lane < total) np4 = a.smooth[nj];
+        bool keep_p = false;
+        float px_p = 0.f, py_p = 0.f, pz_p = 0.f;
+        float4 r0_p = make_float4(0.f, 0.f, 0.f, 0.f), r1_p = r0_p;
+        for (uint32_t base = 0; base < total + 256u; base += 256u) {
+            const uint32_t g = base + 64u * wave + lane;
+            bool keep = false;
+            float px = 0.f, py = 0.f, pz = 0.f;
+            float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0;
+            if (base < total) {
+                const float4 p4 = np4;
+                const uint32_t j = nj;
+                if (base + 256u < total) {
+                    nj = c.br.offset(base + 256u + 64u * wave, g + 256u) + g + 256u;
+                    if (g + 256u < total) np4 = a.smooth[nj];
+                }
+                if (g < total) {
+                    px = p4.x - c.o[0];
+                    py = p4.y - c.o[1];
+                    pz = p4.z - c.o[2];
+                    const float dx = px - __builtin_amdgcn_fmed3f(px, c.b0[0], c.b1[0]);
+                    const float dy = py - __builtin_amdgcn_fmed3f(py, c.b0[1], c.b1[1]);
+                    const float dz = pz - __builtin_amdgcn_fmed3f(pz, c.b0[2], c.b1[2]);
+                    keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < p4.w;
+                }
+                const uint32_t jr = keep ? j : 0u;
+                r0 = a.rec[2ull * jr + 0];
+                r1 = a.rec[2ull * jr + 1];
+            }
+            if (base) {
+                // the previous round's survivors enter the ring
+                const uint64_t m = __ballot(keep_p);
+                if (lane == 0) L.count[wave] = (uint32_t)__popcll(m);
+                __syncthreads();
+                uint32_t before = 0, added = 0;
+#pragma unroll
+                for (uint32_t w = 0; w < kAnisoThreads / 64; ++w) {
+                    const uint32_t n = L.count[w];
+                    before += w < wave ? n : 0u;
+                    added += n;
+                }
+                if (keep_p) {
+                    const uint32_t slot = (head + fill + before + mask_rank(m)) & (kCoopQueue - 1);
+                    af_enter<kCoopStride>(q + slot, px_p, py_p, pz_p, r0_p, r1_p);
+                }
+                fill += added;
+                n_kept += wave == 0 ? added : 0u;
+                __syncthreads();
+                for (; fill >= 64u; fill -= 64u) {
+                    if (mine) {
+                        float part[1] = {0.f};
+                        aniso_tiles<1, kCoopStride>(q + head, 64u, b1, b2, z2, part);
+                        tot += part[0];
+                    }
+                    head = (head + 64u) & (kCoopQueue - 1);
+                }
+            }
+            keep_p = keep;
+            px_p = px; py_p = py; pz_p = pz;
+            r0_p = r0; r1_p = r1;
+        }
+        // the next chunk, fetched under the last batch; in the other one, as a
+        // chunk without candidates has no barrier before this, and a wave may
+        // still have to read this one's
+        parity ^= 1u;
+        if (wave == 0) {
+            const uint32_t nx = items.next(0);
+            if (lane == 0) L.next_chunk[parity] = nx;
+        }
+        if (fill) {
+            // pad to a multiple of 16 (see the wave form)
+            const uint32_t n = (fill + 15u) & ~15u;
+            if (wave == 0 && lane >= fill && lane < n) {
+#pragma unroll
+                for (int rr = 0; rr < kAfRows; ++rr)
+                    q[rr * kCoopStride + head + lane] = rr == kAfOneMinusC ? -1.0f : 0.0f;
+            }
+            __syncthreads();
+            if (mine) {
+                float part[1] = {0.f};
+                aniso_tiles<1, kCoopStride>(q + head, n, b1, b2, z2, part);
+                tot += part[0];
+            }
+        }
+        // the next chunk rewrites the ring from its start
+        __syncthreads();
+        float x = tot;
+        x += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(x), 0x1F | (16 << 10)));
+        x += __shfl_xor(x, 32, 64);
+        if (c.live && (lane >> 4) == wave) af_store(a, c, x);
+    }
+    if (a.work) write_work(a.work, n_staged, n_kept);
+}
+
 // kWaves: the resident waves per SIMD the register allocation is bounded for
-// (5: 96 VGPRs; 4: 128 VGPRs).
+// (5: 96 VGPRs; 4: 128 VGPRs).  kSmall: the build for smaller frames (see
+// few_chunks), with the shared form, taken at up to coop_max chunks, and the
+// fetch for short lists.
 template <int kWaves, bool kSmall>
-__global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFieldArgs a) {
-    __shared__ __align__(16) float queue[kAnisoThreads / 64][kAfRows * kAfStride];
+__global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFieldArgs a,
+                                                                       uint32_t coop_max) {
+    __shared__ __align__(16) union {
+        AfWaveLds waves;
+        AfGroupLds group;
+    } lds;
     __shared__ FetchState fetch;
     fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nch = *a.num_chunks;
-    const int R = a.bc.radius;
-    float* q = queue[wave];
+    if (kSmall && nch <= coop_max) {
+        field_aniso_shared(a, lds.group, nch, &fetch);
+        return;
+    }
+    float* q = lds.waves.queue[wave];
     uint32_t n_staged = 0, n_kept = 0;
     ItemFetch<kAnisoThreads / 64, kSmall> items(a.next, nch, &fetch);
     for (;;) {
         const uint32_t ch = items.next(wave);
         if (ch >= nch) break;
-        const uint32_t v = a.bc.chunk_cell[ch];
-        const int cx = (int)(v % a.bc.vcx) - R;
-        const int cy = (int)((v / a.bc.vcx) % a.bc.vcy) - R;
-        const int cz = (int)(v / (a.bc.vcx * a.bc.vcy)) - R;
-        const uint32_t k = ch - a.bc.chunk_off[v];
-        const uint32_t first = a.bc.cell_off[v] + 64u * k;
-        const uint32_t cnt = min(64u, a.bc.cell_cnt[v] - 64u * k);
-        const float ox = __builtin_fmaf((float)cx, a.sp.cell, a.sp.minx);
-        const float oy = __builtin_fmaf((float)cy, a.sp.cell, a.sp.miny);
-        const float oz = __builtin_fmaf((float)cz, a.sp.cell, a.sp.minz);
-        uint32_t vid = 0;
-        float vx = 0.f, vy = 0.f, vz = 0.f;
-        const bool live = lane < cnt;
-        if (live) {
-            vid = a.bc.cell_band[first + lane];
-            const uint32_t ix = vid % a.sc.rx;
-            const uint32_t iy = (vid / a.sc.rx) % a.sc.ry;
-            const uint32_t iz = vid / (a.sc.rx * a.sc.ry);
-            vx = vertex_coord(ix, a.sc.minx, a.sc.cell) - ox;
-            vy = vertex_coord(iy, a.sc.miny, a.sc.cell) - oy;
-            vz = vertex_coord(iz, a.sc.minz, a.sc.cell) - oz;
-        }
+        AfChunk c;
+        int cell[3];
+        af_vertices(a, ch, c, cell);
+        const float ox = c.o[0], oy = c.o[1], oz = c.o[2];
+        const float vx = c.x[0], vy = c.x[1], vz = c.x[2];
         // the vertex operands (negated terms, and 2z) into the ring's upper half
         float* vt = q + kAfQueue / 2;
         vt[0 * kAfStride + lane] = -(vx * vx);
@@ -1282,27 +1521,14 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
         vt[6 * kAfStride + lane] = 2.0f * vx;
         vt[7 * kAfStride + lane] = 2.0f * vy;
         vt[8 * kAfStride + lane] = 2.0f * vz;
-        float bx0, bx1, by0, by1, bz0, bz1;
-        wave_range(live, vx, &bx0, &bx1);
-        wave_range(live, vy, &by0, &by1);
-        wave_range(live, vz, &bz0, &bz1);
-        // the block's candidate rows; with the non-involved moments only the
-        // cells whose involved particles can reach the chunk's vertices
-        BlockRows br;
-        if (a.block_mom) {
-            CellCull cc;
-            cc.lo = a.cell_lo;
-            cc.hi = a.cell_hi;
-            cc.b0[0] = bx0 + ox; cc.b0[1] = by0 + oy; cc.b0[2] = bz0 + oz;
-            cc.b1[0] = bx1 + ox; cc.b1[1] = by1 + oy; cc.b1[2] = bz1 + oz;
-            br = block_rows<2>(a.ranges, a.sp, cx, cy, cz, &cc);
-        } else {
-            br = block_rows<2>(a.ranges, a.sp, cx, cy, cz);
-        }
+        af_rows(a, cell, c);
+        const float bx0 = c.b0[0], bx1 = c.b1[0], by0 = c.b0[1], by1 = c.b1[1], bz0 = c.b0[2],
+                    bz1 = c.b1[2];
+        BlockRows& br = c.br;
         const uint32_t total = br.total;
         n_staged += total;
         wave_lds_sync();
-        const int nt = (int)((cnt + 15u) >> 4);
+        const int nt = (int)((c.cnt + 15u) >> 4);
         float sum = 0.f;
         // The rest of the chunk, compiled once per tile count NT, so that the
         // vertex operands and sums keep fixed registers across the staging.
@@ -1373,24 +1599,8 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
                 // the previous round's survivors enter the queue
                 const uint64_t m = __ballot(keep_p);
                 if (keep_p) {
-                    const float M00 = r0_p.x, M11 = r0_p.y, M22 = r0_p.z, M01 = r0_p.w;
-                    const float M02 = r1_p.x, M12 = r1_p.y;
-                    const float bx = M00 * px_p + M01 * py_p + M02 * pz_p;
-                    const float by = M01 * px_p + M11 * py_p + M12 * pz_p;
-                    const float bz = M02 * px_p + M12 * py_p + M22 * pz_p;
-                    const float cc = px_p * bx + py_p * by + pz_p * bz;
                     const uint32_t o = (head + fill + mask_rank(m)) & (kAfQueue - 1);
-                    q[0 * kAfStride + o] = M00;
-                    q[1 * kAfStride + o] = M11;
-                    q[2 * kAfStride + o] = M22;
-                    q[3 * kAfStride + o] = M01;
-                    q[4 * kAfStride + o] = M02;
-                    q[5 * kAfStride + o] = M12;
-                    q[6 * kAfStride + o] = bx;
-                    q[7 * kAfStride + o] = by;
-                    q[kAfOneMinusC * kAfStride + o] = 1.0f - cc;
-                    q[kAfBz * kAfStride + o] = bz;
-                    q[kAfCoef * kAfStride + o] = r1_p.z;
+                    af_enter<kAfStride>(q + o, px_p, py_p, pz_p, r0_p, r1_p);
                 }
                 keep_p = keep;
                 px_p = px; py_p = py; pz_p = pz;
@@ -1405,7 +1615,7 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
 #pragma unroll
                     for (int T = 0; T < NT; ++T) part[T] = 0.f;
                     wave_lds_sync();
-                    aniso_tiles<NT>(q + head, 64u, b1, b2, z2, part);
+                    aniso_tiles<NT, kAfStride>(q + head, 64u, b1, b2, z2, part);
                     wave_lds_sync();
 #pragma unroll
                     for (int T = 0; T < NT; ++T) tot[T] += part[T];
@@ -1427,7 +1637,7 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
 #pragma unroll
                 for (int T = 0; T < NT; ++T) part[T] = 0.f;
                 wave_lds_sync();
-                aniso_tiles<NT>(q + head, n, b1, b2, z2, part);
+                aniso_tiles<NT, kAfStride>(q + head, n, b1, b2, z2, part);
                 wave_lds_sync();
 #pragma unroll
                 for (int T = 0; T < NT; ++T) tot[T] += part[T];
@@ -1449,16 +1659,7 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
             case 3: run(std::integral_constant<int, 3>{}); break;
             default: run(std::integral_constant<int, 4>{}); break;
         }
-        if (live) {
-            if (a.block_mom) {
-                const double px = (double)(vx + ox) - a.ox, py = (double)(vy + oy) - a.oy,
-                             pz = (double)(vz + oz) - a.oz;
-                const double pn = noninv_poly(a.block_mom + (uint64_t)kNonInvMoments * v, px, py, pz);
-                a.phi[vid] = (float)((double)sum + pn - 0.5);
-            } else {
-                a.phi[vid] = sum - 0.5f;
-            }
-        }
+        if (c.live) af_store(a, c, sum);
     }
     if (a.work) write_work(a.work, n_staged, n_kept);
 }
@@ -1841,7 +2042,8 @@ fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOu
     auto kernel = field_waves == 4 ? k_field_aniso<4, false> : k_field_aniso<5, false>;
     if (few_chunks(ctx, a.n))
         kernel = field_waves == 4 ? k_field_aniso<4, true> : k_field_aniso<5, true>;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kAnisoThreads), 0, s, fa);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kAnisoThreads), 0, s, fa,
+                       2u * coop_limit(ctx, blocks));
     FSR_LAUNCH_CHECK("k_field_aniso");
     return FSR_OK;
 }
