@@ -43,12 +43,6 @@ constexpr int kAdjThreads = 256;
 
 __constant__ uint64_t cAdjTri[256] = {FSR_MC_TRI_PACKED_VALUES};
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ uint32_t corner_dx(uint32_t c) { return c >= 4 ? 1u : 0u; }
 __device__ __forceinline__ uint32_t corner_dy(uint32_t c) {
     return (c == 2 || c == 3 || c == 6 || c == 7) ? 1u : 0u;
@@ -564,7 +558,7 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
     float4* vpos = coef + V;
     {
         const int blocks = persistent_blocks(ctx, kAdjThreads, 4, TUNE_MC);
-        hipLaunchKernelGGL(k_field_coef, dim3(blocks), dim3(kAdjThreads), 0, s, st.bc.cell_band,
+        hipLaunchKernelGGL(k_field_coef, dim3(blocks), dim3(kAdjThreads), 0, s, st.cell_band,
                            st.saved, g_phi, st.stats, st.sc, coef, vpos);
         FSR_LAUNCH_CHECK("k_field_coef");
     }
@@ -589,7 +583,7 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
     a.next = next;
     a.cell_off = st.bc.cell_off;
     a.cell_cnt = st.bc.cell_cnt;
-    a.cell_band = st.bc.cell_band;
+    a.cell_band = st.cell_band;
     a.coef = coef;
     a.vpos = vpos;
     a.sp = st.sp;

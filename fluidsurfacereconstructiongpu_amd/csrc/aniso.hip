@@ -40,6 +40,7 @@
 #include <type_traits>
 #include <limits>
 
+#include "chunk_list.hpp"
 #include "common.hpp"
 
 namespace fsr {
@@ -66,12 +67,6 @@ constexpr float kNoCull = 3.0e38f;
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) {
     return v < lo ? lo : (v > hi ? hi : v);
-}
-
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Rows (x-runs) of the clamped (2R+1)^3 block around cell (cx, cy, cz), lane
@@ -1277,9 +1272,10 @@ __device__ __forceinline__ void af_store(const AnisoFieldArgs& a, const AfChunk&
     }
 }
 
-// Cell, vertices and their box (the rows follow with af_rows).
-__device__ __forceinline__ void af_vertices(const AnisoFieldArgs& a, uint32_t ch, AfChunk& c,
-                                            int (&cell)[3]) {
+// Cell and vertices, listed through `scratch` (64 words of LDS); their box and the
+// rows follow with af_rows.
+__device__ __forceinline__ void af_vertices(const AnisoFieldArgs& a, uint32_t ch,
+                                            uint32_t* scratch, AfChunk& c, int (&cell)[3]) {
     const uint32_t lane = __lane_id();
     const int R = a.bc.radius;
     c.v = a.bc.chunk_cell[ch];
@@ -1287,16 +1283,15 @@ __device__ __forceinline__ void af_vertices(const AnisoFieldArgs& a, uint32_t ch
     cell[1] = (int)((c.v / a.bc.vcx) % a.bc.vcy) - R;
     cell[2] = (int)(c.v / (a.bc.vcx * a.bc.vcy)) - R;
     const uint32_t k = ch - a.bc.chunk_off[c.v];
-    const uint32_t first = a.bc.cell_off[c.v] + 64u * k;
     c.cnt = min(64u, a.bc.cell_cnt[c.v] - 64u * k);
+    c.vid = chunk_vertex(a.bc, a.sc.rx, a.sc.ry, c.v, k, c.cnt, scratch);
     c.o[0] = __builtin_fmaf((float)cell[0], a.sp.cell, a.sp.minx);
     c.o[1] = __builtin_fmaf((float)cell[1], a.sp.cell, a.sp.miny);
     c.o[2] = __builtin_fmaf((float)cell[2], a.sp.cell, a.sp.minz);
-    c.vid = 0;
     c.x[0] = c.x[1] = c.x[2] = 0.f;
-    c.live = lane < c.cnt;
+    // lanes with a vertex (an id past the grid would mean an empty slot)
+    c.live = lane < c.cnt && c.vid < a.sc.rx * a.sc.ry * a.sc.rz;
     if (c.live) {
-        c.vid = a.bc.cell_band[first + lane];
         const uint32_t ix = c.vid % a.sc.rx;
         const uint32_t iy = (c.vid / a.sc.rx) % a.sc.ry;
         const uint32_t iz = c.vid / (a.sc.rx * a.sc.ry);
@@ -1333,6 +1328,7 @@ struct AfGroupLds {
     float queue[kAfRows * kCoopStride];
     uint32_t count[kAnisoThreads / 64];
     uint32_t next_chunk[2];  // by the chunk's parity: see the loop's end
+    uint32_t ids[kAnisoThreads / 64][64];
 };
 
 // The field with a workgroup's waves sharing each chunk (see coop_limit): a
@@ -1363,7 +1359,7 @@ __device__ __forceinline__ void field_aniso_shared(const AnisoFieldArgs& a, AfGr
     for (uint32_t ch = L.next_chunk[0]; ch < nch; ch = L.next_chunk[parity]) {
         AfChunk c;
         int cell[3];
-        af_vertices(a, ch, c, cell);
+        af_vertices(a, ch, L.ids[wave], c, cell);
         af_rows(a, cell, c);
         const uint32_t total = c.br.total;
         n_staged += wave == 0 ? total : 0u;
@@ -1507,7 +1503,7 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
         if (ch >= nch) break;
         AfChunk c;
         int cell[3];
-        af_vertices(a, ch, c, cell);
+        af_vertices(a, ch, reinterpret_cast<uint32_t*>(q), c, cell);
         const float ox = c.o[0], oy = c.o[1], oz = c.o[2];
         const float vx = c.x[0], vy = c.x[1], vz = c.x[2];
         // the vertex operands (negated terms, and 2z) into the ring's upper half

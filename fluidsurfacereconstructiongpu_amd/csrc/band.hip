@@ -571,20 +571,21 @@ __device__ __forceinline__ uint32_t layer_rows(const AxisMaps& m, const GridDev&
     return b;
 }
 
-// Cell-major band list, built per slab: the slab (cx, cy, z) is the part of
+// Cell-major band order, counted per slab: the slab (cx, cy, z) is the part of
 // virtual cell v = (cz vcy + cy) vcx + cx (cz = vc_z[z]) on scalar layer z.
 // Slabs are stored cell by cell and by layer inside a cell:
 //   slab(cx, cy, z) = vcx vcy lo_z[cz] + (cy vcx + cx) nz(cz) + (z - lo_z[cz]),
-// so the exclusive scan of the slab counts is each slab's offset in the cell
-// list, and a cell's vertices come out in ascending id order (layers z, rows
-// y, then x), i.e. a 64-vertex chunk is a compact slab of the cell, which
-// keeps the candidate culling of the field kernels effective.  The count pass
-// takes one thread per slab (consecutive threads = consecutive cx, which read
-// the same row words); rows without band vertices are skipped with the row
-// occupancy bits.  It writes the slab's band vertex count and adds it to its
-// cell's count (cnt, cleared by k_axis_maps).  The fill pass (k_slab_fill)
-// writes the slab's vertex ids at its scanned offset.  The list itself is
-// deterministic.
+// so a cell's vertices come in ascending id order (layers z, rows y, then x),
+// i.e. a 64-vertex chunk is a compact slab of the cell, which keeps the
+// candidate culling of the field kernels effective.  The list itself is not
+// written: the field kernels read a chunk's vertices from the mask with the
+// slab counts (chunk_vertex).  The count pass takes one thread per slab
+// (consecutive threads = consecutive cx, which read the same row words); rows
+// without band vertices are skipped with the row occupancy bits.  It writes the
+// slab's band vertex count and adds it to its cell's count (cnt, cleared by
+// k_axis_maps).  Writing the list too took 19 us at 113^3 and 41 us at 384^3,
+// and the scan before it 9; listing costs the Yu13
+// field 5 and 20 us there.
 __global__ __launch_bounds__(256) void k_slab_rows(const uint32_t* __restrict__ bits, GridDev sc,
                                                    uint32_t wx, AxisMaps m, uint32_t vcx,
                                                    uint32_t vcy, uint32_t* __restrict__ slab,
@@ -645,101 +646,6 @@ __global__ __launch_bounds__(256) void k_slab_rows(const uint32_t* __restrict__ 
         }
         slab[idx] = o;
         if (o) atomicAdd(&cnt[v], o);
-    }
-}
-
-// Fill pass in slab order: thread t of block b takes slab idx = 256 b + t, so
-// the block's slabs own one contiguous range of the cell list.  The slab's ids
-// are written to LDS (serial over its set bits) and the block then copies the
-// range out with consecutive threads on consecutive entries.  A slab idx
-// decodes as: layer q = idx / (vcx vcy) lies in the layer range of the slab's
-// z-cell cz = vc_z[q]; r = idx - vcx vcy lo_z[cz] = (cy vcx + cx) nz + (z - lo_z).
-__global__ __launch_bounds__(256) void k_slab_fill(const uint32_t* __restrict__ bits, GridDev sc,
-                                                   uint32_t wx, AxisMaps m, uint32_t vcx,
-                                                   uint32_t vcy, const uint32_t* __restrict__ slab,
-                                                   const uint32_t* __restrict__ slab_off,
-                                                   uint32_t* __restrict__ cell_band, uint64_t cap,
-                                                   uint64_t nslabs) {
-    constexpr uint32_t kStage = 8192;
-    __shared__ uint32_t stage[kStage];
-    __shared__ uint32_t range[2];
-    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x;
-    const uint64_t idx = first + threadIdx.x;
-    const uint64_t last = min(first + blockDim.x, nslabs) - 1;
-    if (threadIdx.x == 0) {
-        range[0] = slab_off[first];
-        range[1] = slab_off[last] + slab[last];
-    }
-    __syncthreads();
-    const uint32_t lo = range[0], total = range[1] - range[0];
-    const bool staged = total <= kStage;
-    uint32_t n = idx < nslabs ? slab[idx] : 0u;
-    if (n) {
-        const uint64_t layer = (uint64_t)vcx * vcy;
-        const uint32_t q = (uint32_t)(idx / layer);
-        const uint32_t cz = m.vc[2][q];
-        const uint32_t zlo = m.lo[2][cz], nz = m.hi[2][cz] - zlo;
-        const uint64_t r = idx - layer * zlo;
-        const uint32_t c = (uint32_t)(r / nz);
-        const uint32_t z = zlo + (uint32_t)(r - (uint64_t)c * nz);
-        const uint32_t cx = c % vcx, cy = c / vcx;
-        uint32_t o = slab_off[idx];
-        const uint32_t ylo = m.lo[1][cy], yhi = m.hi[1][cy];
-        const uint32_t xlo = m.lo[0][cx], xhi = m.hi[0][cx];
-        const uint32_t ny = yhi > ylo ? yhi - ylo : 0u;
-        const uint32_t w0 = xlo >> 5;
-        const uint32_t nw = xhi > xlo ? ((xhi + 31u) >> 5) - w0 : 0u;
-        // the slab's ids in row order, then word order
-        auto put = [&](uint64_t row, uint32_t w, uint32_t word) {
-            word = clip_word(word, w, xlo, xhi);
-            const uint32_t base = (uint32_t)(row * sc.rx) + w * 32u;
-            while (word) {
-                const uint32_t id = base + __builtin_ctz(word);
-                if (staged) stage[o - lo] = id;
-                else if (o < cap) cell_band[o] = id;
-                ++o;
-                word &= word - 1u;
-            }
-        };
-        for (uint32_t yb = 0; nw && yb < ny; yb += 32u) {
-            uint32_t rows = layer_rows(m, sc, z, ylo, yb, ny);
-            while (rows) {
-                // up to 4 occupied rows per round; with at most 2 words per
-                // row (the common case) their 8 words are loaded together
-                uint64_t rr[4];
-                bool ok[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    ok[k] = rows != 0u;
-                    const uint32_t dy = ok[k] ? (uint32_t)__builtin_ctz(rows) : 0u;
-                    rr[k] = (uint64_t)z * sc.ry + ylo + yb + dy;
-                    rows &= rows - 1u;
-                }
-                if (nw <= 2u) {
-                    uint32_t v0[4], v1[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        v0[k] = ok[k] ? bits[rr[k] * wx + w0] : 0u;
-                        v1[k] = ok[k] && nw == 2u ? bits[rr[k] * wx + w0 + 1u] : 0u;
-                    }
-                    for (int k = 0; k < 4; ++k) {
-                        if (!ok[k]) break;
-                        put(rr[k], w0, v0[k]);
-                        if (nw == 2u) put(rr[k], w0 + 1u, v1[k]);
-                    }
-                } else {
-                    for (int k = 0; k < 4; ++k) {
-                        if (!ok[k]) break;
-                        for (uint32_t j = 0; j < nw; ++j) put(rr[k], w0 + j, bits[rr[k] * wx + w0 + j]);
-                    }
-                }
-            }
-        }
-    }
-    if (staged) {
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < total; k += blockDim.x)
-            if ((uint64_t)lo + k < cap) cell_band[lo + k] = stage[k];
     }
 }
 
@@ -807,7 +713,7 @@ fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s) {
 
 fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& sc,
                         const GridDev& sp, int radius, Counters* counters, fsr_frame_stats* st,
-                        BandCompactOut* out, hipStream_t s, bool materialize) {
+                        BandCompactOut* out, hipStream_t s) {
     const uint32_t wx = row_words(sc.rx);
     const uint64_t nwords = (uint64_t)wx * sc.ry * sc.rz;
     const uint64_t V = (uint64_t)sc.rx * sc.ry * sc.rz;
@@ -834,7 +740,7 @@ fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& s
     // cell-major work list
     const uint32_t vcx = sp.rx + 2 * radius, vcy = sp.ry + 2 * radius, vcz = sp.rz + 2 * radius;
     const uint64_t nvc = (uint64_t)vcx * vcy * vcz;
-    uint32_t *maps, *cnt, *cell_off, *chunk_off, *cell_band, *chunk_cell;
+    uint32_t *maps, *cnt, *cell_off, *chunk_off, *chunk_cell;
     const uint64_t rows = (uint64_t)sc.ry * sc.rz;
     const uint64_t row_words = 2ull * ((rows + 63) / 64);
     const uint64_t map_len =
@@ -843,8 +749,6 @@ fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& s
     FSR_TRY(arena_typed(ctx, A_CELL_CNT, nvc, &cnt));
     FSR_TRY(arena_typed(ctx, A_CELL_OFF, nvc, &cell_off));
     FSR_TRY(arena_typed(ctx, A_CHUNK_OFF, nvc, &chunk_off));
-    cell_band = nullptr;
-    if (materialize) FSR_TRY(arena_typed(ctx, A_CELL_BAND, V, &cell_band));
     const uint64_t max_chunks = V / 64 + nvc + 1;
     FSR_TRY(arena_typed(ctx, A_CHUNK_CELL, max_chunks, &chunk_cell));
     AxisMaps m;
@@ -865,29 +769,20 @@ fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& s
     hipLaunchKernelGGL(k_axis_maps, dim3(map_blocks, 5), dim3(256), 0, s, sc, sp, radius, m, bits,
                        wx, cnt, nvc);
     FSR_LAUNCH_CHECK("k_axis_maps");
-    // slab counts (and cell counts) -> slab offsets; cell offsets, chunk
-    // offsets and the chunk list in one scan -> slab fill
+    // slab counts (and cell counts); cell offsets, chunk offsets and the chunk
+    // list in one scan
     const uint64_t nslabs = (uint64_t)vcx * vcy * sc.rz;
-    uint32_t *slab, *slab_off;
-    FSR_TRY(arena_typed(ctx, A_SLAB, 2 * nslabs, &slab));
-    slab_off = slab + nslabs;
+    uint32_t* slab;
+    FSR_TRY(arena_typed(ctx, A_SLAB, nslabs, &slab));
     const uint32_t slab_blocks = (uint32_t)std::min<uint64_t>((nslabs + 255) / 256, 16384);
     hipLaunchKernelGGL(k_slab_rows, dim3(slab_blocks), dim3(256), 0, s, bits, sc, wx, m, vcx, vcy,
                        slab, cnt);
     FSR_LAUNCH_CHECK("k_slab_rows");
     FSR_TRY(scan_cells(ctx, cnt, nvc, cell_off, chunk_off, chunk_cell, max_chunks,
                        &counters->num_chunks, s));
-    if (materialize) {
-        FSR_TRY(scan_exclusive(ctx, SCAN_U32, slab, slab_off, nslabs, nullptr, nullptr, s));
-        hipLaunchKernelGGL(k_slab_fill, dim3((uint32_t)((nslabs + 255) / 256)), dim3(256), 0, s,
-                           bits, sc, wx, m, vcx, vcy, (const uint32_t*)slab,
-                           (const uint32_t*)slab_off, cell_band, V, nslabs);
-        FSR_LAUNCH_CHECK("k_slab_fill");
-    }
     out->cell_off = cell_off;
     out->cell_cnt = cnt;
     out->chunk_off = chunk_off;
-    out->cell_band = materialize ? cell_band : nullptr;
     out->chunk_cell = chunk_cell;
     out->bits = bits;
     out->wx = wx;

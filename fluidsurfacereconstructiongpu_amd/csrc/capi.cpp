@@ -330,10 +330,7 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
     ba.all_exceptions = sa.all_exceptions;
     FSR_TRY(band_build(ctx, ba, s));
     BandCompactOut bc;
-    // the cell-major list itself is needed by the anisotropic field and the
-    // adjoint; the ZB05 field lists its chunks from the mask
-    const bool materialize = yu13 || ctx->save_adjoint;
-    FSR_TRY(band_compact(ctx, bits, sc, sp, yu13 ? 2 : 1, counters, stats, &bc, s, materialize));
+    FSR_TRY(band_compact(ctx, bits, sc, sp, yu13 ? 2 : 1, counters, stats, &bc, s));
 
     // 4. field
     // (the dense grid was filled in the frame's first launch)
@@ -382,9 +379,13 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
         fa.phi = phi;
         fa.counters = counters;
         fa.saved = nullptr;
+        fa.cell_band = nullptr;
         fa.work = nullptr;
         fa.num_particles = n;
-        if (ctx->save_adjoint) FSR_TRY(arena_typed(ctx, A_ADJ_VERT, V, &fa.saved));
+        if (ctx->save_adjoint) {
+            FSR_TRY(arena_typed(ctx, A_ADJ_VERT, V, &fa.saved));
+            FSR_TRY(arena_typed(ctx, A_CELL_BAND, V, &fa.cell_band));
+        }
         FSR_TRY(field_zb05(ctx, fa, s));
     }
 
@@ -441,6 +442,7 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
         st.perm = ho.perm;
         st.bc = bc;
         st.saved = static_cast<const float4*>(ctx->arena.ptr[A_ADJ_VERT]);
+        st.cell_band = static_cast<const uint32_t*>(ctx->arena.ptr[A_CELL_BAND]);
         st.phi = phi;
         st.bits = bits;
         st.word_off = static_cast<const uint32_t*>(ctx->arena.ptr[A_WORD_OFF]);

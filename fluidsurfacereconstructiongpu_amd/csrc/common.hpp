@@ -170,6 +170,13 @@ __device__ __forceinline__ void wave_range(bool live, float v, float* lo, float*
     *hi = __int_as_float(float_order(wave_max_i(live ? k : small)));
 }
 
+// Orders a wave's LDS accesses before and after it among the wave's lanes.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Band bits of one mask word (vertices 32 w .. 32 w + 31 of a row) restricted
 // to the vertex range [xlo, xhi).
 __device__ __forceinline__ uint32_t clip_word(uint32_t word, uint32_t w, uint32_t xlo,
@@ -369,11 +376,9 @@ enum ArenaSlot {
 // Band vertices grouped by hash cell (band.hip).
 struct BandCompactOut {
     uint32_t* band_index;   // u32[B]
-    uint32_t* cell_off;     // per virtual cell offset into cell_band
+    uint32_t* cell_off;     // per virtual cell: its first slot in cell-major order
     uint32_t* cell_cnt;
     uint32_t* chunk_off;
-    uint32_t* cell_band;    // u32[B] cell-major, or null when not materialised:
-                            // then a chunk's vertices are read from the mask
     uint32_t* chunk_cell;   // chunk -> virtual cell
     uint32_t vcx, vcy, vcz; // virtual cell grid (hash grid padded by `radius`)
     int radius;             // 1 (3^3 blocks) or 2 (5^3 blocks)
@@ -431,6 +436,7 @@ struct AdjointState {
     const uint32_t* perm = nullptr;          // sorted -> caller index
     BandCompactOut bc{};
     const float4* saved = nullptr;           // cell-major (x - xbar, sum w)
+    const uint32_t* cell_band = nullptr;     // vertex at each cell-major slot
     const float* phi = nullptr;
     const uint32_t* bits = nullptr;          // band mask
     const uint32_t* word_off = nullptr;      // band rank of each mask word
@@ -602,12 +608,10 @@ fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s);
 // the particle, so the band equals a box dilation of the surface cells.
 int band_dilation_exact(const fsr_grid_info& sc, float h);
 
-// materialize: also write the cell-major list (cell_band); otherwise the
-// field kernel lists each chunk's vertices from the mask.
+// The work list of the field kernels, which list each chunk's vertices from the mask.
 fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& sc,
                         const GridDev& sp, int radius, Counters* counters,
-                        fsr_frame_stats* st, BandCompactOut* out, hipStream_t s,
-                        bool materialize = true);
+                        fsr_frame_stats* st, BandCompactOut* out, hipStream_t s);
 
 // field_zb05.hip ------------------------------------------------------------
 struct FieldArgs {
@@ -621,6 +625,7 @@ struct FieldArgs {
     float* phi;
     Counters* counters;
     float4* saved;         // optional, cell-major [B]: (x - xbar, sum w) for the adjoint
+    uint32_t* cell_band;   // with saved: the vertex at each cell-major slot
     uint32_t* work;        // set by field_zb05: per chunk, candidates staged, candidates
                            // kept by the box test, 16 x 16 tile steps evaluated
     uint32_t num_particles;

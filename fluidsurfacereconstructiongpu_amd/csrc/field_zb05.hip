@@ -39,6 +39,7 @@
 // culling leaves every sum unchanged.
 #include <type_traits>
 
+#include "chunk_list.hpp"
 #include "common.hpp"
 
 namespace fsr {
@@ -49,12 +50,6 @@ constexpr int kFieldThreads = 256;
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) {
     return v < lo ? lo : (v > hi ? hi : v);
-}
-
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Lane exchange i <-> i ^ m within each half-wave (m < 32), with no address
@@ -104,72 +99,6 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv& f) {
 struct VertexDiv {
     FastDiv rx, rxy;
 };
-
-// The vertex ids of chunk k of virtual cell v, listed from the band mask in
-// the cell-major order (layer z, row y, then x ascending), when the cell-major
-// list is not materialised: lane l < cnt receives the (64 k + l)-th band vertex
-// of the cell.  The cell's layers (slabs) are consecutive in the slab counts;
-// 64 layers at a time, those that overlap [64 k, 64 k + 64) are expanded word
-// by word, each lane taking one (layer, row, word) of them, and the wanted
-// ranks go to `scratch` (64 LDS words of the wave).
-__device__ uint32_t chunk_vertex(const BandCompactOut& bc, uint32_t rx, uint32_t ry, uint32_t v,
-                                 uint32_t k, uint32_t cnt, uint32_t* scratch) {
-    const uint32_t lane = __lane_id();
-    const uint32_t cxv = v % bc.vcx, cyv = (v / bc.vcx) % bc.vcy, czv = v / (bc.vcx * bc.vcy);
-    const uint32_t* lo_x = bc.axis;
-    const uint32_t* lo_y = lo_x + 2u * bc.vcx;
-    const uint32_t* lo_z = lo_y + 2u * bc.vcy;
-    const uint32_t zlo = lo_z[czv], nz = lo_z[bc.vcz + czv] - zlo;
-    const uint64_t sbase = (uint64_t)bc.vcx * bc.vcy * zlo + ((uint64_t)cyv * bc.vcx + cxv) * nz;
-    const uint32_t ylo = lo_y[cyv], ny = lo_y[bc.vcy + cyv] - ylo;
-    const uint32_t xlo = lo_x[cxv], xhi = lo_x[bc.vcx + cxv];
-    const uint32_t w0 = xlo >> 5, nw = ((xhi + 31u) >> 5) - w0;
-    const uint32_t per = ny * nw;
-    const uint32_t lo = 64u * k, hi = lo + 64u;
-    // every slot starts empty, so a slot the expansion does not fill reads as
-    // "no vertex" rather than as a stale id
-    scratch[lane] = 0xFFFFFFFFu;
-    wave_lds_sync();
-    uint32_t before = 0;  // band vertices of the cell's layers before the group
-    for (uint32_t g0 = 0; g0 < nz && before < hi; g0 += 64u) {
-        const uint32_t sn = g0 + lane < nz ? bc.slab[sbase + g0 + lane] : 0u;
-        const uint32_t sincl = before + wave_inclusive_sum(sn);
-        const uint32_t sexcl = sincl - sn;
-        const uint64_t hit = __ballot(g0 + lane < nz && sn != 0u && sexcl < hi && sincl > lo);
-        if (hit) {
-            // the overlapping layers of the group are consecutive: j0 .. j1
-            const uint32_t j0 = (uint32_t)__builtin_ctzll(hit);
-            const uint32_t j1 = 63u - (uint32_t)__builtin_clzll(hit);
-            const uint32_t items = (j1 - j0 + 1u) * per;
-            uint32_t rank0 = (uint32_t)__builtin_amdgcn_readlane((int)sexcl, (int)j0);
-            for (uint32_t i0 = 0; i0 < items; i0 += 64u) {
-                const uint32_t i = i0 + lane;
-                uint32_t word = 0, base = 0;
-                if (i < items) {
-                    const uint32_t js = g0 + j0 + i / per, rem = i % per;
-                    const uint32_t y = ylo + rem / nw, w = w0 + rem % nw;
-                    const uint64_t row = (uint64_t)(zlo + js) * ry + y;
-                    word = clip_word(bc.bits[row * bc.wx + w], w, xlo, xhi);
-                    base = (uint32_t)(row * rx) + w * 32u;
-                }
-                const uint32_t c = (uint32_t)__popc(word);
-                const uint32_t incl = wave_inclusive_sum(c);
-                uint32_t r = rank0 + incl - c;
-                while (word) {
-                    if (r >= lo && r < hi) scratch[r - lo] = base + (uint32_t)__builtin_ctz(word);
-                    ++r;
-                    word &= word - 1u;
-                }
-                rank0 += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-            }
-        }
-        before = (uint32_t)__builtin_amdgcn_readlane((int)sincl, 63);
-    }
-    wave_lds_sync();
-    const uint32_t id = lane < cnt ? scratch[lane] : 0xFFFFFFFFu;
-    wave_lds_sync();
-    return id;
-}
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -272,8 +201,7 @@ struct Chunk {
     }
 };
 
-// Loads chunk ch: its vertices (listed through `scratch`, 64 words of LDS, when
-// the cell-major list is not materialised), their operands into vt (rows of 64:
+// Loads chunk ch: its vertices (listed through `scratch`, 64 words of LDS), their operands into vt (rows of 64:
 // x', y', z', a_x, a_y, a_z, c_x), their box, and the candidate rows.
 __device__ __forceinline__ Chunk load_chunk(const FieldArgs& a, const BandCompactOut& bc,
                                             const VertexDiv& vd, uint32_t ch, float inv_r2,
@@ -291,12 +219,7 @@ __device__ __forceinline__ Chunk load_chunk(const FieldArgs& a, const BandCompac
     c.cnt = min(64u, ccount - 64u * k);
     // the chunk's vertex ids (before the candidate rows, whose registers live
     // through the staging loop)
-    c.vid = 0;
-    if (bc.cell_band) {
-        if (lane < c.cnt) c.vid = bc.cell_band[c.first + lane];
-    } else {
-        c.vid = chunk_vertex(bc, a.sc.rx, a.sc.ry, v, k, c.cnt, scratch);
-    }
+    c.vid = chunk_vertex(bc, a.sc.rx, a.sc.ry, v, k, c.cnt, scratch);
 
     // candidate rows of the clamped 3^3 block
     const int x0 = clampi(cx - 1, 0, a.sp.rx - 1), x1 = clampi(cx + 1, 0, a.sp.rx - 1);
@@ -373,8 +296,11 @@ __device__ __forceinline__ void store_vertex(const FieldArgs& a, const Chunk& c,
                        a.particle_radius;
         keep_out = make_float4(dx, dy, dz, sw);
     }
-    // for the adjoint: x - xbar and sum w, at the vertex's cell-major slot
-    if (a.saved) a.saved[c.first + lane] = keep_out;
+    // for the adjoint: x - xbar and sum w, and the vertex, at its cell-major slot
+    if (a.saved) {
+        a.saved[c.first + lane] = keep_out;
+        a.cell_band[c.first + lane] = c.vid;
+    }
 }
 
 // One LDS block per wave, so every per-lane LDS address is one base register

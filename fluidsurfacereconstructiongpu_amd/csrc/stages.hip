@@ -589,6 +589,7 @@ fsr_status fsr_update_scalar_grid_values_compacted(
     fa.phi = scalar_field;
     fa.counters = ct;
     fa.saved = nullptr;
+    fa.cell_band = nullptr;
     fa.work = nullptr;
     fa.num_particles = num_particles;
     return field_zb05(ctx, fa, s);

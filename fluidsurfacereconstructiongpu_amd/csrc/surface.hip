@@ -270,12 +270,6 @@ __global__ __launch_bounds__(256) void k_colorfield_tail(SurfaceArgs a, float ma
     block_count_add2(&a.st->num_surface_particles, n_surf, &a.st->band_exceptions, n_exc);
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct ColorChunks {
     const uint32_t* chunk_cell;
     const uint32_t* chunk_off;
