@@ -118,43 +118,82 @@ __device__ __forceinline__ uint32_t dilate_x_word(const uint8_t* __restrict__ in
 }
 
 // The three dilation passes in one launch: a workgroup owns a tile of kTW
-// words x kTY rows x kTZ layers of the output; it x-dilates the tile's input
+// words x kTYZ rows x kTYZ layers of the output; it x-dilates the tile's input
 // with a halo of 3 rows and 3 layers on each side into LDS (from the byte
 // mask), ORs the 7 rows (y), then the 7 layers (z), and writes the tile.
 // Rows and layers outside the grid contribute nothing, as in the separate
-// passes.  1024 threads per tile: a thread loads the tile's 3,872 input
-// words in 4 rounds rather than 16, each round waiting for its loads.
-constexpr int kTW = 8, kTY = 16, kTZ = 16, kH = 3;
-constexpr int kDilateThreads = 1024;
-__global__ __launch_bounds__(kDilateThreads) void k_dilate_box(const uint8_t* __restrict__ in,
-                                                    uint32_t* __restrict__ out, uint32_t wx,
-                                                    GridDev sc) {
-    __shared__ uint32_t xs[kTZ + 2 * kH][kTY + 2 * kH][kTW];
-    __shared__ uint32_t ys[kTZ + 2 * kH][kTY][kTW];
+// passes.  The forms, by the number of 8-word x 16 x 16 tiles:
+//   * at least one per CU: that tile, 1024 threads, kMap.  Reading the seeds
+//     bounds it (the halo nearly doubles their V bytes), and most of a grid has
+//     no seed near: only words that the seeds' map marks are read, and a tile
+//     without one is just cleared.  27 -> 14 us at 320^3, 42 -> 19 at 384^3, 9.2
+//     -> 8.3 at 256^3 (dam breaks).
+//   * fewer: the same tile without the map, whose load would be one more in the
+//     chain that a tile takes: at 192^3 7.8 us, 8.7 with the map.
+//   * fewer than half a tile per CU: 4 words x 8 x 8, 512 threads, which leaves
+//     fewer CUs idle and takes 2 rounds of loads for 4: 7.9 -> 4.4 us at 128^3,
+//     7.5 -> 6.1 at 161^3 (at 192^3 9.2, hence the line).
+constexpr int kH = 3;
+template <int kTW, int kTYZ, int kThreads, bool kMap>
+__global__ __launch_bounds__(kThreads) void k_dilate_box(const uint8_t* __restrict__ in,
+                                                         uint32_t* __restrict__ out, uint32_t wx,
+                                                         GridDev sc) {
+    constexpr int kIn = kTYZ + 2 * kH;
+    __shared__ uint32_t xs[kIn][kIn][kTW];
+    __shared__ uint32_t ys[kIn][kTYZ][kTW];
     const uint32_t w0 = blockIdx.x * kTW;
-    const int y0 = (int)(blockIdx.y * kTY), z0 = (int)(blockIdx.z * kTZ);
-    constexpr int nxs = (kTZ + 2 * kH) * (kTY + 2 * kH) * kTW;
-    for (int t = threadIdx.x; t < nxs; t += blockDim.x) {
+    const int y0 = (int)(blockIdx.y * kTYZ), z0 = (int)(blockIdx.z * kTYZ);
+    constexpr int nxs = kIn * kIn * kTW;
+    constexpr int kRounds = (nxs + kThreads - 1) / kThreads;
+    const uint8_t* map = in + seed_map_offset(sc);
+    // the map entries of the thread's words, loaded together
+    bool seeded[kRounds];
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k) {
+        const int t = (int)threadIdx.x + k * kThreads;
         const int w = t % kTW, r = t / kTW;
-        const int yy = y0 - kH + r % (kTY + 2 * kH), zz = z0 - kH + r / (kTY + 2 * kH);
-        uint32_t v = 0;
-        if (w0 + w < wx && yy >= 0 && yy < (int)sc.ry && zz >= 0 && zz < (int)sc.rz)
-            v = dilate_x_word(in, (((uint64_t)zz * sc.ry + yy) * wx) << 5, w0 + w, wx, sc.rx);
-        xs[r / (kTY + 2 * kH)][r % (kTY + 2 * kH)][w] = v;
+        const int yy = y0 - kH + r % kIn, zz = z0 - kH + r / kIn;
+        seeded[k] = t < nxs && w0 + w < wx && yy >= 0 && yy < (int)sc.ry && zz >= 0 &&
+                    zz < (int)sc.rz &&
+                    (!kMap || map[seed_map_index(sc, w0 + w, yy, zz)] != 0);
     }
-    __syncthreads();
-    constexpr int nys = (kTZ + 2 * kH) * kTY * kTW;
-    for (int t = threadIdx.x; t < nys; t += blockDim.x) {
-        const int w = t % kTW, y = (t / kTW) % kTY, zr = t / (kTW * kTY);
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k) {
+        const int t = (int)threadIdx.x + k * kThreads;
+        const int w = t % kTW, r = t / kTW;
+        const int yy = y0 - kH + r % kIn, zz = z0 - kH + r / kIn;
+        uint32_t v = 0;
+        if (seeded[k])
+            v = dilate_x_word(in, (((uint64_t)zz * sc.ry + yy) * wx) << 5, w0 + w, wx, sc.rx);
+        if (t < nxs) xs[r / kIn][r % kIn][w] = v;
+        any |= seeded[k];
+    }
+    constexpr int nout = kTYZ * kTYZ * kTW;
+    if (kMap) {
+        if (!__syncthreads_or(any)) {
+            // no seed near the tile
+            for (int t = threadIdx.x; t < nout; t += kThreads) {
+                const int w = t % kTW, yy = y0 + (t / kTW) % kTYZ, zz = z0 + t / (kTW * kTYZ);
+                if (w0 + w < wx && yy < (int)sc.ry && zz < (int)sc.rz)
+                    out[((uint64_t)zz * sc.ry + yy) * wx + w0 + w] = 0u;
+            }
+            return;
+        }
+    } else {
+        __syncthreads();
+    }
+    constexpr int nys = kIn * kTYZ * kTW;
+    for (int t = threadIdx.x; t < nys; t += kThreads) {
+        const int w = t % kTW, y = (t / kTW) % kTYZ, zr = t / (kTW * kTYZ);
         uint32_t v = 0;
 #pragma unroll
         for (int d = 0; d <= 2 * kH; ++d) v |= xs[zr][y + d][w];
         ys[zr][y][w] = v;
     }
     __syncthreads();
-    constexpr int nout = kTZ * kTY * kTW;
-    for (int t = threadIdx.x; t < nout; t += blockDim.x) {
-        const int w = t % kTW, y = (t / kTW) % kTY, z = t / (kTW * kTY);
+    for (int t = threadIdx.x; t < nout; t += kThreads) {
+        const int w = t % kTW, y = (t / kTW) % kTYZ, z = t / (kTW * kTYZ);
         const int yy = y0 + y, zz = z0 + z;
         if (w0 + w >= wx || yy >= (int)sc.ry || zz >= (int)sc.rz) continue;
         uint32_t v = 0;
@@ -674,12 +713,20 @@ fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s) {
     // S (bytes) -> tmp (x), tmp -> S (y, its first nwords words), S -> bits
     // (z); `sbits` is consumed
     uint32_t* sb = const_cast<uint32_t*>(a.sbits);
-    const dim3 tiles((wx + kTW - 1) / kTW, (a.sc.ry + kTY - 1) / kTY, (a.sc.rz + kTZ - 1) / kTZ);
+    auto tiles = [&](uint32_t tw, uint32_t tyz) {
+        return dim3((wx + tw - 1) / tw, (a.sc.ry + tyz - 1) / tyz, (a.sc.rz + tyz - 1) / tyz);
+    };
+    const dim3 big = tiles(8, 16), small = tiles(4, 8);
     if (a.all_exceptions) {
         // no seeds: the exact path alone sets bits of the mask the caller cleared
-    } else if (tiles.y <= 65535u && tiles.z <= 65535u) {
-        hipLaunchKernelGGL(k_dilate_box, tiles, dim3(kDilateThreads), 0, s, (const uint8_t*)sb, a.bits, wx,
-                           a.sc);
+    } else if (big.y <= 65535u && big.z <= 65535u) {
+        const uint64_t n = (uint64_t)big.x * big.y * big.z, cus = (uint64_t)ctx->num_cus;
+        const bool fine = 2 * n < cus;
+        auto dilate = fine ? k_dilate_box<4, 8, 512, false>
+                           : (n < cus ? k_dilate_box<8, 16, 1024, false>
+                                      : k_dilate_box<8, 16, 1024, true>);
+        hipLaunchKernelGGL(dilate, fine ? small : big, dim3(fine ? 512 : 1024), 0, s,
+                           (const uint8_t*)sb, a.bits, wx, a.sc);
         FSR_LAUNCH_CHECK("k_dilate_box");
     } else {
         hipLaunchKernelGGL(k_dilate_x, dim3(blocks), dim3(256), 0, s, (const uint8_t*)sb, a.tmp,

@@ -259,7 +259,7 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
     FSR_TRY(arena_typed(ctx, A_COUNTERS, 1, &counters));
     uint32_t *flags, *sbits, *tmp, *bits, *exc;
     FSR_TRY(arena_typed(ctx, A_SURF_FLAGS, n, &flags));
-    FSR_TRY(arena_typed(ctx, A_SBITS, 8ull * W, &sbits));  // byte seed mask
+    FSR_TRY(arena_typed(ctx, A_SBITS, seed_words(sc), &sbits));
     FSR_TRY(arena_typed(ctx, A_BAND_TMP, W, &tmp));
     FSR_TRY(arena_typed(ctx, A_BAND_BITS, W, &bits));
     FSR_TRY(arena_typed(ctx, A_EXCEPTIONS, n, &exc));
@@ -273,7 +273,7 @@ fsr_status frame_impl(const char* who, fsr_context* ctx, fsr_method method,
     if (all_exceptions)
         fills.add(bits, 0u, W);
     else
-        fills.add(sbits, 0u, 8ull * W);
+        fills.add(sbits, 0u, seed_words(sc));
     // the dense field outside the band keeps the fill: 0, or the byte 100 for
     // Yu13 (the reference's memset of the Yu13 grid)
     fills.add(phi, yu13 ? 0x64646464u : 0u, V);

@@ -553,6 +553,21 @@ fsr_status spatial_hash(fsr_context* ctx, float* pos, float* dens, uint32_t n,
                         const fsr_grid_info& sp, fsr_frame_stats* st,
                         HashOut* out, hipStream_t s, const FillList* pre = nullptr);
 
+// Band seeds: a byte mask, one byte per scalar cell with rows padded to whole
+// words of the band mask (32 bytes per word), followed by the map of its touched
+// parts, one byte per mask word and 4 rows x 4 layers: set when the x-dilated
+// word of one of those rows can be nonzero.
+__host__ __device__ inline uint64_t seed_map_offset(const GridDev& sc) {   // in bytes
+    return ((uint64_t)row_words(sc.rx) * sc.ry * sc.rz) << 5;
+}
+__host__ __device__ inline uint64_t seed_map_index(const GridDev& sc, uint32_t word, uint32_t y, uint32_t z) {
+    return ((uint64_t)(z >> 2) * ((sc.ry + 3u) >> 2) + (y >> 2)) * row_words(sc.rx) + word;
+}
+inline uint64_t seed_words(const GridDev& sc) {
+    const uint64_t map = (uint64_t)row_words(sc.rx) * ((sc.ry + 3u) >> 2) * ((sc.rz + 3u) >> 2);
+    return seed_map_offset(sc) / 4 + (map + 3) / 4;
+}
+
 // surface.hip ---------------------------------------------------------------
 struct SurfaceArgs {
     const float4* sorted;
@@ -564,9 +579,8 @@ struct SurfaceArgs {
     GridDev sc;
     float h;
     uint32_t* flags;        // u32[N] surface flags (sorted order)
-    uint32_t* sbits;        // seed mask: one byte per scalar cell of the surface
-                            // particles, rows padded to whole band-mask words
-                            // (32 bytes per word, 8 words of storage each)
+    uint32_t* sbits;        // seed mask and map (seed_words), of the scalar cells of
+                            // the surface particles
     uint32_t* exceptions;   // particles routed to the exact band path
     Counters* counters;
     fsr_frame_stats* st;

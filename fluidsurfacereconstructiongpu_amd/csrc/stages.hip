@@ -473,7 +473,7 @@ fsr_status fsr_estimation_of_surface_vertices(fsr_context* ctx, const fsr_sim_pa
     uint32_t *sbits, *tmp, *bits, *exc;
     float4* p4;
     const uint64_t nn = num_particles ? num_particles : 1;
-    FSR_TRY(arena_typed(ctx, A_SBITS, 8ull * W, &sbits));  // byte seed mask
+    FSR_TRY(arena_typed(ctx, A_SBITS, seed_words(g), &sbits));
     FSR_TRY(arena_typed(ctx, A_BAND_TMP, W, &tmp));
     FSR_TRY(arena_typed(ctx, A_BAND_BITS, W, &bits));
     FSR_TRY(arena_typed(ctx, A_EXCEPTIONS, nn, &exc));
@@ -482,7 +482,7 @@ fsr_status fsr_estimation_of_surface_vertices(fsr_context* ctx, const fsr_sim_pa
     if (all_exceptions)
         FSR_TRY(fill_u32(bits, 0u, W, s));
     else
-        FSR_TRY(fill_u32(sbits, 0u, 8ull * W, s));
+        FSR_TRY(fill_u32(sbits, 0u, seed_words(g), s));
     if (num_particles) {
         hipLaunchKernelGGL(k_pack_f4, dim3(blocks_for(num_particles)), dim3(256), 0, s, particles,
                            (const float*)nullptr, num_particles, p4);

@@ -144,7 +144,13 @@ __device__ __forceinline__ bool seed_particle(const SurfaceArgs& a, uint32_t i, 
         // byte store (every writer stores 1), no read-modify-write
         const uint32_t ix = (uint32_t)(int)qx, iy = (uint32_t)(int)qy, iz = (uint32_t)(int)qz;
         const uint32_t wx = row_words(a.sc.rx);
-        reinterpret_cast<uint8_t*>(a.sbits)[(((uint64_t)iz * a.sc.ry + iy) * wx << 5) + ix] = 1u;
+        uint8_t* seeds = reinterpret_cast<uint8_t*>(a.sbits);
+        seeds[(((uint64_t)iz * a.sc.ry + iy) * wx << 5) + ix] = 1u;
+        // and in the map, the words that its x dilation [ix - 3, ix + 2] meets
+        uint8_t* map = seeds + seed_map_offset(a.sc) + seed_map_index(a.sc, 0, iy, iz);
+        const uint32_t w0 = (ix < 3u ? 0u : ix - 3u) >> 5, w1 = min((ix + 2u) >> 5, wx - 1u);
+        map[w0] = 1u;
+        if (w1 != w0) map[w1] = 1u;
     }
     const uint64_t m = __ballot(exc);
     if (m) {
