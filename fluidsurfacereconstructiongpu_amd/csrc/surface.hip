@@ -21,6 +21,7 @@
 // is not exact for it, it is appended to an exception list that band.hip
 // treats with the reference's per-particle box loop.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -285,33 +286,68 @@ struct ColorChunks {
 };
 
 // The colour-field test of the particles of the hash cells, a wave per chunk of
-// up to 64 particles of one cell: the 9 x-runs of the cell's 3^3 block are
-// staged through LDS and read as broadcasts.  Candidates farther than
-// h * (1 + 5e-5) from the bounding box of the chunk's particles can only add to
-// the neighbour count (d^2 > 0, dist >= h): they are counted and dropped, the
-// others are compacted in order and evaluated with the per-thread kernel's
-// arithmetic, so counts, gradients and flags are identical to it.  Both take
-// the reference's test |r| < h as |r|^2 < h^2 and the distance as
-// |r|^2 rsqrt(|r|^2), one reciprocal square root per pair within h and no
-// square root: the distance enters the gradient through (1 - |r|/h)^2, which
-// vanishes where the two forms of the test could differ.
-template <bool kSmall>
-__global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, ColorChunks cl) {
-    __shared__ float4 queue[4][128];
+// up to 64 particles of one cell, a lane per particle; each lane sums its
+// candidates in their order (x-runs of the cell's 3^3 block), with the arithmetic
+// of the kernel above.  Both take the reference's test |r| < h as |r|^2 < h^2 and
+// the distance as |r|^2 rsqrt(|r|^2), one reciprocal square root per pair within
+// h and no square root: the distance enters the gradient through (1 - |r|/h)^2,
+// which vanishes where the two forms of the test could differ.
+//
+// VALU-bound: a candidate costs the wave some 20 operations, whichever lanes it
+// is within h of (about one in five).  So
+//   * the chunk's lanes form two groups, the halves of its box along x, each with a
+//     queue of its own in LDS.  A candidate enters the queues of the groups whose
+//     box it is within h * (1 + 5e-5) of, and a lane reads its group's: the wave
+//     makes as many steps as the longer queue needs, four fifths of those for one
+//     box around a full cell.  Along x, the order within a run, the queues fill
+//     most evenly.  (Quarters, in x and y, need two thirds of the steps, but twice
+//     the tests, and rings that fill less evenly: 441 us against 398 for the 1M
+//     frame below);
+//   * the count of neighbours (d^2 > 0), which decides for particles with fewer
+//     than 25, is that of the block less those at distance 0, which lie in the
+//     particle's own cell: it is not looked at when the other cells hold 25.  And
+//     only queue parts that can hold own-cell candidates test for distance 0 (the
+//     particle itself): particles of different cells differ in a coordinate (the
+//     host checks that the square of the least difference does not underflow);
+//   * four candidates are loaded together; in smaller frames (kSmall), where a SIMD
+//     has few waves to change to, their terms are formed side by side with no
+//     branch between them, a pair that is not within h weighing 0.
+// Akinci12 frames, before (one group, counting every pair) and now: 1M-particle
+// dam break 472 -> 383 us, 150k particles 179 -> 141, 16k 126 -> 66.
+//
+// A queue is a ring of kColorRing entries.  When a ring holds more than kColorRing
+// - 64, steps are made for both groups at once, as many as the shorter queue holds,
+// or as many more as the next staging round needs; a lane whose ring has fewer
+// idles.  Heads stay multiples of 4 (the last step's 4 are padded with entries out
+// of reach).
+constexpr uint32_t kColorRing = 128;
+constexpr uint32_t kOgt = 2, kOlt = 4;  // ordered > and <, as the compare builtin numbers them
+
+template <bool kSmall, bool kRadius>
+__global__ __launch_bounds__(256, kSmall ? 6 : 8) void k_colorfield(SurfaceArgs a, float mass,
+                                                                    ColorChunks cl,
+                                                                    int own_zero_only) {
+    constexpr int G = 2;
+    // a group's ring starts 4 banks after the one before
+    __shared__ float4 queue[4][G][kColorRing + 1];
     __shared__ FetchState fetch;
     fetch_init(&fetch);
     const uint32_t lane = __lane_id();
     const uint32_t wave = threadIdx.x >> 6;
-    float4* q = queue[wave];
     const uint32_t nch = *cl.num_chunks;
+    if (kSmall) {
+        // entries that no group's candidate was put in are multiplied by 0 there
+        for (uint32_t t = lane; t < (uint32_t)G * (kColorRing + 1u); t += 64u)
+            (&queue[wave][0][0])[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     const float h = a.h;
     const float inv_h = 1.0f / h;
     const float gcoef = -45.0f / (3.14159265358979f * (h * h) * (h * h));
     const float cull2 = (h * h) * 1.0001f;
     const float h2 = h * h;
+    constexpr float kFar = 3.0e38f;  // a coordinate out of reach: its distance is infinite
     uint32_t n_surf = 0, n_exc = 0;
-    // work of this wave: candidates staged and kept (wave-uniform), and this
-    // lane's pairs within h
+    // work of this wave: candidates staged, kept for a group, and pairs within h
     uint32_t n_staged = 0, n_kept = 0, n_inh = 0;
     ItemFetch<4, kSmall> items(cl.next, nch, &fetch);
     for (;;) {
@@ -370,31 +406,98 @@ __global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, C
             }
             return off;
         };
-        float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
+        // the candidate indices of the own cell's particles
+        const uint32_t oj = (uint32_t)((cz - z0) * ny + (cy - y0));
+        const uint32_t own_first = own.start - (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)oj);
+        const uint32_t own_n = own.end - own.start;
+        const bool need_count = kRadius || !own_zero_only || total - own_n < 25u;
+
+        float4 p = make_float4(-kFar, -kFar, -kFar, 0.f);
         if (live) p = a.sorted[i];
-        float bx0, bx1, by0, by1, bz0, bz1;
+        float bx0, bx1;
         wave_range(live, p.x, &bx0, &bx1);
-        wave_range(live, p.y, &by0, &by1);
-        wave_range(live, p.z, &bz0, &bz1);
-        uint32_t count = 0, count_r = 0, kept = 0, fill = 0;
+        const uint32_t grp = p.x > 0.5f * (bx0 + bx1) ? 1u : 0u;
+        // the groups' boxes; an empty one is out of reach
+        float lo[G][3], hi[G][3];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const bool in = live && grp == (uint32_t)g;
+            wave_range(in, p.x, &lo[g][0], &hi[g][0]);
+            wave_range(in, p.y, &lo[g][1], &hi[g][1]);
+            wave_range(in, p.z, &lo[g][2], &hi[g][2]);
+            if (!__ballot(in)) lo[g][0] = hi[g][0] = kFar;
+        }
+        // rings: entries [head, head + fill) of each wait for evaluation
+        uint32_t head[G], fill[G], done[G], put[G], mark[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) head[g] = fill[g] = done[g] = put[g] = mark[g] = 0;
+        uint32_t zeros = 0, count_r = 0;
         float gx = 0.f, gy = 0.f, gz = 0.f;
-        auto run = [&](uint32_t n) {
-            for (uint32_t t = 0; t < n; ++t) {
-                const float4 qq = q[t];
-                const float rx = p.x - qq.x, ry = p.y - qq.y, rz = p.z - qq.z;
-                const float d2 = __builtin_fmaf(rz, rz, __builtin_fmaf(ry, ry, rx * rx));
-                if (d2 > 0.0f) {
-                    ++count;
-                    if (d2 < h2) {
-                        ++count_r;
-                        const float ri = __builtin_amdgcn_rsqf(d2);
-                        const float x = 1.0f - d2 * ri * inv_h;
-                        const float cc = qq.w * x * x * ri;
-                        gx = __builtin_fmaf(cc, rx, gx);
-                        gy = __builtin_fmaf(cc, ry, gy);
-                        gz = __builtin_fmaf(cc, rz, gz);
+        const char* ring = reinterpret_cast<const char*>(&queue[wave][grp][0]);
+        auto by_group = [&](const uint32_t (&v)[G]) { return grp ? v[1] : v[0]; };
+        // the next mine candidates of the lane's ring (a multiple of 4, at most n)
+        auto steps = [&](auto zt, uint32_t n, uint32_t mine, uint32_t at) {
+            constexpr bool kZero = decltype(zt)::value;
+            for (uint32_t t = 0; t < n; t += 4u) {
+                const uint64_t act = __ballot(t < mine);
+                const float4* e =
+                    reinterpret_cast<const float4*>(ring + ((16u * (at + t)) & (16u * kColorRing - 1u)));
+                float rx[4], ry[4], rz[4], d2[4];
+                float4 qq[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) qq[u] = e[u];
+                // whole entries, all four before the first is used
+                asm volatile("" : "+v"(qq[0].w), "+v"(qq[1].w), "+v"(qq[2].w), "+v"(qq[3].w));
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    rx[u] = p.x - qq[u].x;
+                    ry[u] = p.y - qq[u].y;
+                    rz[u] = p.z - qq[u].z;
+                    d2[u] = __builtin_fmaf(rz[u], rz[u], __builtin_fmaf(ry[u], ry[u], rx[u] * rx[u]));
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    // lane masks straight from the compares (a ballot of the
+                    // conditions took two more operations per candidate)
+                    uint64_t in = act & __builtin_amdgcn_fcmpf(d2[u], h2, kOlt);
+                    if (kZero) {
+                        const uint64_t apart = __builtin_amdgcn_fcmpf(d2[u], 0.0f, kOgt);
+                        in &= apart;
+                        zeros += __builtin_amdgcn_inverse_ballot_w64(act & ~apart) ? 1u : 0u;
+                    }
+                    n_inh += (uint32_t)__popcll(in);
+                    const bool take = __builtin_amdgcn_inverse_ballot_w64(in);
+                    if (kRadius) count_r += take ? 1u : 0u;
+                    if (kSmall || take) {
+                        const float ri = __builtin_amdgcn_rsqf(d2[u]);
+                        const float x = 1.0f - d2[u] * ri * inv_h;
+                        float cc = qq[u].w * x * x * ri;
+                        if (kSmall) cc = take ? cc : 0.0f;
+                        gx = __builtin_fmaf(cc, rx[u], gx);
+                        gy = __builtin_fmaf(cc, ry[u], gy);
+                        gz = __builtin_fmaf(cc, rz[u], gz);
                     }
                 }
+            }
+        };
+        auto run = [&](uint32_t n) {
+            uint32_t take[G];
+            bool zero = need_count;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                take[g] = min(n, fill[g] & ~3u);
+                zero |= done[g] < mark[g];
+            }
+            const uint32_t mine = by_group(take), at = by_group(head);
+            wave_lds_sync();
+            if (zero) steps(std::true_type{}, n, mine, at);
+            else steps(std::false_type{}, n, mine, at);
+            wave_lds_sync();
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                fill[g] -= take[g];
+                done[g] += take[g];
+                head[g] = (head[g] + take[g]) & (kColorRing - 1u);
             }
         };
         // each lane's candidate is loaded one staging round ahead
@@ -404,53 +507,59 @@ __global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, C
             if (lane < total) next = a.sorted[off + lane];
         }
         for (uint32_t base = 0; base < total; base += 64u) {
-            const uint32_t g = base + lane;
+            const uint32_t g0 = base + lane;
             const float4 cand = next;
             if (base + 64u < total) {
-                const uint32_t off = row_offset(base + 64u, g + 64u);
-                if (g + 64u < total) next = a.sorted[off + g + 64u];
+                const uint32_t off = row_offset(base + 64u, g0 + 64u);
+                if (g0 + 64u < total) next = a.sorted[off + g0 + 64u];
             }
-            bool keep = false;
-            float4 st;
-            if (g < total) {
+            // (m / rho_j) * gcoef, in the per-thread kernel's operation order
+            const float4 st = make_float4(cand.x, cand.y, cand.z, mass / cand.w * gcoef);
+            const bool has_own = base < own_first + own_n && base + 64u > own_first;
+            uint32_t most = 0, least = kColorRing;
+            uint64_t any = 0;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
                 // c - clamp(c, lo, hi): its square equals that of max(lo - c, c - hi, 0)
-                const float dx = cand.x - __builtin_amdgcn_fmed3f(cand.x, bx0, bx1);
-                const float dy = cand.y - __builtin_amdgcn_fmed3f(cand.y, by0, by1);
-                const float dz = cand.z - __builtin_amdgcn_fmed3f(cand.z, bz0, bz1);
-                keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull2;
-                // (m / rho_j) * gcoef, in the per-thread kernel's operation order
-                st = make_float4(cand.x, cand.y, cand.z, mass / cand.w * gcoef);
+                const float dx = cand.x - __builtin_amdgcn_fmed3f(cand.x, lo[g][0], hi[g][0]);
+                const float dy = cand.y - __builtin_amdgcn_fmed3f(cand.y, lo[g][1], hi[g][1]);
+                const float dz = cand.z - __builtin_amdgcn_fmed3f(cand.z, lo[g][2], hi[g][2]);
+                const bool keep =
+                    g0 < total && __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull2;
+                const uint64_t m = __ballot(keep);
+                if (keep) queue[wave][g][(head[g] + fill[g] + mask_rank(m)) & (kColorRing - 1u)] = st;
+                const uint32_t added = (uint32_t)__popcll(m);
+                any |= m;
+                fill[g] += added;
+                put[g] += added;
+                if (has_own) mark[g] = put[g];
+                most = max(most, fill[g]);
+                least = min(least, fill[g]);
             }
-            const uint64_t m = __ballot(keep);
-            if (keep) q[fill + mask_rank(m)] = st;
-            const uint32_t added = (uint32_t)__popcll(m);
-            fill += added;
-            kept += added;
-            if (fill >= 64u) {
-                wave_lds_sync();
-                run(64u);
-                wave_lds_sync();
-                const uint32_t rem = fill - 64u;
-                if (lane < rem) q[lane] = q[64u + lane];
-                wave_lds_sync();
-                fill = rem;
-            }
+            n_kept += (uint32_t)__popcll(any);
+            if (most > kColorRing - 64u)
+                run(max(least & ~3u, (most - (kColorRing - 64u) + 3u) & ~3u));
         }
-        if (fill) {
-            wave_lds_sync();
-            run(fill);
-            wave_lds_sync();
+        // the rest, each ring padded to a multiple of 4 with entries out of reach
+        uint32_t most = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t n = (fill[g] + 3u) & ~3u;
+            if (lane < n - fill[g])
+                queue[wave][g][(head[g] + fill[g] + lane) & (kColorRing - 1u)] =
+                    make_float4(kFar, kFar, kFar, 0.f);
+            fill[g] = n;
+            most = max(most, n);
         }
-        // every dropped candidate has d^2 > 0: it counts as a neighbour
-        count += total - kept;
-        n_inh += count_r;
+        if (most) run(most);
         n_staged += total;
-        n_kept += kept;
         bool surf = false;
         if (live) {
             const float g2 = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
-            // dropped candidates lie beyond h: they never count in count_r
-            surf = a.radius_count ? count_r < 25u : (count < 25u || __builtin_sqrtf(g2) > 3.0f);
+            // candidates that the lane did not see lie beyond h: they count as
+            // neighbours, and never in count_r
+            surf = kRadius ? count_r < 25u
+                           : ((need_count && total - zeros < 25u) || __builtin_sqrtf(g2) > 3.0f);
             a.flags[i] = surf ? 1u : 0u;
         }
         bool exc = false;
@@ -458,12 +567,11 @@ __global__ __launch_bounds__(256) void k_colorfield(SurfaceArgs a, float mass, C
         n_surf += surf ? 1u : 0u;
         n_exc += exc ? 1u : 0u;
     }
-    const uint32_t inh = wave_sum(n_inh);
     if (lane == 0) {
         uint32_t* w = cl.work + 3u * (blockIdx.x * (blockDim.x >> 6) + wave);
         w[0] = n_staged;
         w[1] = n_kept;
-        w[2] = inh;
+        w[2] = n_inh;
     }
     block_count_add2(&a.st->num_surface_particles, n_surf, &a.st->band_exceptions, n_exc);
 }
@@ -555,9 +663,14 @@ fsr_status surface_colorfield(fsr_context* ctx, const SurfaceArgs& a, float mass
     FSR_TRY(reset_xcd(a.counters, s));
     // n / 64 chunks and up to as many remainders: a list that may be shorter than
     // the waves is dealt out (see ItemFetch)
-    auto kernel = a.n / 64u <= 4u * (uint32_t)(blocks / ctx->in_flight) ? k_colorfield<true>
-                                                                         : k_colorfield<false>;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, a, mass, cl);
+    const bool small = a.n / 64u <= 4u * (uint32_t)(blocks / ctx->in_flight);
+    auto kernel = a.radius_count ? (small ? k_colorfield<true, true> : k_colorfield<false, true>)
+                                 : (small ? k_colorfield<true, false> : k_colorfield<false, false>);
+    // Two floats x whose x - min round to either side of a cell boundary B >= cell
+    // have |x| >= ulp(B) / 4 (min is a float), so they are at least cell * 2^-49
+    // apart; the square of that must not underflow.
+    const int own_zero_only = a.sp.cell > 1.0e-5f ? 1 : 0;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s, a, mass, cl, own_zero_only);
     FSR_LAUNCH_CHECK("k_colorfield");
     // particles outside the grid (a device-side count)
     hipLaunchKernelGGL(k_colorfield_tail, dim3(64), dim3(256), 0, s, a, mass);
