@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from .datasets import Frame
-from .reconstructor import Context, Reconstructor, stats_dict
+from .reconstructor import Context, Reconstructor
 
 
 class SurfaceField:
@@ -52,15 +52,13 @@ class SurfaceField:
         work = pos.detach().contiguous().clone()
         dens = self.dens.clone()
         self.rec.launch(self.fr, work, dens, self.cap, sim=self.sim)
-        torch.cuda.synchronize(self.device)
-        st = stats_dict(self.rec._stats)
+        st = self.rec._finish()
         if st["overflow"]:
             self.cap = st["num_mesh_vertices"] + 1024
             work.copy_(pos.detach())
             dens.copy_(self.dens)
             self.rec.launch(self.fr, work, dens, self.cap, sim=self.sim)
-            torch.cuda.synchronize(self.device)
-            st = stats_dict(self.rec._stats)
+            st = self.rec._finish()
         self.stats = st
         self.generation += 1
         V = self.fr.sc.count
