@@ -565,14 +565,13 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
     // particle chunks per hash cell
     const uint64_t max_chunks = (uint64_t)st.n / 64 + C + 1;
     uint32_t* aux;
-    FSR_TRY(arena_typed(ctx, A_ADJ_AUX, 2ull * C + max_chunks, &aux));
-    uint32_t* cnt = aux;
-    uint32_t* chunk_off = aux + C;
-    uint32_t* chunk_cell = aux + 2ull * C;
+    FSR_TRY(arena_typed(ctx, A_ADJ_AUX, C + max_chunks, &aux));
+    uint32_t* chunk_off = aux;
+    uint32_t* chunk_cell = aux + C;
     uint32_t* total = &st.counters->aux[8];
     uint32_t* next = st.counters->xcd_next;
     FSR_TRY(reset_xcd(st.counters, s));
-    FSR_TRY(cell_chunk_list(ctx, st.ranges, nullptr, C, cnt, chunk_off, chunk_cell, total, s));
+    FSR_TRY(cell_chunk_list(ctx, st.ranges, nullptr, C, chunk_off, chunk_cell, max_chunks, total, s));
     FieldBackArgs a;
     a.sorted = st.sorted;
     a.ranges = st.ranges;

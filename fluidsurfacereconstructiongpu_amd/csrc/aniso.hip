@@ -1771,27 +1771,6 @@ __global__ __launch_bounds__(256) void k_cull_radius_to_w(const float4* __restri
     reinterpret_cast<float*>(smooth)[4ull * i + 3] = w;
 }
 
-__global__ __launch_bounds__(256) void k_cell_counts(const fsr_index_range* __restrict__ ranges,
-                                                     const uint32_t* __restrict__ filter,
-                                                     uint32_t C, uint32_t* __restrict__ cnt) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    const fsr_index_range r = ranges[c];
-    uint32_t n = r.start == 0xFFFFFFFFu ? 0u : r.end - r.start;
-    if (filter && filter[c] == 0) n = 0;
-    cnt[c] = n;
-}
-
-__global__ __launch_bounds__(256) void k_chunks_of_cells(const uint32_t* __restrict__ cnt,
-                                                         const uint32_t* __restrict__ chunk_off,
-                                                         uint32_t C, uint32_t* __restrict__ chunk_cell) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    const uint32_t k = (cnt[c] + 63u) >> 6;
-    const uint32_t o = chunk_off[c];
-    for (uint32_t j = 0; j < k; ++j) chunk_cell[o + j] = c;
-}
-
 }  // namespace
 
 // Largest float t with sqrtf(t) <= r (strict: sqrtf(t) < r), sqrtf correctly
@@ -1803,21 +1782,6 @@ float sqrt_bound(float r, bool strict) {
     while (t > 0.0f && !ok(t)) t = std::nextafter(t, 0.0f);
     while (ok(std::nextafter(t, inf))) t = std::nextafter(t, inf);
     return t;
-}
-
-fsr_status cell_chunk_list(fsr_context* ctx, const fsr_index_range* ranges,
-                           const uint32_t* filter, uint32_t C, uint32_t* cnt,
-                           uint32_t* chunk_off, uint32_t* chunk_cell, uint32_t* d_total,
-                           hipStream_t s) {
-    (void)ctx;
-    hipLaunchKernelGGL(k_cell_counts, dim3((C + 255) / 256), dim3(256), 0, s, ranges, filter, C,
-                       cnt);
-    FSR_LAUNCH_CHECK("k_cell_counts");
-    FSR_TRY(scan_exclusive(ctx, SCAN_CHUNKS64, cnt, chunk_off, C, nullptr, d_total, s));
-    hipLaunchKernelGGL(k_chunks_of_cells, dim3((C + 255) / 256), dim3(256), 0, s, cnt, chunk_off,
-                       C, chunk_cell);
-    FSR_LAUNCH_CHECK("k_chunks_of_cells");
-    return FSR_OK;
 }
 
 // Scratch of the two particle passes: per-cell counts and chunk offsets, and
@@ -1833,17 +1797,16 @@ static fsr_status work_section(fsr_context* ctx, WorkSection w, uint32_t** out) 
 }
 
 struct PassScratch {
-    uint32_t *cnt, *chunk_off, *cnt2, *chunk_off2, *chunk_cell, *chunk_cell2;
+    uint32_t *chunk_off, *chunk_off2, *chunk_cell, *chunk_cell2;
+    uint64_t max_chunks;
 };
 
 static fsr_status pass_scratch(fsr_context* ctx, uint32_t C, uint32_t n, PassScratch* ps) {
-    FSR_TRY(arena_typed(ctx, A_AUX0, 4ull * C, &ps->cnt));
-    ps->chunk_off = ps->cnt + C;
-    ps->cnt2 = ps->chunk_off + C;
-    ps->chunk_off2 = ps->cnt2 + C;
-    const uint64_t max_chunks = (uint64_t)n / 64 + C + 1;
-    FSR_TRY(arena_typed(ctx, A_AUX1, 2ull * max_chunks, &ps->chunk_cell));
-    ps->chunk_cell2 = ps->chunk_cell + max_chunks;
+    FSR_TRY(arena_typed(ctx, A_AUX0, 2ull * C, &ps->chunk_off));
+    ps->chunk_off2 = ps->chunk_off + C;
+    ps->max_chunks = (uint64_t)n / 64 + C + 1;
+    FSR_TRY(arena_typed(ctx, A_AUX1, 2ull * ps->max_chunks, &ps->chunk_cell));
+    ps->chunk_cell2 = ps->chunk_cell + ps->max_chunks;
     return FSR_OK;
 }
 
@@ -1872,16 +1835,9 @@ fsr_status aniso_smooth(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     const int blocks = persistent_blocks(ctx, kAnisoThreads, 5, TUNE_ANISO);
     PassScratch ps;
     FSR_TRY(pass_scratch(ctx, C, a.n, &ps));
-    hipLaunchKernelGGL(k_cell_counts, dim3((C + 255) / 256), dim3(256), 0, s, a.ranges,
-                       (const uint32_t*)nullptr, C, ps.cnt);
-    FSR_LAUNCH_CHECK("k_cell_counts");
-    FSR_TRY(scan_exclusive(ctx, SCAN_CHUNKS64, ps.cnt, ps.chunk_off, C, nullptr,
-                           &a.counters->aux[0], s));
-    hipLaunchKernelGGL(k_chunks_of_cells, dim3((C + 255) / 256), dim3(256), 0, s, ps.cnt,
-                       ps.chunk_off, C, ps.chunk_cell);
-    FSR_LAUNCH_CHECK("k_chunks_of_cells");
+    FSR_TRY(cell_chunk_list(ctx, a.ranges, nullptr, C, ps.chunk_off, ps.chunk_cell,
+                            ps.max_chunks, &a.counters->aux[0], s));
     ChunkList cl{ps.chunk_cell, ps.chunk_off, &a.counters->aux[0], a.counters->xcd_next};
-    FSR_TRY(reset_xcd(a.counters, s));
     uint32_t* work;
     FSR_TRY(work_section(ctx, WORK_SMOOTH, &work));
     // at least n / 64 chunks: a large frame takes the build without the shared form
@@ -1912,15 +1868,9 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     const int blocks_cov = persistent_blocks(ctx, kAnisoThreads, 4, TUNE_ANISO);
     PassScratch ps;
     FSR_TRY(pass_scratch(ctx, C, a.n, &ps));
-    hipLaunchKernelGGL(k_cell_counts, dim3((C + 255) / 256), dim3(256), 0, s, a.ranges,
-                       a.involve, C, ps.cnt2);
-    FSR_LAUNCH_CHECK("k_cell_counts");
-    FSR_TRY(scan_exclusive(ctx, SCAN_CHUNKS64, ps.cnt2, ps.chunk_off2, C, nullptr,
-                           &a.counters->aux[2], s));
-    hipLaunchKernelGGL(k_chunks_of_cells, dim3((C + 255) / 256), dim3(256), 0, s, ps.cnt2,
-                       ps.chunk_off2, C, ps.chunk_cell2);
-    FSR_LAUNCH_CHECK("k_chunks_of_cells");
-    ChunkList cl2{ps.chunk_cell2, ps.chunk_off2, &a.counters->aux[2], a.counters->xcd_next};
+    FSR_TRY(cell_chunk_list(ctx, a.ranges, a.involve, C, ps.chunk_off2, ps.chunk_cell2,
+                            ps.max_chunks, &a.counters->aux[2], s));
+    ChunkList cl2{ps.chunk_cell2, ps.chunk_off2, &a.counters->aux[2], a.counters->xcd_cov};
     CovArgs ca;
     ca.sorted = a.sorted;
     ca.mean = a.mean;
@@ -1941,7 +1891,6 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     ca.rec = a.rec;
     FSR_TRY(work_section(ctx, WORK_COV, &ca.work));
     FSR_TRY(cell_boxes(ctx, a, s, &ca.cell_box));
-    FSR_TRY(reset_xcd(a.counters, s));
     // the chunks hold the involved particles only, at most all
     const uint32_t coop_max = coop_limit(ctx, blocks_cov);
     auto cov = a.n / 64u <= 2u * coop_max ? k_covariance_mc<true> : k_covariance_mc<false>;
@@ -2027,14 +1976,13 @@ fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOu
     fa.sp = a.sp;
     fa.sc = a.sc;
     fa.phi = phi;
-    fa.next = a.counters->xcd_next;
+    fa.next = a.counters->xcd_field;
     fa.num_chunks = &a.counters->num_chunks;
     if (a.n && !moments) {
         hipLaunchKernelGGL(k_cull_radius_to_w, dim3((a.n + 255) / 256), dim3(256), 0, s, a.rec,
                            a.n, a.smooth, 0);
         FSR_LAUNCH_CHECK("k_cull_radius_to_w");
     }
-    FSR_TRY(reset_xcd(a.counters, s));
     auto kernel = field_waves == 4 ? k_field_aniso<4, false> : k_field_aniso<5, false>;
     if (few_chunks(ctx, a.n))
         kernel = field_waves == 4 ? k_field_aniso<4, true> : k_field_aniso<5, true>;

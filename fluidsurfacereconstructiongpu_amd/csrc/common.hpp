@@ -370,7 +370,7 @@ enum ArenaSlot {
     A_INVOLVED_IDX, A_MEAN, A_SMOOTH, A_GMAT, A_SIGMA, A_AUX0, A_AUX1, A_REC,
     A_ADJ_VERT, A_ADJ_COEF, A_ADJ_AUX, A_ADJ_TOUCH, A_EDGE_MASK, A_EDGE_OFF, A_SURF_CHUNKS, A_SLAB, A_BAND_PARTIALS,
     A_FIELD_WORK, A_COLOR_WORK, A_MOM_CELL, A_MOM_T1, A_MOM_T2,
-    A_MOM_BLOCK, A_CELL_BOX, A_ANISO_WORK, A_CELL_BOX_RAW, A_ADJ_CORNER, A_INVOLVE_TMP, A_NUM_SLOTS
+    A_MOM_BLOCK, A_CELL_BOX, A_ANISO_WORK, A_CELL_BOX_RAW, A_ADJ_CORNER, A_NUM_SLOTS
 };
 
 // Band vertices grouped by hash cell (band.hip).
@@ -409,10 +409,12 @@ struct Counters {
     uint32_t mc_next;
     uint32_t aux[12];
     uint32_t pad[12];
-    // fetch counters of the persistent kernels (next_item_xcd), 128 B apart
+    // fetch counters of the persistent kernels (ItemFetch), 128 B apart: of the
+    // colour field or the smoothing, of the covariance, and of the field; each is
+    // used once per frame, so the frame's initial clear resets them (the adjoint,
+    // which may run more than once after a frame, clears the first itself)
     uint32_t xcd_next[kFetchSegments * 32];
-    // the same for the ZB05 field kernel, used once per frame, so the frame's
-    // initial clear is its reset
+    uint32_t xcd_cov[kFetchSegments * 32];
     uint32_t xcd_field[kFetchSegments * 32];
 };
 
@@ -490,7 +492,7 @@ fsr_status arena_typed(fsr_context* ctx, ArenaSlot s, uint64_t n, T** out) {
 // ---------------------------------------------------------------------------
 
 // scan.hip ------------------------------------------------------------------
-enum ScanInput { SCAN_U32 = 0, SCAN_POPC = 1, SCAN_CHUNKS64 = 2, SCAN_NONZERO = 3 };
+enum ScanInput { SCAN_U32 = 0, SCAN_POPC = 1, SCAN_NONZERO = 2 };
 // Exclusive scan of f(in[i]) for i < n, where n = *d_count when d_count is not
 // null (bounded by n_max) and n_max otherwise.  Writes the total to *d_total
 // when d_total is not null.
@@ -511,6 +513,13 @@ fsr_status scan_exclusive_noalloc(int device, const uint32_t* in, uint32_t* out,
 fsr_status scan_cells(fsr_context* ctx, const uint32_t* cnt, uint64_t n, uint32_t* cell_off,
                       uint32_t* chunk_off, uint32_t* chunk_cell, uint64_t max_chunks,
                       uint32_t* d_num_chunks, hipStream_t s);
+
+// Chunks of up to 64 particles per hash cell (cells with filter[c] == 0 are
+// skipped when filter is not null): exclusive chunk offsets, chunk -> cell map (at
+// most max_chunks entries), and the total chunk count.
+fsr_status cell_chunk_list(fsr_context* ctx, const fsr_index_range* ranges, const uint32_t* filter,
+                           uint32_t C, uint32_t* chunk_off, uint32_t* chunk_cell,
+                           uint64_t max_chunks, uint32_t* d_num_chunks, hipStream_t s);
 
 // Marching-cubes offsets: vert_off = exclusive scan of the per-cube vertex
 // counts nv (live length *d_count, at most n_max) and valid_idx = the cubes
@@ -719,13 +728,6 @@ fsr_status aniso_involved(fsr_context* ctx, const AnisoArgs& a, hipStream_t s);
 fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s);
 fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOut& bc,
                        float* phi, hipStream_t s);
-// Chunks of up to 64 particles per hash cell (cells with filter[c] == 0 are
-// skipped when filter is not null): counts, exclusive chunk offsets, chunk ->
-// cell map, total chunk count into *d_total.
-fsr_status cell_chunk_list(fsr_context* ctx, const fsr_index_range* ranges,
-                           const uint32_t* filter, uint32_t C, uint32_t* cnt,
-                           uint32_t* chunk_off, uint32_t* chunk_cell, uint32_t* d_total,
-                           hipStream_t s);
 
 // adjoint.hip: backward passes over the state a frame left in ctx->adj
 fsr_status mc_vertex_backward(fsr_context* ctx, const float* g_tri_pos, float* g_phi,

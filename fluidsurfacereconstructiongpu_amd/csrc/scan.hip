@@ -38,7 +38,6 @@ constexpr uint32_t kMaxScanBlocks = 1024;
 template <int F>
 __device__ __forceinline__ uint32_t xform(uint32_t v) {
     if (F == SCAN_POPC) return (uint32_t)__popc(v);
-    if (F == SCAN_CHUNKS64) return (v + 63u) >> 6;
     if (F == SCAN_NONZERO) return v ? 1u : 0u;
     return v;
 }
@@ -320,15 +319,28 @@ __device__ __forceinline__ uint64_t cell_segment(uint64_t n, uint32_t g) {
     return (seg + kCellTile - 1) / kCellTile * kCellTile;
 }
 
+// A cell's count: given, or that of its particles when a filter, if any, is not 0.
+struct CellCounts {
+    const uint32_t* cnt;  // null: from ranges and filter
+    const fsr_index_range* ranges;
+    const uint32_t* filter;
+    __device__ __forceinline__ uint32_t operator()(uint64_t i) const {
+        if (cnt) return cnt[i];
+        const fsr_index_range r = ranges[i];
+        const uint32_t take = filter ? filter[i] : 1u;
+        return r.start == 0xFFFFFFFFu || take == 0u ? 0u : r.end - r.start;
+    }
+};
+
 __global__ __launch_bounds__(kScanThreads) void k_cells_scan_reduce(
-    const uint32_t* __restrict__ cnt, uint64_t n, uint32_t* __restrict__ partials) {
+    CellCounts cnt, uint64_t n, uint32_t* __restrict__ partials) {
     __shared__ uint32_t lds[kScanThreads / 64];
     const uint64_t seg = cell_segment(n, gridDim.x);
     const uint64_t lo = (uint64_t)blockIdx.x * seg;
     const uint64_t hi = lo + seg < n ? lo + seg : n;
     uint32_t sum = 0, ch = 0;
     for (uint64_t i = lo + threadIdx.x; i < hi; i += kScanThreads) {
-        const uint32_t c = cnt[i];
+        const uint32_t c = cnt(i);
         sum += c;
         ch += chunks64(c);
     }
@@ -342,7 +354,7 @@ __global__ __launch_bounds__(kScanThreads) void k_cells_scan_reduce(
 }
 
 __global__ __launch_bounds__(kScanThreads) void k_cells_scan_down(
-    const uint32_t* __restrict__ cnt, uint64_t n, const uint32_t* __restrict__ partials,
+    CellCounts cnt, uint64_t n, const uint32_t* __restrict__ partials,
     uint32_t* __restrict__ cell_off, uint32_t* __restrict__ chunk_off,
     uint32_t* __restrict__ chunk_cell, uint64_t max_chunks, uint32_t* d_num_chunks) {
     __shared__ uint32_t lds[kScanThreads / 64];
@@ -371,14 +383,14 @@ __global__ __launch_bounds__(kScanThreads) void k_cells_scan_down(
     uint32_t run_c = block_exclusive(s1, lds, &excl);
     for (uint64_t base = lo; base < hi; base += kCellTile) {
         const uint64_t i = base + threadIdx.x;
-        const uint32_t c = i < hi ? cnt[i] : 0u;
+        const uint32_t c = i < hi ? cnt(i) : 0u;
         const uint32_t nch = chunks64(c);
         uint32_t ev, ec;
         const uint32_t totv = block_exclusive(c, lds, &ev);
         const uint32_t totc = block_exclusive(nch, lds, &ec);
         if (i < hi) {
             const uint32_t rc = run_c + ec;
-            cell_off[i] = run_v + ev;
+            if (cell_off) cell_off[i] = run_v + ev;
             chunk_off[i] = rc;
             for (uint32_t j = 0; j < nch; ++j)
                 if ((uint64_t)rc + j < max_chunks) chunk_cell[rc + j] = (uint32_t)i;
@@ -527,8 +539,6 @@ fsr_status scan_exclusive(fsr_context* ctx, ScanInput f, const uint32_t* in, uin
     switch (f) {
         case SCAN_U32: return scan_impl<SCAN_U32>(ctx, in, out, n_max, d_count, d_total, s);
         case SCAN_POPC: return scan_impl<SCAN_POPC>(ctx, in, out, n_max, d_count, d_total, s);
-        case SCAN_CHUNKS64:
-            return scan_impl<SCAN_CHUNKS64>(ctx, in, out, n_max, d_count, d_total, s);
         case SCAN_NONZERO:
             return scan_impl<SCAN_NONZERO>(ctx, in, out, n_max, d_count, d_total, s);
     }
@@ -556,9 +566,9 @@ fsr_status scan_mc(fsr_context* ctx, const uint32_t* nv, uint64_t n_max, const u
     return FSR_OK;
 }
 
-fsr_status scan_cells(fsr_context* ctx, const uint32_t* cnt, uint64_t n, uint32_t* cell_off,
-                      uint32_t* chunk_off, uint32_t* chunk_cell, uint64_t max_chunks,
-                      uint32_t* d_num_chunks, hipStream_t s) {
+static fsr_status scan_cell_counts(fsr_context* ctx, const CellCounts& cnt, uint64_t n,
+                                   uint32_t* cell_off, uint32_t* chunk_off, uint32_t* chunk_cell,
+                                   uint64_t max_chunks, uint32_t* d_num_chunks, hipStream_t s) {
     const uint64_t want = (n + kCellTile - 1) / kCellTile;
     const uint32_t g = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, kMaxCellBlocks));
     uint32_t* partials = nullptr;
@@ -569,6 +579,20 @@ fsr_status scan_cells(fsr_context* ctx, const uint32_t* cnt, uint64_t n, uint32_
                        cell_off, chunk_off, chunk_cell, max_chunks, d_num_chunks);
     FSR_LAUNCH_CHECK("k_cells_scan_down");
     return FSR_OK;
+}
+
+fsr_status scan_cells(fsr_context* ctx, const uint32_t* cnt, uint64_t n, uint32_t* cell_off,
+                      uint32_t* chunk_off, uint32_t* chunk_cell, uint64_t max_chunks,
+                      uint32_t* d_num_chunks, hipStream_t s) {
+    return scan_cell_counts(ctx, CellCounts{cnt, nullptr, nullptr}, n, cell_off, chunk_off,
+                            chunk_cell, max_chunks, d_num_chunks, s);
+}
+
+fsr_status cell_chunk_list(fsr_context* ctx, const fsr_index_range* ranges, const uint32_t* filter,
+                           uint32_t C, uint32_t* chunk_off, uint32_t* chunk_cell,
+                           uint64_t max_chunks, uint32_t* d_num_chunks, hipStream_t s) {
+    return scan_cell_counts(ctx, CellCounts{nullptr, ranges, filter}, C, nullptr, chunk_off,
+                            chunk_cell, max_chunks, d_num_chunks, s);
 }
 
 fsr_status fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {
