@@ -223,13 +223,24 @@ __device__ __forceinline__ void wave_box(bool live, float x, float y, float z, f
 constexpr float kRadiusCull = 1.001f;
 
 
+// The field kernel tests a candidate's box distance against the candidate's
+// squared culling radius (w of its second record word) before it reads the
+// records: a copy of that radius stands in the w of the smoothed position, put
+// there by the kernels that make the records.  With the non-involved moments,
+// those particles (never culled otherwise) get a negative radius: the box test
+// then drops them.
+__device__ __forceinline__ float field_cull_w(float w, int drop_noninv) {
+    return drop_noninv && w == kNoCull ? -1.0f : w;
+}
+
 // ---------------------------------------------------------------- K8 --------
 // Involved list and the per-particle field records of non-involved particles.
 __global__ __launch_bounds__(256) void k_involved(
     const uint32_t* __restrict__ keys, const fsr_index_range* __restrict__ ranges,
     const uint32_t* __restrict__ involve, const uint32_t* __restrict__ involve_off,
     const float4* __restrict__ sorted, uint32_t n, uint32_t C, float mass,
-    uint32_t* __restrict__ involved_idx, float4* __restrict__ rec) {
+    uint32_t* __restrict__ involved_idx, float4* __restrict__ rec, float4* __restrict__ smooth,
+    int drop_noninv) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t c = keys[i];
@@ -240,6 +251,7 @@ __global__ __launch_bounds__(256) void k_involved(
         // units) covers the whole candidate block, so it is never culled
         rec[2ull * i + 0] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
         rec[2ull * i + 1] = make_float4(0.0f, 0.0f, kSigma * (mass / sorted[i].w), kNoCull);
+        smooth[i].w = field_cull_w(kNoCull, drop_noninv);
     }
 }
 
@@ -300,6 +312,8 @@ struct CovArgs {
     float mass;
     fsr_matrix* gmat;       // [I]
     float4* sigma;          // [I] eigenvalues, descending
+    float4* smooth;     // its w gets the culling radius (may be null)
+    int drop_noninv;
     float4* rec;            // [2N] field records
     uint32_t* work;         // work records (may be null)
     const float4* cell_box; // per cell lo[C], hi[C] (k_cell_box)
@@ -357,7 +371,9 @@ __device__ __forceinline__ void cov_finish(const CovArgs& a, uint32_t gi, uint32
     const float coef = kSigma * det * (a.mass / a.sorted[i].w);
     a.rec[2ull * i + 0] = make_float4(M[0][0], M[1][1], M[2][2], M[0][1]);
     // squared culling radius of the field kernel, with a 1% margin
-    a.rec[2ull * i + 1] = make_float4(M[0][2], M[1][2], coef, kCullMargin / (gmin * gmin));
+    const float cull = kCullMargin / (gmin * gmin);
+    a.rec[2ull * i + 1] = make_float4(M[0][2], M[1][2], coef, cull);
+    if (a.smooth) a.smooth[i].w = field_cull_w(cull, a.drop_noninv);
 }
 
 
@@ -1756,19 +1772,12 @@ __global__ __launch_bounds__(256) void k_window5(const double* __restrict__ in,
     out[t] = acc;
 }
 
-// The field kernel tests a candidate's box distance against the candidate's
-// squared culling radius (w of its second record word) before it reads the
-// records: a copy of that radius goes into the w of the smoothed position.
-// With the non-involved moments, those particles (never culled otherwise)
-// get a negative radius: the box test then drops them.
+// The same copy for records that the caller gives (the field on its own).
 __global__ __launch_bounds__(256) void k_cull_radius_to_w(const float4* __restrict__ rec,
-                                                          uint32_t n, float4* __restrict__ smooth,
-                                                          int drop_noninv) {
+                                                          uint32_t n,
+                                                          float4* __restrict__ smooth) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float w = rec[2ull * i + 1].w;
-    if (drop_noninv && w == kNoCull) w = -1.0f;
-    reinterpret_cast<float*>(smooth)[4ull * i + 3] = w;
+    if (i < n) smooth[i].w = rec[2ull * i + 1].w;
 }
 
 }  // namespace
@@ -1782,6 +1791,20 @@ float sqrt_bound(float r, bool strict) {
     while (t > 0.0f && !ok(t)) t = std::nextafter(t, 0.0f);
     while (ok(std::nextafter(t, inf))) t = std::nextafter(t, inf);
     return t;
+}
+
+// Whether every particle of a clamped 5^3 block lies within distance 1 of
+// every vertex whose cell owns the block, smoothing displacement included: the
+// reference's non-involved kernel then never reaches its cutoff |r| >= 1 and
+// the block sum is the polynomial of noninv_poly.
+static bool noninv_polynomial_exact(const GridDev& sp, float smoothing_radius) {
+    const double reach = std::sqrt(3.0) * 6.0 * (double)sp.cell + 2.0 * (double)smoothing_radius;
+    return reach < 0.9;
+}
+
+// Whether the field sums the non-involved particles by moments.
+static bool sums_moments(const AnisoArgs& a) {
+    return a.noninv_moments && noninv_polynomial_exact(a.sp, a.aniso_radius);
 }
 
 // Scratch of the two particle passes: per-cell counts and chunk offsets, and
@@ -1835,8 +1858,9 @@ fsr_status aniso_smooth(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     const int blocks = persistent_blocks(ctx, kAnisoThreads, 5, TUNE_ANISO);
     PassScratch ps;
     FSR_TRY(pass_scratch(ctx, C, a.n, &ps));
-    FSR_TRY(cell_chunk_list(ctx, a.ranges, nullptr, C, ps.chunk_off, ps.chunk_cell,
-                            ps.max_chunks, &a.counters->aux[0], s));
+    if (!a.lists_ready)
+        FSR_TRY(cell_chunk_list(ctx, a.ranges, nullptr, C, ps.chunk_off, ps.chunk_cell,
+                                ps.max_chunks, &a.counters->aux[0], s));
     ChunkList cl{ps.chunk_cell, ps.chunk_off, &a.counters->aux[0], a.counters->xcd_next};
     uint32_t* work;
     FSR_TRY(work_section(ctx, WORK_SMOOTH, &work));
@@ -1851,12 +1875,13 @@ fsr_status aniso_smooth(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
 
 fsr_status aniso_involved(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     const uint32_t C = a.sp.rx * a.sp.ry * a.sp.rz;
-    FSR_TRY(scan_exclusive(ctx, SCAN_U32, a.involve, a.involve_off, C, nullptr,
-                           &a.st->num_involved_particles, s));
+    if (!a.lists_ready)
+        FSR_TRY(scan_exclusive(ctx, SCAN_U32, a.involve, a.involve_off, C, nullptr,
+                               &a.st->num_involved_particles, s));
     if (a.n) {
         hipLaunchKernelGGL(k_involved, dim3((a.n + 255) / 256), dim3(256), 0, s, a.keys, a.ranges,
                            a.involve, a.involve_off, a.sorted, a.n, C, a.mass, a.involved_idx,
-                           a.rec);
+                           a.rec, a.smooth, sums_moments(a) ? 1 : 0);
         FSR_LAUNCH_CHECK("k_involved");
     }
     return FSR_OK;
@@ -1868,8 +1893,9 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     const int blocks_cov = persistent_blocks(ctx, kAnisoThreads, 4, TUNE_ANISO);
     PassScratch ps;
     FSR_TRY(pass_scratch(ctx, C, a.n, &ps));
-    FSR_TRY(cell_chunk_list(ctx, a.ranges, a.involve, C, ps.chunk_off2, ps.chunk_cell2,
-                            ps.max_chunks, &a.counters->aux[2], s));
+    if (!a.lists_ready)
+        FSR_TRY(cell_chunk_list(ctx, a.ranges, a.involve, C, ps.chunk_off2, ps.chunk_cell2,
+                                ps.max_chunks, &a.counters->aux[2], s));
     ChunkList cl2{ps.chunk_cell2, ps.chunk_off2, &a.counters->aux[2], a.counters->xcd_cov};
     CovArgs ca;
     ca.sorted = a.sorted;
@@ -1889,6 +1915,8 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     ca.gmat = a.gmat;
     ca.sigma = a.sigma;
     ca.rec = a.rec;
+    ca.smooth = a.smooth;
+    ca.drop_noninv = sums_moments(a) ? 1 : 0;
     FSR_TRY(work_section(ctx, WORK_COV, &ca.work));
     FSR_TRY(cell_boxes(ctx, a, s, &ca.cell_box));
     // the chunks hold the involved particles only, at most all
@@ -1900,21 +1928,19 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
 }
 
 fsr_status aniso_run(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
-    // the cell boxes once for both neighbour passes
+    // the cell boxes and the work lists once for both neighbour passes
     AnisoArgs b = a;
     FSR_TRY(cell_boxes(ctx, a, s, &b.cell_box));
+    const uint32_t C = a.sp.rx * a.sp.ry * a.sp.rz;
+    PassScratch ps;
+    FSR_TRY(pass_scratch(ctx, C, a.n, &ps));
+    FSR_TRY(pass_lists(ctx, a.ranges, a.involve, C, ps.chunk_off, ps.chunk_cell, ps.chunk_off2,
+                       ps.chunk_cell2, ps.max_chunks, a.involve_off, &a.counters->aux[0],
+                       &a.counters->aux[2], &a.st->num_involved_particles, s));
+    b.lists_ready = true;
     FSR_TRY(aniso_smooth(ctx, b, s));
     FSR_TRY(aniso_involved(ctx, b, s));
     return aniso_cov(ctx, b, s);
-}
-
-// Whether every particle of a clamped 5^3 block lies within distance 1 of
-// every vertex whose cell owns the block, smoothing displacement included: the
-// reference's non-involved kernel then never reaches its cutoff |r| >= 1 and
-// the block sum is the polynomial of noninv_poly.
-static bool noninv_polynomial_exact(const GridDev& sp, float smoothing_radius) {
-    const double reach = std::sqrt(3.0) * 6.0 * (double)sp.cell + 2.0 * (double)smoothing_radius;
-    return reach < 0.9;
 }
 
 fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOut& bc,
@@ -1932,7 +1958,7 @@ fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOu
     fa.ox = a.sp.minx;
     fa.oy = a.sp.miny;
     fa.oz = a.sp.minz;
-    const bool moments = a.noninv_moments && noninv_polynomial_exact(a.sp, a.aniso_radius);
+    const bool moments = sums_moments(a);
     if (moments) {
         const uint32_t C = a.sp.rx * a.sp.ry * a.sp.rz;
         const uint32_t rx = a.sp.rx, ry = a.sp.ry, rz = a.sp.rz;
@@ -1946,12 +1972,7 @@ fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOu
         FSR_TRY(arena_typed(ctx, A_CELL_BOX, 2ull * C, &boxes));
         fa.cell_lo = boxes;
         fa.cell_hi = boxes + C;
-        // the boxes need the culling radii in the w of the smoothed positions
-        if (a.n) {
-            hipLaunchKernelGGL(k_cull_radius_to_w, dim3((a.n + 255) / 256), dim3(256), 0, s,
-                               a.rec, a.n, a.smooth, 1);
-            FSR_LAUNCH_CHECK("k_cull_radius_to_w");
-        }
+        // (the culling radii are in the w of the smoothed positions)
         hipLaunchKernelGGL(k_cell_moments_boxes, dim3(C), dim3(64), 0, s, a.ranges, a.involve,
                            (const float4*)a.smooth, a.sorted, a.mass, fa.ox, fa.oy, fa.oz, cm,
                            boxes, boxes + C);
@@ -1978,9 +1999,10 @@ fsr_status aniso_field(fsr_context* ctx, const AnisoArgs& a, const BandCompactOu
     fa.phi = phi;
     fa.next = a.counters->xcd_field;
     fa.num_chunks = &a.counters->num_chunks;
-    if (a.n && !moments) {
+    if (a.n && !a.noninv_moments) {
+        // records of the caller, not of aniso_run
         hipLaunchKernelGGL(k_cull_radius_to_w, dim3((a.n + 255) / 256), dim3(256), 0, s, a.rec,
-                           a.n, a.smooth, 0);
+                           a.n, a.smooth);
         FSR_LAUNCH_CHECK("k_cull_radius_to_w");
     }
     auto kernel = field_waves == 4 ? k_field_aniso<4, false> : k_field_aniso<5, false>;

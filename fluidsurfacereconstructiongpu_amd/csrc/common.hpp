@@ -521,6 +521,14 @@ fsr_status cell_chunk_list(fsr_context* ctx, const fsr_index_range* ranges, cons
                            uint32_t C, uint32_t* chunk_off, uint32_t* chunk_cell,
                            uint64_t max_chunks, uint32_t* d_num_chunks, hipStream_t s);
 
+// cell_chunk_list of all particles and of the involved cells (involve: their
+// particle counts, else 0), and the exclusive scan of involve, with their totals.
+fsr_status pass_lists(fsr_context* ctx, const fsr_index_range* ranges, const uint32_t* involve,
+                      uint32_t C, uint32_t* chunk_off, uint32_t* chunk_cell, uint32_t* chunk_off2,
+                      uint32_t* chunk_cell2, uint64_t max_chunks, uint32_t* involve_off,
+                      uint32_t* d_chunks, uint32_t* d_chunks2, uint32_t* d_involved,
+                      hipStream_t s);
+
 // Marching-cubes offsets: vert_off = exclusive scan of the per-cube vertex
 // counts nv (live length *d_count, at most n_max) and valid_idx = the cubes
 // with nv > 0 in ascending order; the totals go to the two device counters.
@@ -719,6 +727,9 @@ struct AnisoArgs {
     // smoothing and covariance (float4 lo[C], hi[C]); computed by the first
     // of those kernels when null
     const float4* cell_box = nullptr;
+    // the chunk lists of both passes and involve_off are made (pass_lists); else
+    // each step makes its own
+    bool lists_ready = false;
 };
 fsr_status aniso_run(fsr_context* ctx, const AnisoArgs& a, hipStream_t s);
 // steps of aniso_run: smoothing (K10), involved list + non-involved field

@@ -401,6 +401,79 @@ __global__ __launch_bounds__(kScanThreads) void k_cells_scan_down(
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *d_num_chunks = run_c;
 }
 
+// The lists of the two Yu13 particle passes in one scan: of all particles' chunks,
+// of the involved cells' chunks, and the involved cells' particle offsets.
+struct PassLists {
+    uint32_t *chunk_off, *chunk_cell, *chunk_off2, *chunk_cell2, *involve_off;
+    uint32_t *d_chunks, *d_chunks2, *d_involved;
+    uint64_t max_chunks;
+};
+
+__global__ __launch_bounds__(kScanThreads) void k_pass_scan_reduce(
+    CellCounts all, const uint32_t* __restrict__ involve, uint64_t n,
+    uint32_t* __restrict__ partials) {
+    __shared__ uint32_t lds[kScanThreads / 64];
+    const uint64_t seg = cell_segment(n, gridDim.x);
+    const uint64_t lo = (uint64_t)blockIdx.x * seg;
+    const uint64_t hi = lo + seg < n ? lo + seg : n;
+    uint32_t sum[3] = {0, 0, 0};
+    for (uint64_t i = lo + threadIdx.x; i < hi; i += kScanThreads) {
+        const uint32_t a = all(i), v = involve[i];
+        sum[0] += chunks64(a);
+        sum[1] += chunks64(v);
+        sum[2] += v;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        uint32_t excl;
+        const uint32_t t = block_exclusive(sum[k], lds, &excl);
+        if (threadIdx.x == 0) partials[(uint32_t)k * gridDim.x + blockIdx.x] = t;
+    }
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_pass_scan_down(
+    CellCounts all, const uint32_t* __restrict__ involve, uint64_t n,
+    const uint32_t* __restrict__ partials, PassLists l) {
+    __shared__ uint32_t lds[kScanThreads / 64];
+    const uint64_t seg = cell_segment(n, gridDim.x);
+    const uint64_t lo = (uint64_t)blockIdx.x * seg;
+    const uint64_t hi = lo + seg < n ? lo + seg : n;
+    uint32_t before[3] = {0, 0, 0}, run[3], excl;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kScanThreads) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) before[k] += partials[(uint32_t)k * gridDim.x + i];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) run[k] = block_exclusive(before[k], lds, &excl);
+    for (uint64_t base = lo; base < hi; base += kCellTile) {
+        const uint64_t i = base + threadIdx.x;
+        const uint32_t a = i < hi ? all(i) : 0u, v = i < hi ? involve[i] : 0u;
+        const uint32_t na = chunks64(a), nv = chunks64(v);
+        uint32_t ea, ev, eo;
+        const uint32_t ta = block_exclusive(na, lds, &ea);
+        const uint32_t tv = block_exclusive(nv, lds, &ev);
+        const uint32_t to = block_exclusive(v, lds, &eo);
+        if (i < hi) {
+            const uint32_t oa = run[0] + ea, ov = run[1] + ev;
+            l.chunk_off[i] = oa;
+            l.chunk_off2[i] = ov;
+            l.involve_off[i] = run[2] + eo;
+            for (uint32_t j = 0; j < na; ++j)
+                if ((uint64_t)oa + j < l.max_chunks) l.chunk_cell[oa + j] = (uint32_t)i;
+            for (uint32_t j = 0; j < nv; ++j)
+                if ((uint64_t)ov + j < l.max_chunks) l.chunk_cell2[ov + j] = (uint32_t)i;
+        }
+        run[0] += ta;
+        run[1] += tv;
+        run[2] += to;
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        *l.d_chunks = run[0];
+        *l.d_chunks2 = run[1];
+        *l.d_involved = run[2];
+    }
+}
+
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (uint64_t)gridDim.x * blockDim.x)
@@ -593,6 +666,27 @@ fsr_status cell_chunk_list(fsr_context* ctx, const fsr_index_range* ranges, cons
                            uint64_t max_chunks, uint32_t* d_num_chunks, hipStream_t s) {
     return scan_cell_counts(ctx, CellCounts{nullptr, ranges, filter}, C, nullptr, chunk_off,
                             chunk_cell, max_chunks, d_num_chunks, s);
+}
+
+fsr_status pass_lists(fsr_context* ctx, const fsr_index_range* ranges, const uint32_t* involve,
+                      uint32_t C, uint32_t* chunk_off, uint32_t* chunk_cell, uint32_t* chunk_off2,
+                      uint32_t* chunk_cell2, uint64_t max_chunks, uint32_t* involve_off,
+                      uint32_t* d_chunks, uint32_t* d_chunks2, uint32_t* d_involved,
+                      hipStream_t s) {
+    const uint32_t want = (uint32_t)(((uint64_t)C + kCellTile - 1) / kCellTile);
+    const uint32_t g = std::max(1u, std::min(want, kMaxCellBlocks));
+    uint32_t* partials = nullptr;
+    FSR_TRY(arena_typed(ctx, A_SCAN_PARTIALS, 3ull * kMaxCellBlocks, &partials));
+    const CellCounts all{nullptr, ranges, nullptr};
+    const PassLists l{chunk_off, chunk_cell, chunk_off2, chunk_cell2, involve_off,
+                      d_chunks,  d_chunks2,  d_involved, max_chunks};
+    hipLaunchKernelGGL(k_pass_scan_reduce, dim3(g), dim3(kScanThreads), 0, s, all, involve,
+                       (uint64_t)C, partials);
+    FSR_LAUNCH_CHECK("k_pass_scan_reduce");
+    hipLaunchKernelGGL(k_pass_scan_down, dim3(g), dim3(kScanThreads), 0, s, all, involve,
+                       (uint64_t)C, partials, l);
+    FSR_LAUNCH_CHECK("k_pass_scan_down");
+    return FSR_OK;
 }
 
 fsr_status fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {
