@@ -78,9 +78,27 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) {
 // wave-uniform reads, each lane taking the last one that starts at or before
 // its index (an empty row shares its first index with the next row, visited
 // after it).
+//
+// index(nb) is the sorted index of a lane's candidate of that round: one lookup
+// while the round lies inside the row that the last one ended in (row_off, up to
+// candidate row_end), which most do; lanes past the end get particle 0.
 struct BlockRows {
     uint32_t rp, ro, total, jc;
     int nrows;
+    uint32_t row_off, row_end;
+    __device__ __forceinline__ uint32_t index(uint32_t nb) {
+        const uint32_t lane = __lane_id();
+        uint32_t at = row_off + nb + lane;
+        if (nb + 64u > row_end) {
+            const uint32_t off = offset(nb, nb + lane);
+            at = nb + lane < total ? off + nb + lane : 0u;
+            row_off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
+            row_end = jc + 1u < (uint32_t)nrows
+                          ? (uint32_t)__builtin_amdgcn_readlane((int)rp, (int)jc + 1)
+                          : total;
+        }
+        return at;
+    }
     __device__ __forceinline__ uint32_t offset(uint32_t nb, uint32_t gg) {
         uint32_t off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
         for (uint32_t jj = jc + 1u; jj < (uint32_t)nrows; ++jj) {
@@ -92,6 +110,17 @@ struct BlockRows {
         return off;
     }
 };
+
+// x, y, z of a sorted particle (one 12-byte load)
+__device__ __forceinline__ float3 load_xyz(const float4* p) {
+    return *reinterpret_cast<const float3*>(p);
+}
+
+// The lanes with d2 < limit among the first `left` of a staging round.
+__device__ __forceinline__ uint64_t round_mask(float d2, float limit, uint32_t left) {
+    constexpr uint32_t kOlt = 4;  // ordered <, as the compare builtin numbers it
+    return __builtin_amdgcn_fcmpf(d2, limit, kOlt) & (left < 64u ? (1ull << left) - 1ull : ~0ull);
+}
 
 // Cell-level culling (cell_lo / cell_hi may be null): a cell counts only when
 // the bounding box of its particles (cell_lo.xyz, cell_hi.xyz), grown by their
@@ -171,6 +200,8 @@ __device__ __forceinline__ BlockRows block_rows(const fsr_index_range* __restric
     b.ro = rs - b.rp;
     b.jc = 0;
     b.nrows = nrows;
+    b.row_off = 0;
+    b.row_end = 0;
     return b;
 }
 
@@ -561,28 +592,17 @@ __device__ __forceinline__ void nb_chunk(float* __restrict__ q, const float* __r
         for (int g = 0; g < G; ++g) acc[g][T] = v4f{0.f, 0.f, 0.f, 0.f};
     }
     uint32_t head = 0, fill = 0;
-    float4 next = make_float4(0.f, 0.f, 0.f, 0.f);
-    {
-        const uint32_t off = br.offset(0u, lane);
-        if (lane < total) next = sorted[off + lane];
-    }
+    float3 next = make_float3(0.f, 0.f, 0.f);
+    if (total) next = load_xyz(sorted + br.index(0u));
     for (uint32_t base = 0; base < total; base += 64u) {
-        const uint32_t g = base + lane;
-        const float4 cand = next;
-        if (base + 64u < total) {
-            const uint32_t off = br.offset(base + 64u, g + 64u);
-            if (g + 64u < total) next = sorted[off + g + 64u];
-        }
-        bool keep = false;
-        float px = 0.f, py = 0.f, pz = 0.f;
-        if (g < total) {
-            px = cand.x - ox;
-            py = cand.y - oy;
-            pz = cand.z - oz;
-            keep = box_dist2(px, py, pz, bb0, bb1) < cull2;
-        }
-        const uint64_t m = __ballot(keep);
-        if (keep) {
+        float px = next.x - ox, py = next.y - oy, pz = next.z - oz;
+        // (before the next load, which takes the same registers: the wait for this
+        // one must not cover it)
+        asm volatile("" : "+v"(px), "+v"(py), "+v"(pz));
+        if (base + 64u < total) next = load_xyz(sorted + br.index(base + 64u));
+        // lane mask from the compare, less the last round's lanes past the end
+        const uint64_t m = round_mask(box_dist2(px, py, pz, bb0, bb1), cull2, total - base);
+        if (__builtin_amdgcn_inverse_ballot_w64(m)) {
             const uint32_t slot = (head + fill + mask_rank(m)) & (kNbQueue - 1);
             q[slot] = px;
             q[kNbStride + slot] = py;
@@ -1569,52 +1589,52 @@ __global__ __launch_bounds__(kAnisoThreads, kWaves) void k_field_aniso(AnisoFiel
             // or 64.
             uint32_t head = 0, fill = 0;
             float4 np4 = make_float4(0.f, 0.f, 0.f, 0.f);
-            uint32_t nj;
-            {
-                nj = br.offset(0u, lane) + lane;
-                if (lane < total) np4 = a.smooth[nj];
+            uint32_t nj = 0;
+            if (total) {
+                nj = br.index(0u);
+                np4 = a.smooth[nj];
             }
-            bool keep_p = false;
+            uint64_t m_p = 0;  // the previous round's survivors
             float px_p = 0.f, py_p = 0.f, pz_p = 0.f;
             float4 r0_p = make_float4(0.f, 0.f, 0.f, 0.f), r1_p = r0_p;
             for (uint32_t base = 0; base < total + 64u; base += 64u) {
-                const uint32_t g = base + lane;
-                bool keep = false;
+                uint64_t keep = 0;
                 float px = 0.f, py = 0.f, pz = 0.f;
                 float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0;
                 if (base < total) {
-                    const float4 p4 = np4;
-                    const uint32_t j = nj;
+                    px = np4.x - ox;
+                    py = np4.y - oy;
+                    pz = np4.z - oz;
+                    float w = np4.w;
+                    uint32_t j = nj;
+                    // (before the next load, which takes the same registers)
+                    asm volatile("" : "+v"(px), "+v"(py), "+v"(pz), "+v"(w), "+v"(j));
                     if (base + 64u < total) {
-                        nj = br.offset(base + 64u, g + 64u) + g + 64u;
-                        if (g + 64u < total) np4 = a.smooth[nj];
+                        nj = br.index(base + 64u);
+                        np4 = a.smooth[nj];
                     }
-                    if (g < total) {
-                        px = p4.x - ox;
-                        py = p4.y - oy;
-                        pz = p4.z - oz;
-                        const float dx = px - __builtin_amdgcn_fmed3f(px, bx0, bx1);
-                        const float dy = py - __builtin_amdgcn_fmed3f(py, by0, by1);
-                        const float dz = pz - __builtin_amdgcn_fmed3f(pz, bz0, bz1);
-                        keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < p4.w;
-                    }
-                    const uint32_t jr = keep ? j : 0u;
+                    const float dx = px - __builtin_amdgcn_fmed3f(px, bx0, bx1);
+                    const float dy = py - __builtin_amdgcn_fmed3f(py, by0, by1);
+                    const float dz = pz - __builtin_amdgcn_fmed3f(pz, bz0, bz1);
+                    keep = round_mask(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)), w,
+                                      total - base);
+                    const uint32_t jr = __builtin_amdgcn_inverse_ballot_w64(keep) ? j : 0u;
                     r0 = a.rec[2ull * jr + 0];
                     r1 = a.rec[2ull * jr + 1];
                 }
                 if (base == 0) {
-                    keep_p = keep;
+                    m_p = keep;
                     px_p = px; py_p = py; pz_p = pz;
                     r0_p = r0; r1_p = r1;
                     continue;
                 }
                 // the previous round's survivors enter the queue
-                const uint64_t m = __ballot(keep_p);
-                if (keep_p) {
+                const uint64_t m = m_p;
+                if (__builtin_amdgcn_inverse_ballot_w64(m)) {
                     const uint32_t o = (head + fill + mask_rank(m)) & (kAfQueue - 1);
                     af_enter<kAfStride>(q + o, px_p, py_p, pz_p, r0_p, r1_p);
                 }
-                keep_p = keep;
+                m_p = keep;
                 px_p = px; py_p = py; pz_p = pz;
                 r0_p = r0; r1_p = r1;
                 fill += (uint32_t)__popcll(m);
