@@ -373,16 +373,26 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
         const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         const uint32_t rp = incl - len;
         const uint32_t ro = rs - rp;
-        uint32_t jc = 0;
-        auto run_offset = [&](uint32_t nb, uint32_t gg) {
-            uint32_t off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
-            for (uint32_t jj = jc + 1u; jj < 9u; ++jj) {
-                const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)rp, (int)jj);
-                if (pj >= nb + 64u) break;
-                if (gg >= pj) off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jj);
-                jc = jj;
+        // the slot of this lane's vertex of the 64 that start at nb: one lookup
+        // while they lie inside the run that the last ones ended in; lanes past
+        // the end take slot 0.  (With one load site and no branch around the box
+        // test: 567 -> 543 us for 256k particles, 286 -> 274 for 64k.)
+        uint32_t jc = 0, run_off = 0, run_end = 0;
+        auto slot_of = [&](uint32_t nb) {
+            uint32_t at = run_off + nb + lane;
+            if (nb + 64u > run_end) {
+                uint32_t off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
+                for (uint32_t jj = jc + 1u; jj < 9u; ++jj) {
+                    const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)rp, (int)jj);
+                    if (pj >= nb + 64u) break;
+                    if (nb + lane >= pj) off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jj);
+                    jc = jj;
+                }
+                at = nb + lane < total ? off + nb + lane : 0u;
+                run_off = (uint32_t)__builtin_amdgcn_readlane((int)ro, (int)jc);
+                run_end = jc < 8u ? (uint32_t)__builtin_amdgcn_readlane((int)rp, (int)jc + 1) : total;
             }
-            return off;
+            return at;
         };
 
         const float ox = __builtin_fmaf((float)qcx, a.sp.cell, a.sp.minx);
@@ -409,35 +419,29 @@ __global__ __launch_bounds__(kAdjThreads, 6) void k_field_zb05_backward_mc(Field
         const float bk = (lane >> 4) == 3u ? 1.0f : bt * (0.5f * a.radius_sq);
         uint32_t head = 0, fill = 0;
         float4 ncf = make_float4(0.f, 0.f, 0.f, 0.f), nvp = ncf;
-        {
-            const uint32_t g0 = 64u * wave;
-            const uint32_t off = run_offset(g0, g0 + lane);
-            if (g0 + lane < total) {
-                ncf = a.coef[off + g0 + lane];
-                nvp = a.vpos[off + g0 + lane];
-            }
+        if (64u * wave < total) {
+            const uint32_t at = slot_of(64u * wave);
+            ncf = a.coef[at];
+            nvp = a.vpos[at];
         }
         for (uint32_t base = 0; base < total; base += 256u) {
-            const uint32_t gi = base + 64u * wave + lane;
-            const float4 cf = ncf, vp = nvp;
-            if (base + 256u < total) {
-                const uint32_t off = run_offset(base + 256u + 64u * wave, gi + 256u);
-                if (gi + 256u < total) {
-                    ncf = a.coef[off + gi + 256u];
-                    nvp = a.vpos[off + gi + 256u];
-                }
+            const uint32_t nb = base + 64u * wave;
+            float4 cf = ncf;
+            float xx = nvp.x - ox, xy = nvp.y - oy, xz = nvp.z - oz;
+            // (before the next loads, which take the same registers)
+            asm volatile("" : "+v"(cf.x), "+v"(cf.y), "+v"(cf.z), "+v"(cf.w), "+v"(xx), "+v"(xy),
+                         "+v"(xz));
+            if (nb + 256u < total) {
+                const uint32_t at = slot_of(nb + 256u);
+                ncf = a.coef[at];
+                nvp = a.vpos[at];
             }
-            bool keep = false;
-            float xx = 0.f, xy = 0.f, xz = 0.f;
-            if (gi < total && (cf.x != 0.0f || cf.y != 0.0f || cf.z != 0.0f || cf.w != 0.0f)) {
-                xx = vp.x - ox;
-                xy = vp.y - oy;
-                xz = vp.z - oz;
-                const float dx = xx - __builtin_amdgcn_fmed3f(xx, bx0, bx1);
-                const float dy = xy - __builtin_amdgcn_fmed3f(xy, by0, by1);
-                const float dz = xz - __builtin_amdgcn_fmed3f(xz, bz0, bz1);
-                keep = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull_r2;
-            }
+            const float dx = xx - __builtin_amdgcn_fmed3f(xx, bx0, bx1);
+            const float dy = xy - __builtin_amdgcn_fmed3f(xy, by0, by1);
+            const float dz = xz - __builtin_amdgcn_fmed3f(xz, bz0, bz1);
+            const bool keep =
+                nb + lane < total && (cf.x != 0.0f || cf.y != 0.0f || cf.z != 0.0f || cf.w != 0.0f) &&
+                __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) < cull_r2;
             const uint64_t m = __ballot(keep);
             if (lane == 0) count[wave] = (uint32_t)__popcll(m);
             __syncthreads();
