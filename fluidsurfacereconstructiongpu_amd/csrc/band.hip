@@ -425,8 +425,8 @@ __global__ __launch_bounds__(64 * kExcWaves) void k_band_exceptions(BandArgs a, 
 }
 
 // Compaction of the band mask into the ascending band index (the reference's
-// scan + compactSurfaceVertex), in two launches: k_band_partials counts the
-// set bits of every 256-word block; k_band_emit gives each block its offset
+// scan + compactSurfaceVertex): k_axis_maps counts the set bits of every 256-word
+// block; then band_emit gives each block its offset
 // (the sum of the counts of the blocks before it, at most 8 words per thread
 // from L2), scans its words' counts, writes each word's offset (word_off, the
 // band rank of the word's first vertex) and the block's vertices, 16 lanes for a
@@ -436,26 +436,15 @@ __global__ __launch_bounds__(64 * kExcWaves) void k_band_exceptions(BandArgs a, 
 // us for a 1M dam break at 256^3, 39 -> 10.5 with the wider band of Akinci12, 25
 // -> 12 at 384^3; 3.0 -> 4.1 where the grid has a few full words only.
 // The last block writes the band size.
-__global__ __launch_bounds__(256) void k_band_partials(const uint32_t* __restrict__ bits,
-                                                       uint64_t nwords,
-                                                       uint32_t* __restrict__ partials) {
-    __shared__ uint32_t part[4];
-    const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t c = wave_sum(w < nwords ? (uint32_t)__popc(bits[w]) : 0u);
-    if (__lane_id() == 0) part[threadIdx.x >> 6] = c;
-    __syncthreads();
-    if (threadIdx.x == 0) partials[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
-}
-
-__global__ __launch_bounds__(256) void k_band_emit(const uint32_t* __restrict__ bits,
-                                                   const uint32_t* __restrict__ partials,
-                                                   uint64_t nwords, uint32_t wx, uint32_t rx,
-                                                   uint32_t* __restrict__ word_off,
-                                                   uint32_t* __restrict__ band_index,
-                                                   uint64_t cap, uint32_t* __restrict__ total,
-                                                   int scanned) {
+__device__ __forceinline__ void band_emit(uint32_t block, uint32_t blocks,
+                                          const uint32_t* __restrict__ bits,
+                                          const uint32_t* __restrict__ partials, uint64_t nwords,
+                                          uint32_t wx, uint32_t rx,
+                                          uint32_t* __restrict__ word_off,
+                                          uint32_t* __restrict__ band_index, uint64_t cap,
+                                          uint32_t* __restrict__ total, int scanned) {
     __shared__ uint32_t part[8];
-    const uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t w = (uint64_t)block * blockDim.x + threadIdx.x;
     const bool live = w < nwords;
     const uint32_t b = live ? bits[w] : 0u;
     const uint32_t c = (uint32_t)__popc(b);
@@ -463,14 +452,14 @@ __global__ __launch_bounds__(256) void k_band_emit(const uint32_t* __restrict__ 
     // `scanned`, partials already holds the exclusive offsets)
     uint32_t before = 0;
     if (scanned) {
-        before = threadIdx.x == 0 ? partials[blockIdx.x] : 0u;
+        before = threadIdx.x == 0 ? partials[block] : 0u;
     } else {
         // at most 4096 blocks: up to 16 counts per thread, loaded together
         uint32_t pv[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
             const uint32_t i = threadIdx.x + 256u * k;
-            pv[k] = i < blockIdx.x ? partials[i] : 0u;
+            pv[k] = i < block ? partials[i] : 0u;
         }
 #pragma unroll
         for (int k = 0; k < 16; ++k) before += pv[k];
@@ -493,7 +482,7 @@ __global__ __launch_bounds__(256) void k_band_emit(const uint32_t* __restrict__ 
     }
     const uint32_t o = lo + wave_off + incl - c;
     if (live) word_off[w] = o;
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = lo + block_total;
+    if (block == blocks - 1 && threadIdx.x == 0) *total = lo + block_total;
     const uint64_t row = w / wx;
     const uint32_t vbase = (uint32_t)(row * rx) + (uint32_t)(w % wx) * 32u;
     // four words at a time, 16 lanes each: lane l of the 16 takes bits 2l and 2l + 1
@@ -530,11 +519,27 @@ struct AxisMaps {
 
 // blockIdx.y = 0, 1, 2: the maps of axis x, y, z; blockIdx.y = 3: the row
 // occupancy bits, one wave per 64 rows (each wave writes its two words);
-// blockIdx.y = 4: clears the per-cell band counts cnt[ncells].
+// blockIdx.y = 4: clears the per-cell band counts cnt[ncells]; blockIdx.y = 5: the
+// band vertices of every 256 mask words (partials), for k_band_lists.
 __global__ __launch_bounds__(256) void k_axis_maps(GridDev sc, GridDev sp, int radius, AxisMaps m,
                                                    const uint32_t* __restrict__ bits, uint32_t wx,
-                                                   uint32_t* __restrict__ cnt, uint64_t ncells) {
+                                                   uint32_t* __restrict__ cnt, uint64_t ncells,
+                                                   uint64_t nwords,
+                                                   uint32_t* __restrict__ partials) {
+    __shared__ uint32_t part[4];
     const uint32_t axis = blockIdx.y;
+    if (axis == 5) {
+        const uint32_t groups = (uint32_t)((nwords + 255) / 256);
+        for (uint32_t g = blockIdx.x; g < groups; g += gridDim.x) {
+            const uint64_t w = (uint64_t)g * 256u + threadIdx.x;
+            const uint32_t c = wave_sum(w < nwords ? (uint32_t)__popc(bits[w]) : 0u);
+            if (__lane_id() == 0) part[threadIdx.x >> 6] = c;
+            __syncthreads();
+            if (threadIdx.x == 0) partials[g] = part[0] + part[1] + part[2] + part[3];
+            __syncthreads();
+        }
+        return;
+    }
     if (axis == 4) {
         for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < ncells;
              i += (uint64_t)gridDim.x * blockDim.x)
@@ -628,13 +633,14 @@ __device__ __forceinline__ uint32_t layer_rows(const AxisMaps& m, const GridDev&
 // k_axis_maps).  Writing the list too took 19 us at 113^3 and 41 us at 384^3,
 // and the scan before it 9; listing costs the Yu13
 // field 5 and 20 us there.
-__global__ __launch_bounds__(256) void k_slab_rows(const uint32_t* __restrict__ bits, GridDev sc,
-                                                   uint32_t wx, AxisMaps m, uint32_t vcx,
-                                                   uint32_t vcy, uint32_t* __restrict__ slab,
-                                                   uint32_t* __restrict__ cnt) {
+__device__ __forceinline__ void slab_rows(uint32_t block, uint32_t blocks,
+                                          const uint32_t* __restrict__ bits, const GridDev& sc,
+                                          uint32_t wx, const AxisMaps& m, uint32_t vcx,
+                                          uint32_t vcy, uint32_t* __restrict__ slab,
+                                          uint32_t* __restrict__ cnt) {
     const uint64_t total = (uint64_t)vcx * vcy * sc.rz;
-    for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-         t += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t t = (uint64_t)block * blockDim.x + threadIdx.x; t < total;
+         t += (uint64_t)blocks * blockDim.x) {
         const uint32_t cx = (uint32_t)(t % vcx);
         const uint32_t cy = (uint32_t)((t / vcx) % vcy);
         const uint32_t z = (uint32_t)(t / ((uint64_t)vcx * vcy));
@@ -689,6 +695,24 @@ __global__ __launch_bounds__(256) void k_slab_rows(const uint32_t* __restrict__ 
         slab[idx] = o;
         if (o) atomicAdd(&cnt[v], o);
     }
+}
+
+// Both lists in one launch: workgroups [0, emit_blocks) write the band index, the
+// others count the slabs.  Each waits on chains of loads, so one launch after the
+// other took the sum of their times: 10.4 us for 6.0 at 128^3, 14.6 for 12.3 at
+// 256^3, and a launch more (a second with the counts now in k_axis_maps).
+__global__ __launch_bounds__(256) void k_band_lists(
+    uint32_t emit_blocks, const uint32_t* __restrict__ bits, const uint32_t* __restrict__ partials,
+    uint64_t nwords, GridDev sc, uint32_t wx, uint32_t* __restrict__ word_off,
+    uint32_t* __restrict__ band_index, uint64_t cap, uint32_t* __restrict__ total, int scanned,
+    AxisMaps m, uint32_t vcx, uint32_t vcy, uint32_t* __restrict__ slab,
+    uint32_t* __restrict__ cnt) {
+    if (blockIdx.x < emit_blocks)
+        band_emit(blockIdx.x, emit_blocks, bits, partials, nwords, wx, sc.rx, word_off, band_index,
+                  cap, total, scanned);
+    else
+        slab_rows(blockIdx.x - emit_blocks, gridDim.x - emit_blocks, bits, sc, wx, m, vcx, vcy,
+                  slab, cnt);
 }
 
 }  // namespace
@@ -773,18 +797,6 @@ fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& s
     const uint32_t emit_blocks = (uint32_t)((nwords + 255) / 256);
     uint32_t* partials;
     FSR_TRY(arena_typed(ctx, A_BAND_PARTIALS, emit_blocks, &partials));
-    hipLaunchKernelGGL(k_band_partials, dim3(emit_blocks), dim3(256), 0, s, bits, nwords,
-                       partials);
-    FSR_LAUNCH_CHECK("k_band_partials");
-    // up to 4096 blocks each block sums the counts before it (at most 16 words
-    // per thread); beyond, the counts are scanned first
-    const int scanned = emit_blocks > 4096u ? 1 : 0;
-    if (scanned)
-        FSR_TRY(scan_exclusive(ctx, SCAN_U32, partials, partials, emit_blocks, nullptr, nullptr,
-                               s));
-    hipLaunchKernelGGL(k_band_emit, dim3(emit_blocks), dim3(256), 0, s, bits, partials, nwords,
-                       wx, sc.rx, word_off, band_index, V, &st->num_band_vertices, scanned);
-    FSR_LAUNCH_CHECK("k_band_emit");
     out->band_index = band_index;
 
     // cell-major work list
@@ -816,18 +828,25 @@ fsr_status band_compact(fsr_context* ctx, const uint32_t* bits, const GridDev& s
     const uint32_t maxres = std::max(sc.rx + vcx, std::max(sc.ry + vcy, sc.rz + vcz));
     const uint32_t map_blocks = (uint32_t)std::max<uint64_t>(
         (maxres + 255) / 256, std::min<uint64_t>((rows + 255) / 256, 1024));
-    hipLaunchKernelGGL(k_axis_maps, dim3(map_blocks, 5), dim3(256), 0, s, sc, sp, radius, m, bits,
-                       wx, cnt, nvc);
+    hipLaunchKernelGGL(k_axis_maps, dim3(map_blocks, 6), dim3(256), 0, s, sc, sp, radius, m, bits,
+                       wx, cnt, nvc, nwords, partials);
     FSR_LAUNCH_CHECK("k_axis_maps");
+    // up to 4096 blocks each block sums the counts before it (at most 16 words
+    // per thread); beyond, the counts are scanned first
+    const int scanned = emit_blocks > 4096u ? 1 : 0;
+    if (scanned)
+        FSR_TRY(scan_exclusive(ctx, SCAN_U32, partials, partials, emit_blocks, nullptr, nullptr,
+                               s));
     // slab counts (and cell counts); cell offsets, chunk offsets and the chunk
     // list in one scan
     const uint64_t nslabs = (uint64_t)vcx * vcy * sc.rz;
     uint32_t* slab;
     FSR_TRY(arena_typed(ctx, A_SLAB, nslabs, &slab));
     const uint32_t slab_blocks = (uint32_t)std::min<uint64_t>((nslabs + 255) / 256, 16384);
-    hipLaunchKernelGGL(k_slab_rows, dim3(slab_blocks), dim3(256), 0, s, bits, sc, wx, m, vcx, vcy,
-                       slab, cnt);
-    FSR_LAUNCH_CHECK("k_slab_rows");
+    hipLaunchKernelGGL(k_band_lists, dim3(emit_blocks + slab_blocks), dim3(256), 0, s, emit_blocks,
+                       bits, partials, nwords, sc, wx, word_off, band_index, V,
+                       &st->num_band_vertices, scanned, m, vcx, vcy, slab, cnt);
+    FSR_LAUNCH_CHECK("k_band_lists");
     FSR_TRY(scan_cells(ctx, cnt, nvc, cell_off, chunk_off, chunk_cell, max_chunks,
                        &counters->num_chunks, s));
     out->cell_off = cell_off;
