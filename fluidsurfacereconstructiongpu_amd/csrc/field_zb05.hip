@@ -26,8 +26,8 @@
 // absolute-coordinate sum has.  Candidates are staged in the reference's
 // order (z, y, x cells, then range order); each vertex's sums are formed as
 // four interleaved partial sums that are added at the end.  Work is
-// distributed dynamically, one chunk per atomic fetch, each XCD starting on
-// its own contiguous eighth of the chunk list.
+// distributed by ItemFetch: each XCD starts on its own contiguous eighth of the
+// chunk list.  A smaller frame's workgroup shares each chunk (field_shared).
 //
 // Culling: a chunk's vertices are a compact slab of its cell (the cell-major
 // list is in ascending vertex id), so many block candidates lie farther than R

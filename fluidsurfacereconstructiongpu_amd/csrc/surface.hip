@@ -6,8 +6,7 @@
 //                       not on the last layer of the grid and has an empty cell in
 //                       its clamped 3^3 block is a surface cell.
 //   k_involve_window    the involve half of the latter: every cell of the clamped
-//                       5^3 block of a surface cell gets its particle count (the
-//                       block test as three separable 5-wide passes).
+//                       5^3 block of a surface cell gets its particle count.
 //   k_flags_from_cells  marks the particles of surface cells (the reference's
 //                       per-cell loop over the cell's range, written per particle).
 //   k_colorfield        extractionOfSurfaceParticlesUsingColorField
