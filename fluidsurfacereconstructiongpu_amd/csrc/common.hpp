@@ -536,7 +536,7 @@ fsr_status scan_mc(fsr_context* ctx, const uint32_t* nv, uint64_t n_max, const u
                    uint32_t* vert_off, uint32_t* valid_idx, uint32_t* d_total_verts,
                    uint32_t* d_total_valid, hipStream_t s);
 
-// Several independent u32 fills in one launch.
+// Several independent u32 fills, done in the launch that hashes the particles.
 constexpr int kMaxFillJobs = 8;
 struct FillList {
     uint32_t* p[kMaxFillJobs];
@@ -550,7 +550,6 @@ struct FillList {
         ++count;
     }
 };
-fsr_status fill_multi(const FillList& l, hipStream_t s);
 // Zeroes the per-XCD fetch counters before a persistent kernel that uses them.
 inline fsr_status reset_xcd(Counters* c, hipStream_t s) {
     return fill_u32(c->xcd_next, 0u, sizeof(c->xcd_next) / 4, s);

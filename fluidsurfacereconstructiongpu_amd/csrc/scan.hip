@@ -492,36 +492,6 @@ __global__ void k_fill_f32(float* p, float v, uint64_t n) {
         p[i] = v;
 }
 
-struct FillArgs {
-    uint32_t* p[kMaxFillJobs];
-    uint64_t n[kMaxFillJobs];
-    uint32_t value[kMaxFillJobs];
-    uint32_t blk_end[kMaxFillJobs];  // cumulative block counts
-    int count;
-};
-
-// Blocks [blk_end[j-1], blk_end[j]) fill job j (block-uniform job lookup):
-// 16-byte stores from the first 16-byte boundary, single words around them.
-__global__ __launch_bounds__(256) void k_fill_multi(FillArgs a) {
-    int j = 0;
-    while (j + 1 < a.count && blockIdx.x >= a.blk_end[j]) ++j;
-    const uint32_t b0 = j ? a.blk_end[j - 1] : 0u;
-    const uint64_t nb = a.blk_end[j] - b0;
-    uint32_t* p = a.p[j];
-    const uint32_t v = a.value[j];
-    const uint64_t n = a.n[j];
-    const uint64_t t = (uint64_t)(blockIdx.x - b0) * blockDim.x + threadIdx.x;
-    const uint64_t stride = nb * blockDim.x;
-    const uint64_t head = min<uint64_t>(((16u - ((uintptr_t)p & 15u)) & 15u) >> 2, n);
-    const uint64_t n4 = (n - head) >> 2;
-    uint4* p4 = reinterpret_cast<uint4*>(p + head);
-    const uint4 q = make_uint4(v, v, v, v);
-    for (uint64_t i = t; i < n4; i += stride) p4[i] = q;
-    if (t < head) p[t] = v;
-    const uint64_t tail = head + 4 * n4;
-    if (t < n - tail) p[tail + t] = v;
-}
-
 // Workgroups of a scan over n_max elements (each owns whole 4096-element tiles).
 uint32_t scan_blocks(uint64_t n_max) {
     const uint64_t want = (n_max + kScanTile - 1) / kScanTile;
@@ -695,25 +665,6 @@ fsr_status fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)blocks), dim3(256), 0, s, p, value, n);
     FSR_LAUNCH_CHECK("k_fill_u32");
-    return FSR_OK;
-}
-
-fsr_status fill_multi(const FillList& l, hipStream_t s) {
-    FillArgs a;
-    a.count = 0;
-    uint32_t blocks = 0;
-    for (int j = 0; j < l.count; ++j) {
-        if (l.n[j] == 0) continue;
-        const int k = a.count++;
-        a.p[k] = l.p[j];
-        a.n[k] = l.n[j];
-        a.value[k] = l.value[j];
-        blocks += (uint32_t)std::min<uint64_t>((l.n[j] + 1023) / 1024, 4096);
-        a.blk_end[k] = blocks;
-    }
-    if (!a.count) return FSR_OK;
-    hipLaunchKernelGGL(k_fill_multi, dim3(blocks), dim3(256), 0, s, a);
-    FSR_LAUNCH_CHECK("k_fill_multi");
     return FSR_OK;
 }
 

