@@ -766,8 +766,8 @@ fsr_status band_build(fsr_context* ctx, const BandArgs& a, hipStream_t s) {
                            (uint64_t)wx * a.sc.ry, a.sc.rz, (uint64_t)a.sc.rz);
         FSR_LAUNCH_CHECK("k_dilate_rows(z)");
     }
-    // six workgroups of 4 waves per CU
-    const uint32_t eb = 6u * (uint32_t)ctx->num_cus;
+    // six workgroups of 4 waves per CU, within the band class's limit
+    const uint32_t eb = (uint32_t)persistent_blocks(ctx, 64 * kExcWaves, 6, TUNE_BAND);
     // 1.5 h in double, as the smallest float that is not below it: for a float
     // d, (double)d < L holds exactly when d < that float
     const double L = (double)a.h * 1.5;
