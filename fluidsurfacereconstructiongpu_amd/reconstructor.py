@@ -168,9 +168,16 @@ class Reconstructor:
         torch = self.torch
         n = fr.n
         off = (3 * n + 63) // 64 * 64  # each array on a 256-byte boundary
-        if off + n > _STAGE_FLOATS or n == 0:
-            return (torch.from_numpy(fr.pos).to(self.device),
-                    torch.from_numpy(fr.dens).to(self.device))
+        # arrays of another form (a column of densities, spare ones past the last
+        # particle) keep it on the device, so they go as they are
+        plain = (isinstance(fr.pos, np.ndarray) and isinstance(fr.dens, np.ndarray)
+                 and fr.pos.shape == (n, 3) and fr.dens.shape == (n,))
+        if off + n > _STAGE_FLOATS or n == 0 or not plain:
+            pos, dens = torch.from_numpy(fr.pos), torch.from_numpy(fr.dens)
+            if pos.numel() < 3 * n or dens.numel() < n:
+                raise ValueError("%d particles, but %d coordinates and %d densities"
+                                 % (n, pos.numel(), dens.numel()))
+            return pos.to(self.device), dens.to(self.device)
         if self._stage_busy:  # the call before did not get to its synchronisation
             torch.cuda.synchronize(self.device)
         if self._stage is None or self._stage.numel() < off + n:
