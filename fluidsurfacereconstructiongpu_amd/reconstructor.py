@@ -205,8 +205,10 @@ class Reconstructor:
             return
         ptr, _ = self.ctx.buffer_ptr("permutation")
         perm = torch.as_tensor(_DeviceWords(ptr, n), device=self.device).long()
-        for t in (pos, dens):
-            t[perm] = t.clone()
+        # the n rows of 3 and the n values that the frame sorted, in tensors of any form
+        for t, width in ((pos, 3), (dens, 1)):
+            rows = t.as_strided((n, width), (width, 1))
+            rows[perm] = rows.clone()
 
     def launch(self, fr: Frame, pos, dens, tri_capacity: int, sim=None, stream=None):
         """Enqueues one frame; pos (N, 3) and dens (N,) are device tensors that

@@ -68,3 +68,37 @@ def test_too_few_values_are_refused(torch_cuda, n):
     for short in (dict(dens=fr.dens[:1]), dict(dens=fr.dens[:-1]), dict(pos=fr.pos[:, :2].copy())):
         with pytest.raises(ValueError):
             rc.Reconstructor("zb05").run(dataclasses.replace(fr, **short))
+
+
+@pytest.mark.parametrize("indexed", [False, True])
+@pytest.mark.parametrize("form", ["column", "longer", "spare rows", "part"])
+def test_rerun_restores_given_tensors(torch_cuda, form, indexed):
+    """The rerun after an overflow puts device tensors back in order whatever their
+    form: the same bits as a run with room from the start."""
+    print(f"\n[gpu case] rerun forms {form} indexed={indexed}", flush=True)
+    n = 5003
+    fr = ds.scattered(n=n, extent=0.02 * n ** (1 / 3), ratio=2)
+    fr.dens = np.random.default_rng(3).uniform(900.0, 1100.0, n).astype(np.float32)
+
+    def run(cap):
+        pos, dens = torch_cuda.from_numpy(fr.pos).cuda(), torch_cuda.from_numpy(fr.dens).cuda()
+        spare = torch_cuda.full((7,), -5.0, device="cuda")
+        if form == "column":
+            dens = dens[:, None]
+        elif form == "longer":
+            dens = torch_cuda.cat([dens, spare])
+        elif form == "spare rows":
+            dens = torch_cuda.cat([dens, spare]).view(-1, 10)   # 5,010 in rows of 10
+        else:   # inside a larger buffer
+            dens = torch_cuda.cat([spare, dens, spare])[7:7 + n]
+        rec = rc.Reconstructor("zb05")
+        if indexed:
+            phi, vtx, nrm, idx, stats = rec.run_indexed(fr, cap, cap, pos=pos, dens=dens)
+            out = [phi, vtx, nrm, idx]
+        else:
+            res = rec.run(fr, cap, pos=pos, dens=dens)
+            out, stats = [res.phi, *res.soup()], res.stats
+        assert rec.dens_sorted is dens and not stats["overflow"]
+        return [t.cpu().numpy().tobytes() for t in out + [pos, dens]]
+
+    assert run(1) == run(64 * n + 4096)
