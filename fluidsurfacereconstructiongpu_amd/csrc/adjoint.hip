@@ -246,10 +246,9 @@ struct FieldBackArgs {
     uint32_t* next;               // per-XCD fetch counters (ItemFetch)
     const uint32_t* cell_off;     // virtual cell -> first cell-major slot
     const uint32_t* cell_cnt;
-    const uint32_t* cell_band;    // cell-major slot -> vertex id
     const float4* coef;           // cell-major slot -> (u, c)
     const float4* vpos;           // cell-major slot -> vertex position
-    GridDev sp, sc;
+    GridDev sp;
     uint32_t vcx, vcy;
     int radius;
     float radius_sq;
@@ -586,11 +585,9 @@ fsr_status field_zb05_backward(fsr_context* ctx, const float* g_phi, float* g_po
     a.next = next;
     a.cell_off = st.bc.cell_off;
     a.cell_cnt = st.bc.cell_cnt;
-    a.cell_band = st.cell_band;
     a.coef = coef;
     a.vpos = vpos;
     a.sp = st.sp;
-    a.sc = st.sc;
     a.vcx = st.bc.vcx;
     a.vcy = st.bc.vcy;
     a.radius = st.bc.radius;

@@ -333,9 +333,9 @@ struct CovArgs {
     const uint32_t* involve_off;
     GridDev sp;
     float radius;           // anisotropic radius r
-    // the reference's tests on the correctly rounded distance, as exact tests
-    // on d^2: sqrt(d2) <= r  <=>  d2 <= d2_le_r;  sqrt(d2) < r  <=>  d2 <= d2_lt_r
-    float d2_le_r, d2_lt_r;
+    // the reference's test on the correctly rounded distance, as an exact test on
+    // d^2: sqrt(d2) <= r  <=>  d2 <= d2_le_r
+    float d2_le_r;
     float h2;               // smoothing radius squared
     float inv_h;            // 1 / h
     float kr, kn;
@@ -1925,7 +1925,6 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     ca.sp = a.sp;
     ca.radius = a.aniso_radius;
     ca.d2_le_r = sqrt_bound(a.aniso_radius, false);
-    ca.d2_lt_r = sqrt_bound(a.aniso_radius, true);
     ca.h2 = a.h2;
     ca.inv_h = a.inv_h;
     ca.kr = a.kr;
