@@ -621,13 +621,9 @@ __device__ __forceinline__ void nb_chunk(float* __restrict__ q, const float* __r
         fill += (uint32_t)__popcll(m);
         n_kept += (uint32_t)__popcll(m);
         if (fill >= 64u) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_lds_sync();
             nb_tiles<kCov, NT, kNbStride>(q + head, 64u, b1, acc, cnt, le_s2);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_lds_sync();
             head ^= 64u;
             fill -= 64u;
         }
@@ -646,13 +642,9 @@ __device__ __forceinline__ void nb_chunk(float* __restrict__ q, const float* __r
                 for (int k = 0; k < 6; ++k) q[(kNbXX + k) * kNbStride + head + lane] = 0.f;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
         nb_tiles<kCov, NT, kNbStride>(q + head, n, b1, acc, cnt, le_s2);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
     }
     // the four partial sums of each lane-particle; lane l keeps those of
     // particle 16 T + l % 16 with T = l / 16, i.e. particle l

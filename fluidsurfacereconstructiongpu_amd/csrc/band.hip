@@ -214,12 +214,6 @@ __device__ __forceinline__ int trunc_clamped(float q, int res) {
     return (int)q;
 }
 
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The reference's per-particle band loop (the exact path), for the exception
 // list or, when every surface particle takes it, for the surface flags in
 // particle order.  A wave takes `group` consecutive list entries (particles),
@@ -364,7 +358,7 @@ __global__ __launch_bounds__(64 * kExcWaves) void k_band_exceptions(BandArgs a, 
         } else {
             if (windowed)
                 for (int t = (int)lane; t < nwin; t += 64) win[t] = 0u;
-            wave_sync_lds();
+            wave_lds_sync();
         }
         for (uint32_t it = 0; it < n; it += kExcPart) {
             const uint32_t slot = it + lane / kExcLanes;
@@ -417,9 +411,9 @@ __global__ __launch_bounds__(64 * kExcWaves) void k_band_exceptions(BandArgs a, 
             mb.flush(win, a.bits, a.sc, wx, (int)threadIdx.x, 64 * kExcWaves);
             __syncthreads();
         } else {
-            wave_sync_lds();
+            wave_lds_sync();
             if (windowed && n) mb.flush(win, a.bits, a.sc, wx, (int)lane, 64);
-            wave_sync_lds();
+            wave_lds_sync();
         }
     }
 }

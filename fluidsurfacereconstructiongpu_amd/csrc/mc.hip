@@ -155,9 +155,7 @@ __device__ __forceinline__ void emit_cube(const McArgs& a, uint32_t vid, uint32_
         corner[threadIdx.x][0] = make_float4(val, cpx, cpy, cpz);
         corner[threadIdx.x][1] = make_float4(nx, ny, nz, 0.0f);
         const uint32_t f = group8_or((val <= a.iso) ? (1u << c) : 0u);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
         const uint32_t nv = case_vertices(f);
         if ((uint64_t)off + nv <= a.capacity) {
             const uint64_t tri = cMcTri[f];
@@ -209,9 +207,7 @@ __device__ __forceinline__ void emit_cube(const McArgs& a, uint32_t vid, uint32_
             }
         }
         // the group's corner slots are rewritten by its next cube
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
     }
 }
 

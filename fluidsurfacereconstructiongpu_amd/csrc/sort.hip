@@ -171,12 +171,6 @@ __global__ __launch_bounds__(kSortThreads) void k_digit_scan(uint32_t* __restric
     if (t == 0) totals[blockIdx.x] = carry;
 }
 
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Stable scatter of one 2048-key tile by kScatterWaves waves.  Wave w owns the
 // contiguous keys [256 w, 256 w + 256) of the tile, in 4 rounds of 64:
 //   1. per round, the lanes holding the same digit are found with 8 ballots;
@@ -267,9 +261,9 @@ __global__ __launch_bounds__(kScatterThreads) void k_radix_scatter(
         }
         const uint32_t rank = mask_rank(peers);
         const uint32_t pre = wcnt[wave][d];
-        wave_sync_lds();
+        wave_lds_sync();
         if (valid && rank == 0) wcnt[wave][d] = pre + (uint32_t)__popcll(peers);
-        wave_sync_lds();
+        wave_lds_sync();
         loc[j] = pre + rank;
     }
     __syncthreads();
