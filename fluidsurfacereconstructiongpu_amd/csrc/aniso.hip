@@ -343,7 +343,7 @@ struct CovArgs {
     float mass;
     fsr_matrix* gmat;       // [I]
     float4* sigma;          // [I] eigenvalues, descending
-    float4* smooth;     // its w gets the culling radius (may be null)
+    float4* smooth;         // its w gets the culling radius (may be null)
     int drop_noninv;
     float4* rec;            // [2N] field records
     uint32_t* work;         // work records (may be null)
@@ -1819,8 +1819,6 @@ static bool sums_moments(const AnisoArgs& a) {
     return a.noninv_moments && noninv_polynomial_exact(a.sp, a.aniso_radius);
 }
 
-// Scratch of the two particle passes: per-cell counts and chunk offsets, and
-// the chunk -> cell lists.
 // The work-record sections (see write_work), one arena slot for the three
 // kernels.
 static fsr_status work_section(fsr_context* ctx, WorkSection w, uint32_t** out) {
@@ -1831,6 +1829,8 @@ static fsr_status work_section(fsr_context* ctx, WorkSection w, uint32_t** out) 
     return FSR_OK;
 }
 
+// Scratch of the two particle passes (smoothing; covariance: 2): each cell's first
+// chunk, and the chunk -> cell lists.
 struct PassScratch {
     uint32_t *chunk_off, *chunk_off2, *chunk_cell, *chunk_cell2;
     uint64_t max_chunks;
@@ -1930,7 +1930,9 @@ fsr_status aniso_cov(fsr_context* ctx, const AnisoArgs& a, hipStream_t s) {
     ca.drop_noninv = sums_moments(a) ? 1 : 0;
     FSR_TRY(work_section(ctx, WORK_COV, &ca.work));
     FSR_TRY(cell_boxes(ctx, a, s, &ca.cell_box));
-    // the chunks hold the involved particles only, at most all
+    // The shared form up to coop_max chunks, as in the smoothing.  The chunks hold
+    // the involved particles only, a count that the host does not know, so the
+    // build with that form is taken up to twice as many particles.
     const uint32_t coop_max = coop_limit(ctx, blocks_cov);
     auto cov = a.n / 64u <= 2u * coop_max ? k_covariance_mc<true> : k_covariance_mc<false>;
     hipLaunchKernelGGL(cov, dim3(blocks_cov), dim3(kAnisoThreads), 0, s, ca, cl2, coop_max);

@@ -19,16 +19,18 @@
 // grid, and every particle when the condition fails, go through the exact
 // per-particle loop of the reference (k_band_exceptions).
 //
-// Compaction: popcount per word -> exclusive scan -> each word writes its set
-// bits in ascending order (the reference's surfaceVerticesIndexArray).
+// Compaction: set bits counted per 256 words -> each block of 256 words offsets
+// and scans its words' counts -> 16 lanes a word write its set bits in ascending
+// order (the reference's surfaceVerticesIndexArray; see band_emit).
 //
-// Cell-major list: the field kernels process the band grouped by the hash cell
+// Cell-major work list: the field kernels process the band grouped by the hash cell
 // each vertex falls in (getIndex3D of the vertex position, exactly as the
 // reference's field kernels compute it), so that all 64 lanes of a wave share
 // one neighbour-cell block.  Cells outside the hash grid are folded into a ring
 // of `radius` virtual cells on each side (their clamped neighbour blocks
-// coincide).  The order of vertices inside a cell's list does not affect any
-// value: every vertex sums its candidates in the cell's fixed order.
+// coincide).  The list holds 64-vertex chunks, not vertices: a chunk's are read
+// from the mask (chunk_vertex).  The order of vertices inside a cell does not
+// affect any value: every vertex sums its candidates in the cell's fixed order.
 #include <algorithm>
 #include <cmath>
 #include <limits>
@@ -424,11 +426,12 @@ __global__ __launch_bounds__(64 * kExcWaves) void k_band_exceptions(BandArgs a, 
 // (the sum of the counts of the blocks before it, at most 8 words per thread
 // from L2), scans its words' counts, writes each word's offset (word_off, the
 // band rank of the word's first vertex) and the block's vertices, 16 lanes for a
-// word: its lanes store to consecutive entries.  (A lane for
-// each word, writing its ids into LDS for the block to copy out, met bank
-// conflicts, and stored directly when the block had more than 4096.)  12.4 -> 8.0
-// us for a 1M dam break at 256^3, 39 -> 10.5 with the wider band of Akinci12, 25
-// -> 12 at 384^3; 3.0 -> 4.1 where the grid has a few full words only.
+// word: its lanes store to consecutive entries.  (A lane for each word, writing
+// its ids into LDS for the block to copy out, met bank conflicts, and stored
+// directly when the block had more than 4096.)  12.4 -> 8.0 us for a 1M dam break
+// at 256^3, 39 -> 10.5 with the wider band of Akinci12, 25 -> 12 at 384^3; 3.0 ->
+// 4.1 where the grid has a few full words only, beside the slab counts, which
+// take as long.
 // The last block writes the band size.
 __device__ __forceinline__ void band_emit(uint32_t block, uint32_t blocks,
                                           const uint32_t* __restrict__ bits,
@@ -625,8 +628,7 @@ __device__ __forceinline__ uint32_t layer_rows(const AxisMaps& m, const GridDev&
 // without band vertices are skipped with the row occupancy bits.  It writes the
 // slab's band vertex count and adds it to its cell's count (cnt, cleared by
 // k_axis_maps).  Writing the list too took 19 us at 113^3 and 41 us at 384^3,
-// and the scan before it 9; listing costs the Yu13
-// field 5 and 20 us there.
+// and the scan before it 9; listing costs the Yu13 field 5 and 20 us there.
 __device__ __forceinline__ void slab_rows(uint32_t block, uint32_t blocks,
                                           const uint32_t* __restrict__ bits, const GridDev& sc,
                                           uint32_t wx, const AxisMaps& m, uint32_t vcx,

@@ -5,8 +5,8 @@
 namespace fsr {
 
 // The vertex ids of chunk k of virtual cell v, listed from the band mask in
-// the cell-major order (layer z, row y, then x ascending): lane l < cnt receives the (64 k + l)-th band vertex
-// of the cell.  The cell's layers (slabs) are consecutive in the slab counts;
+// the cell-major order (layer z, row y, then x ascending): lane l < cnt receives
+// the (64 k + l)-th band vertex of the cell.  The cell's layers (slabs) are consecutive in the slab counts;
 // 64 layers at a time, those that overlap [64 k, 64 k + 64) are expanded word
 // by word, each lane taking one (layer, row, word) of them, and the wanted
 // ranks go to `scratch` (64 LDS words of the wave).

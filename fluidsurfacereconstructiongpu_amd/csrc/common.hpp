@@ -11,8 +11,10 @@
 //                  scalar vertex instead of the reference's dense u32[V] flags
 //   band index     u32[B] ascending linear vertex ids (the reference's
 //                  surfaceVerticesIndexArray)
-//   cell-major     u32[B] the same ids grouped by the hash cell each vertex
-//                  falls in, cut into 64-vertex chunks for the field kernels
+//   cell-major     work list of the field kernels: the band vertices grouped by
+//                  the hash cell each falls in, in 64-vertex chunks (chunk -> cell,
+//                  each cell's count and offsets, slab counts); the ids themselves,
+//                  u32[B], only in a frame kept for the adjoint
 //   phi            float[V] caller buffer
 #pragma once
 

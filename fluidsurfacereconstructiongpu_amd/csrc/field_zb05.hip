@@ -10,8 +10,8 @@
 // (the caller's fill, 0).  The same field serves the Akinci12 method.
 //
 // MI355X mapping.  A wave owns a chunk of up to 64 band vertices of one hash
-// cell (the cell-major list built in band.hip), so all lanes share one
-// candidate block: the 9 x-runs of the 3^3 block (x-adjacent cells are
+// cell, listed from the band mask in cell-major order (chunk_vertex), so all
+// lanes share one candidate block: the 9 x-runs of the 3^3 block (x-adjacent cells are
 // contiguous in the sorted particle array).  The wave stages candidates in LDS
 // (one coalesced 16-byte load per lane, one candidate per lane) and evaluates
 // them against the chunk's vertices in 16 x 16 tiles on the matrix cores:
@@ -29,8 +29,8 @@
 // distributed by ItemFetch: each XCD starts on its own contiguous eighth of the
 // chunk list.  A smaller frame's workgroup shares each chunk (field_shared).
 //
-// Culling: a chunk's vertices are a compact slab of its cell (the cell-major
-// list is in ascending vertex id), so many block candidates lie farther than R
+// Culling: a chunk's vertices are a compact slab of its cell (cell-major order
+// is by ascending vertex id), so many block candidates lie farther than R
 // from the chunk's bounding box.  At staging every candidate is tested against
 // that box with R^2 (1 + 1e-4); survivors are compacted in order (ballot rank)
 // into a 128-entry LDS queue that is drained 64 at a time.  A culled candidate
@@ -202,8 +202,9 @@ struct Chunk {
     }
 };
 
-// Loads chunk ch: its vertices (listed through `scratch`, 64 words of LDS), their operands into vt (rows of 64:
-// x', y', z', a_x, a_y, a_z, c_x), their box, and the candidate rows.
+// Loads chunk ch: its vertices (listed through `scratch`, 64 words of LDS), their
+// operands into vt (rows of 64: x', y', z', a_x, a_y, a_z, c_x), their box, and
+// the candidate rows.
 __device__ __forceinline__ Chunk load_chunk(const FieldArgs& a, const BandCompactOut& bc,
                                             const VertexDiv& vd, uint32_t ch, float inv_r2,
                                             float* __restrict__ vt, uint32_t* scratch) {

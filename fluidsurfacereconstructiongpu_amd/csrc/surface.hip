@@ -15,10 +15,11 @@
 //                       |sum m/rho_j gradW_spiky(r) r_hat| > 3.  With the radius-count
 //                       surface mode (either method): surface iff fewer than 25
 //                       particles at 0 < |r|^2 < h^2 (FP32 squared distances).
-// Every surface particle then seeds the band: its scalar cell is set in a bit
-// mask of "surface scalar cells" that band.hip dilates, or, when the dilation
-// is not exact for it, it is appended to an exception list that band.hip
-// treats with the reference's per-particle box loop.
+// Every surface particle then seeds the band: its scalar cell is set in a byte
+// mask of "surface scalar cells" that band.hip dilates, or, when it lies outside
+// the scalar grid, it is appended to an exception list that band.hip treats with
+// the reference's per-particle box loop.  On a grid where the dilation is exact
+// for no particle there is neither: band.hip walks the surface flags.
 #include <algorithm>
 #include <type_traits>
 
